@@ -342,16 +342,17 @@ int mdy_minimize_dev(mdy_ctx *ctx, const mdy_cg_params *params, double *d_coord,
 /* Batched form: n independent minimizations (CGMethod::minimize per network,
  * as above) in one cooperative launch. ctxs[i] holds network i with its
  * neighbor lists; all contexts share one device and one precision and appear
- * once. The resident blocks (threads_per_block = 64, 128 or 256; 0 = 64) are
- * split into one cluster per network in proportion to weights[i] (nullable:
- * default the per-evaluation work, interactions + 2 x beads), at least one
- * block each; each cluster runs its own minimization with its own barrier.
+ * once. The resident blocks (of at least threads_per_block = 64, 128 or 256
+ * threads, 0 = 64; of up to 512 while every network gets one) are split into
+ * one cluster per network in proportion to weights[i] (nullable: default the
+ * per-evaluation work, interactions + 2 x beads), at least one block each and
+ * at most one thread per interaction lane; each cluster runs its own minimization with its own barrier.
  * Networks beyond the resident block count run in further launches.
  * first_pass_calls > 0 runs the batch in passes: pass k suspends each
  * minimization at the top of an iteration after first_pass_calls * 4^(k-1)
  * force calls, and the next pass resumes the suspended ones where they
  * stopped, on the blocks the finished networks released (uncapped once each
- * gets 64 blocks or more). first_pass_calls = -k (k = 1..1024) ends the
+ * gets 4096 threads or more). first_pass_calls = -k (k = 1..1024) ends the
  * passes by completions instead: once max(1, m / k) of a launch's m networks
  * have finished, the others suspend at the top of their next iteration and
  * the next pass re-splits the blocks among them, down to one network on all

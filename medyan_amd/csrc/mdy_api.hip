@@ -40,7 +40,7 @@ Dev Ctx::dev() const {
     D.slot_ev = D.slot_bp + 3 * n_bp;
     D.slot_bd = D.slot_ev + 4 * D.n_ev;
     D.n_slots = D.slot_bd + D.n_bd;
-    D.st_off = st_off.p; D.st_idx = st_idx.p; D.dy_off = dy_off.p; D.dy_idx = dy_idx.p;
+    D.row_off = row_off4.p; D.row_idx = row_idx.p;
     D.coplanar_mode = opts.coplanar_mode;
     D.evq = nullptr;   // set by the one-shot launchers in quadrature mode
     D.cq = std::cos(0.5 * M_PI);   // BranchingPositionCosine.cpp:235, 372 (posheta = pi/2)
@@ -170,8 +170,8 @@ void mdy_destroy(mdy_ctx *ctx) {
     release(c.mid); release(c.cell_of); release(c.cell_cnt); release(c.cell_off); release(c.cell_cur);
     release(c.cell_list); release(c.row_cnt); release(c.row_keep); release(c.row_off); release(c.row_keep_off);
     release(c.pairs); release(c.ev_bs); release(c.ev_kr); release(c.bd_flag); release(c.bd_off); release(c.bd_bead);
-    release(c.bd_plane); release(c.bd_k); release(c.bd_sl); release(c.dy_cnt); release(c.dy_off); release(c.dy_cur);
-    release(c.dy_idx); release(c.scan_tmp); release(c.bbox); release(c.x); release(c.xt); release(c.f);
+    release(c.bd_plane); release(c.bd_k); release(c.bd_sl); release(c.row_cnt4); release(c.row_off4);
+    release(c.row_cur); release(c.row_idx); release(c.row_tmp); release(c.scan_tmp); release(c.bbox); release(c.x); release(c.xt); release(c.f);
     release(c.batch_args); release(c.batch_map); release(c.batch_done); release(c.evq); release(c.qpan); release(c.qcnt); release(c.qoff);
     release(c.qmap); release(c.qpart); release(c.qpe); release(c.qtot);
     release(c.contrib); release(c.red); release(c.out); release(c.qe); release(c.qf); release(c.qn); release(c.err);
@@ -308,6 +308,7 @@ int mdy_set_network(mdy_ctx *ctx, const mdy_system *s) {
         for (size_t s2 = 0; s2 < owner.size(); s2++) idx[cur[owner[s2]]++] = (int)s2;
         rc |= upload(c.st_off, off.data(), off.size(), st);
         rc |= upload(c.st_idx, idx.data(), idx.size(), st);
+        c.n_static = (int)idx.size();
         if (hipStreamSynchronize(st) != hipSuccess) return hipfail(ctx, "upload");
     }
     // cylinders

@@ -6,7 +6,7 @@
 // One cooperative launch; every block runs the same control flow and derives
 // every decision from grid reductions that all blocks evaluate in the same
 // fixed order (exact sums), so decisions are identical without a broadcast.
-// Phases are separated by a flag-array grid barrier.
+// Phases are separated by a grid barrier.
 //
 // Every line-search trial evaluates energy AND force slots at the trial point,
 // so an accepted trial needs no second pass over the interactions. An
@@ -33,7 +33,7 @@ struct CgArgs {
     double *qe_u;         // 3 * kQueueCap
     double *spart;        // 6 * nblk * kRed
     int *qe, *qf, *qn;    // 3 * kQueueCap each; qn: 3 x 4 counters
-    unsigned long long *bar;  // [0] abort flag; block b arrival flag at [64 + 16 b]
+    unsigned long long *bar;  // [0] abort flag, [16] arrivals
     unsigned long long *acc;  // 3 x kAccWords phase accumulators
     double *out;          // result record
     long long *prof;      // phase profile, 5 words per phase: barrier exit (block 0), latest
@@ -52,6 +52,7 @@ struct CgArgs {
     // batched passes: suspend at the top of an iteration once this many force
     // calls are done (0: never), and resume from the state a suspension saved
     int suspend_calls, resume;
+    int poll_sleep;       // barrier: 128-clock sleeps between two polls
 };
 
 // result record layout (doubles)
@@ -76,33 +77,24 @@ constexpr int kAcc0 = 0, kAcc1 = 8, kAccMax = 16, kAccDone = 19;
 // phase kinds recorded by the profile
 enum { PK_ENERGY = 1, PK_EFALLBACK, PK_EVAL, PK_FFALLBACK, PK_GATHER, PK_REDUCE, PK_RESTORE };
 
-// result of one hot-loop evaluation: the computeEnergy total (+inf sentinel),
-// the extra accumulator, and the force-fallback queue it filled
-struct Eval {
-    double E;
-    double xa;     // s.F, when requested
-    int nqf;       // queued force fallbacks
-    int qb;        // queue buffer (0..2)
-};
-
 template <bool MIXED>
 struct Cg {
     using Slot = typename SlotT<MIXED>::T;   // force records: double, or float in the mixed form
     const CgArgs &A;
     double *lds;
+    XBlock &xb;                  // the block's exact sums of the current phase
     unsigned long long *accl;    // LDS copy of the words a phase's decisions read
     int G, blk, tid, gtid, gs;
     int ph = 0;                  // phase counter (uniform)
     // batched passes by completions: the launch's count of finished
-    // minimizations (nullable), and its value as of the last gather (uniform)
+    // minimizations (nullable)
     int *done_ctr = nullptr;
-    int done_seen = 0;
-    bool aborted = false;
-    int status = MDY_OK;
+    int status = MDY_OK;         // set by a collective step, the same in every thread
 
     // blk: this block's index within the cluster of G blocks that runs the
     // minimization (the whole grid, or one network's share of a batch)
-    __device__ Cg(const CgArgs &a, double *l, unsigned long long *al, int blk_, int G_) : A(a), lds(l), accl(al) {
+    __device__ Cg(const CgArgs &a, double *l, XBlock &x, unsigned long long *al, int blk_, int G_)
+        : A(a), lds(l), xb(x), accl(al) {
         G = G_; blk = blk_; tid = threadIdx.x;
         gtid = blk * blockDim.x + tid; gs = G * blockDim.x;
     }
@@ -117,63 +109,64 @@ struct Cg {
     __device__ double *red(int p) const { return A.red + (size_t)(p % 3) * G * kRed; }
     __device__ double *qeu(int b) const { return A.qe_u + (size_t)b * kQueueCap; }
 
-    // Grid barrier. Arrival: one agent-scope release per block, then a store of
-    // the phase number to the block's own flag line (no shared counter).
-    // Departure: every block polls all flags itself (thread t polls blocks t,
-    // t+256, ...), then one agent-scope acquire per block. A watchdog on the
-    // poll sets the shared abort flag; every waiting block sees it and leaves.
-    __attribute__((always_inline)) __device__ bool sync(int kind) {
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        const unsigned long long epoch = (unsigned long long)(ph + 1);
-        unsigned long long *flags = A.bar + 64;
-        if (tid == 0) {
-            if (ph < A.prof_cap) {
-                const unsigned long long t = wall_clock64();
-                atomicMax(reinterpret_cast<unsigned long long *>(A.prof) + 5 * (size_t)ph + 1, t);
-                if (blk == 0) A.prof[5 * (size_t)ph + 4] = (long long)t;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            __hip_atomic_store(flags + (size_t)blk * 16, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // Grid barrier, run by the block's first wave. Arrival: one agent-scope
+    // release, then one added to the cluster's count. Departure: lane 0 polls the
+    // count until every block has arrived in this phase, then one agent-scope
+    // acquire. A watchdog on the poll sets the shared abort flag; every waiting
+    // block sees it and leaves. Returns false on abort. The block's other waves
+    // wait at a __syncthreads.
+    __attribute__((always_inline)) __device__ bool barrier(int kind) {
+        const unsigned long long target = (unsigned long long)(ph + 1) * (unsigned long long)G;
+        unsigned long long *count = A.bar + 16;
+        if (tid == 0 && ph < A.prof_cap) {
+            const unsigned long long t = wall_clock64();
+            atomicMax(reinterpret_cast<unsigned long long *>(A.prof) + 5 * (size_t)ph + 1, t);
+            if (blk == 0) A.prof[5 * (size_t)ph + 4] = (long long)t;
         }
-        __shared__ int s_abort;
-        if (tid == 0) s_abort = 0;
-        __syncthreads();
-        int ab = 0;
-        for (int b = tid; b < G; b += blockDim.x) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        bool ab = false;
+        if (tid == 0) {
+            __hip_atomic_fetch_add(count, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             long long spins = 0;
-            while (__hip_atomic_load(flags + (size_t)b * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
-                __builtin_amdgcn_s_sleep(64);   // ~4k cycles between polls: less L2 traffic while others work
+            while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+                for (int q = 0; q < A.poll_sleep; q++) __builtin_amdgcn_s_sleep(2);
                 if (__builtin_expect((++spins & 255) == 0, 0)) {
-                    if (__hip_atomic_load(A.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) { ab = 1; break; }
+                    if (__hip_atomic_load(A.bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) { ab = true; break; }
                     if (spins > A.spin_limit) {
                         __hip_atomic_store(A.bar, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        ab = 1;
+                        ab = true;
                         break;
                     }
                 }
             }
-            if (ab) break;
         }
-        if (ab) s_abort = 1;
-        __syncthreads();
-        if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         if (blk == 0 && tid == 0 && ph < A.prof_cap) {
             A.prof[5 * (size_t)ph] = wall_clock64();
             A.prof_kind[ph] = kind;
         }
-        ph++;
-        if (s_abort) aborted = true;
-        // recycle the queue counters of buffer (ph+1)%3: last written two phases ago,
+        // recycle the queue counters of phase ph + 2: last written two phases ago,
         // read by every block before the barrier just passed
-        if (blk == 0 && tid < 4) A.qn[4 * ((ph + 1) % 3) + tid] = 0;
+        if (blk == 0 && tid < 4) A.qn[4 * ((ph + 2) % 3) + tid] = 0;
         // and the accumulator set of that phase (read by every block right
         // after its barrier, which every block has since left)
         if (blk == 0 && tid < kAccWords)
-            __hip_atomic_store(A.acc + (size_t)((ph + 1) % 3) * kAccWords + tid, 0ull, __ATOMIC_RELAXED,
+            __hip_atomic_store(A.acc + (size_t)((ph + 2) % 3) * kAccWords + tid, 0ull, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-        return !aborted;
+        return __ballot(ab) == 0;
+    }
+    // a whole block's barrier: what it wrote before is visible to every block after
+    __attribute__((always_inline)) __device__ bool sync(int kind) {
+        __shared__ int s_ok;
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (tid < 64) {
+            const bool ok = barrier(kind);
+            if (tid == 0) s_ok = ok ? 1 : 0;
+        }
+        ph++;
+        __syncthreads();
+        return s_ok != 0;
     }
 
     // profile marks of block 0 inside a phase: 0 = work start, 1 = end of the main loop
@@ -190,36 +183,30 @@ struct Cg {
     // A set is read right after its phase's barrier and zeroed by block 0 one
     // barrier later.
     __device__ unsigned long long *accs(int p) const { return A.acc + (size_t)(p % 3) * kAccWords; }
-    // all threads hold the block total `s` (after block_reduce_xsum)
-    __attribute__((always_inline)) __device__ void acc_push(unsigned long long *base, const mdy_xsum &s) const {
-        if (tid < 8) {
-            const long long v = tid == 0 ? s.d[0] : tid == 1 ? s.d[1] : tid == 2 ? s.d[2] : tid == 3 ? s.d[3]
-                              : tid == 4 ? s.d[4] : tid == 5 ? s.d[5] : tid == 6 ? s.d[6] : (long long)s.flags;
-            if (v != 0) {
-                if (tid < 7) atomicAdd(base + tid, (unsigned long long)v);
-                else atomicOr(base + 7, (unsigned long long)v);
-            }
+    // the block's sums and maximum into the set of phase p (after a __syncthreads)
+    __attribute__((always_inline)) __device__ void acc_push(int p) const {
+        const unsigned long long v = xblock_take(xb);
+        if (tid < 17 && v != 0) {
+            unsigned long long *w = accs(p) + tid;
+            if (tid == kAccMax) atomicMax(w, v);
+            else if ((tid & 7) == 7) atomicOr(w, v);
+            else atomicAdd(w, v);
         }
     }
-    __attribute__((always_inline)) __device__ double acc_value(const unsigned long long *base) const {
-        mdy_xsum X;
-#pragma unroll
-        for (int k = 0; k < MDY_XS_N; k++)
-            X.d[k] = (long long)__hip_atomic_load(base + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        X.flags = (int)__hip_atomic_load(base + 7, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        X.cnt = 0;
-        return mdy_xs_value(&X);
-    }
-    // After a barrier every thread needs the same accumulator words: the
-    // first wave loads them once per block into LDS (one request instead of
-    // one per wave to the same L2 lines), then every thread reads LDS.
-    // extra0/extra1 (nullable): counters loaded into words 17 and 18.
-    __attribute__((always_inline)) __device__ void acc_fetch(const unsigned long long *base, const int *extra0,
-                                                             const int *extra1) const {
-        if (tid < 17) accl[tid] = __hip_atomic_load(base + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // After a barrier the first wave loads the words its decisions read into LDS.
+    // extra0..2 (nullable): counters loaded into words 17 to 19. Lane t < 2 returns
+    // the value of sum t.
+    __attribute__((always_inline)) __device__ double acc_fetch(int p, const int *extra0, const int *extra1) const {
+        const unsigned long long *base = accs(p);
+        if (tid < 17 || tid == kAccDone)
+            accl[tid] = __hip_atomic_load(base + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         else if (tid == 17 && extra0) accl[17] = (unsigned long long)(unsigned)ld_i(extra0);
         else if (tid == 18 && extra1) accl[18] = (unsigned long long)(unsigned)ld_i(extra1);
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // LDS of one wave: in order
+        __builtin_amdgcn_wave_barrier();
+        if (tid >= 2) return 0.0;
+        const mdy_xsum X = acc_local(8 * tid);
+        return mdy_xs_value(&X);
     }
     __attribute__((always_inline)) __device__ mdy_xsum acc_local(int off) const {
         mdy_xsum X;
@@ -261,42 +248,13 @@ struct Cg {
         return sync(PK_EFALLBACK);
     }
 
-    // ---- hot loop: all interactions at `pos`, energy (exact total) and force
-    // slots. sd: this thread's share of s.F (zero without a new direction),
-    // reduced together with the energy into the phase's second accumulator;
-    // with_sd: its value lands in ev.xa. Returns false on abort; a queue
-    // overflow sets `status`.
-    __attribute__((always_inline)) __device__ bool eval(const PosAny &pos, Eval &ev, bool with_sd, mdy_xsum &sd) {
-        const int p0 = ph, qb = p0 % 3;
-        Dev d = dv(qb);
-        mdy_xsum xs;
-        mdy_xs_zero(&xs);
-        const int total = d.n_items();
+    // ---- hot loop: all interactions at `pos`, energy (the block's first sum)
+    // and force slots
+    __attribute__((always_inline)) __device__ void eval(const PosAny &pos) {
+        const Dev d = dv(ph % 3);
         mark(0);
-        sweep<MIXED>(d, pos, gtid, gs, nullptr, xs, slots(), false, true);
+        sweep<MIXED, false>(d, pos, blk, G, nullptr, &xb, slots(), false, true);
         mark(1);
-        block_reduce_xsum2_lds(xs, sd, ldsl());
-        acc_push(accs(p0) + kAcc0, xs);
-        acc_push(accs(p0) + kAcc1, sd);
-        if (!sync(PK_EVAL)) return false;
-        acc_fetch(accs(p0), d.qe_n, d.qf_n);
-        mdy_xsum X = acc_local(kAcc0);
-        if (with_sd) {
-            mdy_xsum Y = acc_local(kAcc1);
-            ev.xa = mdy_xs_value(&Y);
-        }
-        const int nqe = (int)accl[17];
-        ev.nqf = (int)accl[18];
-        ev.qb = qb;
-        if (__builtin_expect(nqe > kQueueCap || ev.nqf > kQueueCap, 0)) {
-            status = MDY_ERR_CAPACITY;
-            return true;
-        }
-        if (__builtin_expect(nqe > 0, 0) && !energy_fallback(pos, d, nqe, qb)) return false;
-        double e[kNFF + 2];
-        energy_finish(X, nullptr, nqe, d.qe, qeu(qb), e);
-        ev.E = e[kNFF];
-        return true;
     }
 
     // ---- computeIndividualEnergies at x (energies only, per force field):
@@ -308,15 +266,11 @@ struct Cg {
         double acc[kNFF];
 #pragma unroll
         for (int k = 0; k < kNFF; k++) acc[k] = 0.0;
-        mdy_xsum xs;
-        mdy_xs_zero(&xs);
-        const int total = d.n_items();
-        sweep<MIXED>(d, pos, gtid, gs, acc, xs, nullptr, true, false);
+        sweep<MIXED, false>(d, pos, blk, G, acc, &xb, nullptr, true, false);
         double *r = red(p0);
         block_reduce<kNFF>(acc, lds);
         if (tid < kNFF) r[(size_t)blk * kRed + tid] = acc[tid];
-        block_reduce_xsum(xs, ldsl());
-        acc_push(accs(p0) + kAcc0, xs);
+        acc_push(p0);
         if (!sync(PK_ENERGY)) return false;
         mdy_xsum X = acc_read(accs(p0) + kAcc0);
         const int nqe = ld_i(d.qe_n);
@@ -340,9 +294,9 @@ struct Cg {
     // ---- quadrature forces for the pairs an accepted evaluation queued
     // (CylinderExclVolRepulsion.cpp:1001-1254, 1017-1022 retry with the first
     // cylinder moved off the plane). The slots are written by block 0.
-    __attribute__((always_inline)) __device__ bool force_fallback(const PosAny &pos, const Eval &ev) {
-        const int *qf = A.qf + ev.qb * kQueueCap;
-        for (int q = 0; q < ev.nqf; q++) {
+    __attribute__((always_inline)) __device__ bool force_fallback(const PosAny &pos, int nqf, int qb) {
+        const int *qf = A.qf + qb * kQueueCap;
+        for (int q = 0; q < nqf; q++) {
             const int i = ld_i(qf + q);
             int4 b = A.D.ev_bs[i];
             bool done = false;
@@ -396,507 +350,537 @@ struct Cg {
         return true;
     }
 
-    // ---- per-bead forces from the slots into Fout; x += lam*d when `move`.
-    // Returns max|F_i|, F.F and F.Fprev (Fprev may be null), sums exact.
-    template <bool WIDE, bool BATCH>
-    __attribute__((always_inline)) __device__ bool gather(double *Fout, const double *Fprev, bool move, const double *dvec, double lam, double &maxF,
-                           double &FF, double &FFp) {
-        const int p1 = ph;
-        double m[1] = {0.0};
-        mdy_xsum sff, sfp;
-        mdy_xs_zero(&sff);
-        mdy_xs_zero(&sfp);
+    // ---- forces from the slots into Fout, one lane per coordinate; x += lam*d
+    // when `move`. The block's sums: F.F and F.Fprev (Fprev may be null), and max|F_i|.
+    template <bool BATCH>
+    __attribute__((always_inline)) __device__ void gather(double *Fout, const double *Fprev, bool move,
+                                                          const double *dvec, double lam) {
+        const int ndof = A.D.ndof;
+        double m = 0.0;
         mark(0);
-        for (int b = gtid; b < A.D.nb; b += gs) {
-            d3 f = WIDE ? gather_bead_w<12, 24>(A.D, slots(), b) : gather_bead_w<8, 8>(A.D, slots(), b);
-            const int o = 3 * b;
-            Fout[o] = f.x; Fout[o + 1] = f.y; Fout[o + 2] = f.z;
-            m[0] = fmax(m[0], fmax(fabs(f.x), fmax(fabs(f.y), fabs(f.z))));
-#pragma clang loop unroll(disable)
-            for (int k = 0; k < 3; k++) {
-                const double fk = k == 0 ? f.x : k == 1 ? f.y : f.z;
-                mdy_xs_add(&sff, fk * fk);
-                if (Fprev) mdy_xs_add(&sfp, fk * Fprev[o + k]);
+        int turn = 0;
+        for (int base = blk * blockDim.x; base < ndof; base += gs) {
+            if (turn == kXTurns) { xblock_norm(xb); turn = 0; }
+            turn++;
+            const int o = base + tid;
+            if (o < ndof) {
+                const double f = gather_coord(A.D, slots(), o);
+                Fout[o] = f;
+                m = fmax(m, fabs(f));
+                XAdd{&xb, 0}(f * f);
+                if (Fprev) XAdd{&xb, 8}(f * Fprev[o]);
+                if (move) A.x[o] = A.x[o] + lam * dvec[o];
             }
-            if (move) {
-                A.x[o] = A.x[o] + lam * dvec[o];
-                A.x[o + 1] = A.x[o + 1] + lam * dvec[o + 1];
-                A.x[o + 2] = A.x[o + 2] + lam * dvec[o + 2];
-            }
+            if (ndof - base <= gs) break;
         }
+        xblock_max(xb, m);
         mark(1);
-        block_reduce_xsum2_lds(sff, sfp, ldsl(), m);   // F.F and F.Fprev together, and max|F|
-        unsigned long long *a = accs(p1);
-        if (tid == 0) atomicMax(a + kAccMax, (unsigned long long)__double_as_longlong(m[0]));
         // the cluster's blocks all read the launch's completion count as one
         // block saw it, through this phase's accumulators
         if (BATCH && done_ctr && blk == 0 && tid == 0)
-            atomicMax(a + kAccDone, (unsigned long long)(unsigned)ld_i(done_ctr));
-        acc_push(a + kAcc0, sff);
-        acc_push(a + kAcc1, sfp);
-        if (!sync(PK_GATHER)) return false;
-        acc_fetch(a, nullptr, nullptr);
-        maxF = __longlong_as_double((long long)accl[kAccMax]);
-        if (BATCH && done_ctr)
-            done_seen = (int)__hip_atomic_load(a + kAccDone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        double v2[2];
-#pragma clang loop unroll(disable)
-        for (int k = 0; k < 2; k++) {
-            mdy_xsum Y = acc_local(k == 0 ? kAcc0 : kAcc1);
-            v2[k] = mdy_xs_value(&Y);
-        }
-        FF = v2[0];
-        FFp = Fprev ? v2[1] : 0.0;
-        return true;
+            atomicMax(accs(ph) + kAccDone, (unsigned long long)(unsigned)ld_i(done_ctr));
     }
 };
 
-// s = F + beta * d for every bead into Sn, and this thread's share of s.F
-// into sd (reduced with the phase's energy, or on its own without a trial)
+// s = F + beta * d for every coordinate into Sn, and s.F into the block's
+// second sum (reduced with the phase's energy, or on its own without a trial)
 template <bool MIXED>
 __device__ __attribute__((always_inline)) void spec_direction(Cg<MIXED> &K, const double *Fn, const double *dprev,
-                                                              double beta, double *Sn, mdy_xsum &sd) {
-    // thread t takes beads gs-1-t, 2gs-1-t, ...: the first threads carry the
-    // most excluded-volume items in the sweep that follows in the same phase
-    for (int b = K.gs - 1 - K.gtid; b < K.A.D.nb; b += K.gs) {
-        const int o = 3 * b;
-        for (int k = 0; k < 3; k++) {
-            double s = Fn[o + k] + beta * dprev[o + k];
-            Sn[o + k] = s;
-            mdy_xs_add(&sd, s * Fn[o + k]);
+                                                              double beta, double *Sn) {
+    int turn = 0;
+    for (int base = K.blk * blockDim.x; base < K.A.D.ndof; base += K.gs) {
+        if (turn == kXTurns) { xblock_norm(K.xb); turn = 0; }
+        turn++;
+        const int o = base + K.tid;
+        if (o < K.A.D.ndof) {
+            const double f = Fn[o], s = f + beta * dprev[o];
+            Sn[o] = s;
+            XAdd{&K.xb, 8}(s * f);
         }
+        if (K.A.D.ndof - base <= K.gs) break;
     }
 }
 
-// The minimizer as a state machine: every loop turn performs at most one kind
-// of device work (each with a single call site, so each is inlined once) and
-// then advances the CGMethod::minimize control flow
-// (CGMethod.hpp:826-1743, backtrackingLineSearch CGMethod.cpp:43-360).
+// The minimizer as a state machine: every turn performs one kind of device
+// work (each with a single call site, so each is inlined once), and one thread
+// of every block then advances the CGMethod::minimize control flow
+// (CGMethod.hpp:826-1743, backtrackingLineSearch CGMethod.cpp:43-360) from the
+// reduced sums, which are the same bits in every block. Its state and the next
+// work's operands are in LDS: held in registers by every thread, as the same
+// value 64 times per wave, they left room for one wave per SIMD.
 // The first trial of a line search that follows an accepted step is taken
 // along s = F + beta*d while s itself is formed in the same phase; if s.F <= 0
 // (resetCGParams) that trial is discarded and redone along F.
-enum Op { OP_NONE, OP_EVAL_FF, OP_EVAL, OP_GATHER, OP_MINSTEP, OP_SDONLY, OP_RESTORE };
+enum Op { OP_NONE, OP_EVAL_FF, OP_EVAL, OP_EFALLBACK, OP_GATHER, OP_MINSTEP, OP_SDONLY, OP_RESTORE, OP_EXIT };
 enum Stage {
     ST_INIT_FF, ST_INIT_F, ST_INIT_G, ST_ITER, ST_TRIAL, ST_SD, ST_QUAD, ST_QUAD_EVAL, ST_QUAD_DONE, ST_QUAD_AT,
     ST_LS_DONE, ST_ACCEPT, ST_REC_STEP, ST_REC_EVAL, ST_REC_GATHER, ST_FINAL, ST_FINAL_DONE, ST_FINISH
 };
 
-// One minimization run by a cluster of G blocks (blk = index within it).
-// QUAD: compiled with the quadratic line-search stages (a separate kernel, so
-// the backtracking kernel carries none of their state in registers).
-// WIDE: the wide per-bead gather (one bead per thread). BATCH: the batched
-// launch's passes ended by completions.
-template <bool MIXED, bool QUAD, bool WIDE, bool BATCH>
-__device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *lds, int blk, int G,
-                                                      int *done = nullptr, int suspend_done = 0) {
-    __shared__ unsigned long long accl[24];
-    Cg<MIXED> K(A, lds, accl, blk, G);
-    if (BATCH) K.done_ctr = done;
-    double *R = A.out;
-    const bool leader = (K.blk == 0 && K.tid == 0);
-    if (leader) R[R_T0] = (double)wall_clock64();
-#define FB(i) ((i) ? A.F1 : A.F0)
-#define SB(i) ((i) ? A.S1 : A.S0)
-    unsigned flags = 0;
-    int nEC = 0, nFC = 0, nIter = 0, nEE = 0, nSM = 0, nRec = 0;
-    long long trn = 0;
-    double gradInf = INFINITY, relE = INFINITY;
-    bool after = true;   // compute energiesAfter / output force
-    bool suspended = false;
-    int cur = 0, sidx = 0;
-    const double *dvec = nullptr;
-    double maxF = 0, FF = 0, FFp = 0, FFcur = 0;
-    double E0 = 0, prevEnergy = 0, lastFDotF = 0, slope = 0;
-    int safeMode = 0;
-    double minimumE = INFINITY;
-    bool haveMin = false;
-    double lam = 0, newE = 0, armijo = 0, reducedSlope = 0, sdF = 0, stepRec = 0, beta = 0;
+// vectors by number: 0 F0, 1 F1, 2 S0, 3 S1, -1 none
+struct CgState {
+    // the next device work: its kind and positions (PosAny along vector d, or
+    // F + beta d), the gather's output and previous force, the new direction
+    int op, mode, pd, pF, gOut, gPrev, gMove, sNew, ffAfter, saveMin;
+    int nqe, nqf, qb;           // fallback queues of the last evaluation
+    double plam, pbeta;
+    // results of collective work
+    double Eff, Effp, stepRec;
+    // control
+    int stage, status, cur, sidx, dv, dprev, safeMode, haveMin, pendingSpec, after, suspended, quadLS;
+    unsigned flags;
+    int nEC, nFC, nIter, nEE, nSM, nRec, doneSeen;
+    long long trn;
+    double gradInf, relE, maxF, FF, FFp, FFcur, E, xa, E0, prevEnergy, lastFDotF, slope, minimumE, lam, newE, armijo,
+        reducedSlope, sdF, beta, lamEval, Eacc;
     // quadratic line search (quadraticLineSearchV2): trial count, the last
     // rejected trial, the first record, the highest later record, the
     // parabola's bracket, its refinement count, and the last evaluated step
-    bool quadLS = false;
-    int qIter = 0, qRef = 0;
-    double qPrevL = 0, qPrevE = 0, qL0 = 0, qE0 = 0, qMax = 0, qBt = 0;
-    double qx0 = 0, qx1 = 0, qx2 = 0, qy0 = 0, qy1 = 0, qy2 = 0, qLam = 0;
-    double lamEval = 0, Eacc = 0;    // step of the last trial and the energy at the accepted point
-    bool pendingSpec = false;        // an accepted step's s is not formed yet
-    const double *dprev = nullptr;   // the direction s extends
-    double *Snew = nullptr;          // where s goes
-    Eval ev{0.0, 0.0, 0, 0};
-    double Eff = 0, Effp = 0;
-    // the device work of the next turn and its operands
-    int op = OP_EVAL_FF, stage = ST_INIT_FF;
-    PosAny P = PosAny::at(A.x);
-    double *ffout = R + R_EB;
-    double *gOut = nullptr;
-    const double *gPrev = nullptr;
-    bool gMove = false;
-    auto callLimit = [&]() {
-        return (A.energy_call_limit != 0 && nEC > A.energy_call_limit) ||
-               (A.force_call_limit != 0 && nFC > A.force_call_limit);
-    };
-    auto converged = [&]() { return gradInf < A.grad_tol || relE < A.energy_rel_tol; };
-    // Suspension: everything the iterations carry from one to the next; the
-    // vectors (x, forces, directions, minimum-energy backup, trace) stay in
-    // the network's buffers. The phase counter restarts at 0 with cleared
-    // accumulators, which changes no value.
-    auto bufid = [&](const double *q) {
-        return q == A.F0 ? 0.0 : q == A.F1 ? 1.0 : q == A.S0 ? 2.0 : q == A.S1 ? 3.0 : -1.0;
-    };
-    auto bufptr = [&](double id) -> double * {
-        return id == 0.0 ? A.F0 : id == 1.0 ? A.F1 : id == 2.0 ? A.S0 : id == 3.0 ? A.S1 : nullptr;
-    };
-    if (leader) R[R_SUSP] = 0.0;
-    if (A.resume) {
-        const double *S = R + R_RS;
-        flags = (unsigned)S[0]; nEC = (int)S[1]; nFC = (int)S[2]; nIter = (int)S[3]; nEE = (int)S[4];
-        nSM = (int)S[5]; nRec = (int)S[6]; trn = (long long)S[7]; gradInf = S[8]; relE = S[9];
-        cur = (int)S[10]; sidx = (int)S[11]; dvec = bufptr(S[12]); maxF = S[13]; FFcur = S[14]; E0 = S[15];
-        prevEnergy = S[16]; lastFDotF = S[17]; slope = S[18]; safeMode = (int)S[19]; minimumE = S[20];
-        haveMin = S[21] != 0.0; beta = S[22]; pendingSpec = S[23] != 0.0; dprev = bufptr(S[24]);
-        Snew = bufptr(S[25]);
-        op = OP_NONE; stage = ST_ITER;
+    int qIter, qRef;
+    double qPrevL, qPrevE, qL0, qE0, qMax, qBt, qx0, qx1, qx2, qy0, qy1, qy2, qLam;
+
+    __device__ void at_x() { mode = PosAny::X; pd = pF = -1; plam = pbeta = 0.0; }
+    __device__ void line(int d, double l) { mode = PosAny::LINE; pd = d; pF = -1; plam = l; pbeta = 0.0; }
+    __device__ void spec(int F, int d, double b, double l) { mode = PosAny::SPEC; pd = d; pF = F; plam = l; pbeta = b; }
+    __device__ void eval_line(int d, double l, int st) { op = OP_EVAL; line(d, l); stage = st; }
+    __device__ void gather_step(int st) {
+        op = OP_GATHER;
+        gOut = 1 - cur; gPrev = cur; gMove = 1;
+        stage = st;
     }
-    auto trace = [&](double l, double e, double b) {
-        if (leader && trn < A.tr_cap) {
-            A.tr_lam[trn] = l; A.tr_e[trn] = e; A.tr_mf[trn] = gradInf; A.tr_beta[trn] = b;
-            A.tr_safe[trn] = safeMode;
-        }
-        trn++;
+    __device__ void reset() { dv = cur; lastFDotF = FFcur; slope = FFcur; }   // resetCGParams
+    __device__ void stop(int code) { status = code; after = 0; stage = ST_FINISH; }
+};
+
+// One block's thread 0: the control flow from the work just done to the next
+// (s.op). Returns nothing; s.op = OP_EXIT at the end.
+template <bool QUAD, bool BATCH>
+__device__ __attribute__((always_inline)) void cg_control(CgState &s, const CgArgs &A, bool leader, int suspend_done) {
+    double *R = A.out;
+    auto callLimit = [&]() {
+        return (A.energy_call_limit != 0 && s.nEC > A.energy_call_limit) ||
+               (A.force_call_limit != 0 && s.nFC > A.force_call_limit);
     };
-
-    for (;;) {
-        // ---- device work
-        bool ok = true;
-        switch (op) {
-        case OP_EVAL_FF:
-            ok = K.eval_ff(P, ffout, Eff, Effp);
-            break;
-        case OP_EVAL:
-        case OP_SDONLY: {
-            const int p1 = K.ph;
-            mdy_xsum sd;
-            mdy_xs_zero(&sd);
-            if (P.mode == PosAny::SPEC) spec_direction(K, P.F, P.d, P.beta, Snew, sd);
-            if (op == OP_EVAL) {
-                ok = K.eval(P, ev, P.mode == PosAny::SPEC, sd);
-                nEE++;
-            } else {   // s.F only (max|F| = 0: no trial)
-                block_reduce_xsum(sd, K.ldsl());
-                K.acc_push(K.accs(p1) + kAcc1, sd);
-                ok = K.sync(PK_REDUCE);
-                if (ok) sdF = K.acc_value(K.accs(p1) + kAcc1);
-            }
-            break;
+    auto converged = [&]() { return s.gradInf < A.grad_tol || s.relE < A.energy_rel_tol; };
+    auto trace = [&](double l, double e, double b) {
+        if (leader && s.trn < A.tr_cap) {
+            A.tr_lam[s.trn] = l; A.tr_e[s.trn] = e; A.tr_mf[s.trn] = s.gradInf; A.tr_beta[s.trn] = b;
+            A.tr_safe[s.trn] = s.safeMode;
         }
-        case OP_GATHER:
-            if (__builtin_expect(ev.nqf != 0, 0)) ok = K.force_fallback(P, ev);
-            if (ok && !K.status) ok = K.template gather<WIDE, BATCH>(gOut, gPrev, gMove, P.d, P.lam, maxF, FF, FFp);
-            break;
-        case OP_MINSTEP: {
-            // MController::moveAlongDirectionLimitingBeadMove_: step = min maxDist/|d_i|
-            double v[1] = {INFINITY};
-            for (int o = K.gtid; o < A.D.ndof; o += K.gs) v[0] = smin(v[0], A.max_dist / fabs(dvec[o]));
-            block_reduce<1>(v, lds, 0u, 0x1u);
-            const int p1 = K.ph;
-            if (K.tid == 0) K.red(p1)[(size_t)K.blk * kRed] = v[0];
-            ok = K.sync(PK_REDUCE);
-            if (ok) {
-                grid_partials_reduce<1>(K.red(p1), K.G, v, lds, 0u, 0x1u);
-                stepRec = v[0];
-            }
-            break;
-        }
-        case OP_RESTORE:
-            for (int o = K.gtid; o < A.D.ndof; o += K.gs) A.x[o] = A.xmin[o];
-            ok = K.sync(PK_RESTORE);
-            break;
-        default:
-            break;
-        }
-        if (__builtin_expect(!ok, 0)) goto aborted;
-        op = OP_NONE;
-        if (__builtin_expect(K.status != 0, 0) && stage != ST_FINISH) { after = false; stage = ST_FINISH; }
-
-        // ---- control
-    control:
-        switch (stage) {
+        s.trn++;
+    };
+    s.op = OP_NONE;
+    if (__builtin_expect(s.status != 0, 0) && s.stage != ST_FINISH) { s.after = 0; s.stage = ST_FINISH; }
+    while (s.op == OP_NONE) {
+        switch (s.stage) {
         case ST_INIT_FF:   // energiesBefore = computeIndividualEnergies(x); E(x) for the first line search
-            nEC++; nEE++;
-            E0 = Eff; prevEnergy = Effp;
-            op = OP_EVAL; P = PosAny::at(A.x); stage = ST_INIT_F;
+            s.nEC++; s.nEE++;
+            s.E0 = s.Eff; s.prevEnergy = s.Effp;
+            s.op = OP_EVAL; s.at_x(); s.stage = ST_INIT_F;
             break;
         case ST_INIT_F:    // forces at x
-            op = OP_GATHER; gOut = FB(cur); gPrev = nullptr; gMove = false; stage = ST_INIT_G;
+            s.op = OP_GATHER; s.gOut = s.cur; s.gPrev = -1; s.gMove = 0; s.stage = ST_INIT_G;
             break;
         case ST_INIT_G:
-            nFC++;
-            gradInf = maxF;
-            if (__builtin_expect(!isfinite(gradInf), 0)) { K.status = MDY_ERR_NONFINITE; after = false; stage = ST_FINISH; break; }
-            FFcur = FF;
-            dvec = FB(cur); lastFDotF = FF; slope = FF;   // resetCGParams
-            stage = ST_ITER;
+            s.nFC++;
+            s.gradInf = s.maxF;
+            if (__builtin_expect(!isfinite(s.gradInf), 0)) { s.stop(MDY_ERR_NONFINITE); break; }
+            s.FFcur = s.FF;
+            s.reset();
+            s.stage = ST_ITER;
             break;
         case ST_ITER:
             if (callLimit() || converged()) {
-                if (callLimit() && haveMin && A.report_call_limit) op = OP_RESTORE;
-                stage = ST_FINAL;
+                if (callLimit() && s.haveMin && A.report_call_limit) s.op = OP_RESTORE;
+                s.stage = ST_FINAL;
                 break;
             }
-            if ((A.suspend_calls > 0 && nFC >= A.suspend_calls) ||
-                (BATCH && suspend_done > 0 && K.done_seen >= suspend_done)) {   // this pass ends; the next resumes here
+            if ((A.suspend_calls > 0 && s.nFC >= A.suspend_calls) ||
+                (BATCH && suspend_done > 0 && s.doneSeen >= suspend_done)) {   // this pass ends; the next resumes here
                 if (leader) {
                     double *S = R + R_RS;
-                    S[0] = flags; S[1] = nEC; S[2] = nFC; S[3] = nIter; S[4] = nEE; S[5] = nSM; S[6] = nRec;
-                    S[7] = (double)trn; S[8] = gradInf; S[9] = relE; S[10] = cur; S[11] = sidx; S[12] = bufid(dvec);
-                    S[13] = maxF; S[14] = FFcur; S[15] = E0; S[16] = prevEnergy; S[17] = lastFDotF; S[18] = slope;
-                    S[19] = safeMode; S[20] = minimumE; S[21] = haveMin ? 1.0 : 0.0; S[22] = beta;
-                    S[23] = pendingSpec ? 1.0 : 0.0; S[24] = bufid(dprev); S[25] = bufid(Snew);
+                    S[0] = s.flags; S[1] = s.nEC; S[2] = s.nFC; S[3] = s.nIter; S[4] = s.nEE; S[5] = s.nSM;
+                    S[6] = s.nRec; S[7] = (double)s.trn; S[8] = s.gradInf; S[9] = s.relE; S[10] = s.cur; S[11] = s.sidx;
+                    S[12] = s.dv; S[13] = s.maxF; S[14] = s.FFcur; S[15] = s.E0; S[16] = s.prevEnergy;
+                    S[17] = s.lastFDotF; S[18] = s.slope; S[19] = s.safeMode; S[20] = s.minimumE; S[21] = s.haveMin;
+                    S[22] = s.beta; S[23] = s.pendingSpec; S[24] = s.dprev; S[25] = s.sNew;
                     R[R_SUSP] = 1.0;
                 }
-                suspended = true;
-                after = false;
-                stage = ST_FINISH;
+                s.suspended = 1;
+                s.after = 0;
+                s.stage = ST_FINISH;
                 break;
             }
-            nIter++;
-            armijo = safeMode ? 0.0 : 0.4;
-            quadLS = QUAD && A.line_search == MDY_LS_QUADRATIC && !safeMode;
-            qIter = 0;
-            qMax = -INFINITY;
-            lam = 0.0; newE = 0.0;
-            if (maxF != 0.0) {
-                lam = smin(A.lambda_max, A.max_dist / maxF);
-                nEC++;   // currentEnergy = computeEnergy(x): E0, known bitwise from the accepting trial
-                op = OP_EVAL;
-                P = pendingSpec ? PosAny::spec(A.x, FB(cur), dprev, beta, lam) : PosAny::line(A.x, dvec, lam);
-                reducedSlope = armijo * slope;
-                stage = ST_TRIAL;
-            } else if (pendingSpec) {
-                op = OP_SDONLY; P = PosAny::spec(A.x, FB(cur), dprev, beta, 0.0); stage = ST_SD;
+            s.nIter++;
+            s.armijo = s.safeMode ? 0.0 : 0.4;
+            s.quadLS = QUAD && A.line_search == MDY_LS_QUADRATIC && !s.safeMode;
+            s.qIter = 0;
+            s.qMax = -INFINITY;
+            s.lam = 0.0; s.newE = 0.0;
+            if (s.maxF != 0.0) {
+                s.lam = smin(A.lambda_max, A.max_dist / s.maxF);
+                s.nEC++;   // currentEnergy = computeEnergy(x): E0, known bitwise from the accepting trial
+                s.op = OP_EVAL;
+                if (s.pendingSpec) s.spec(s.cur, s.dprev, s.beta, s.lam);
+                else s.line(s.dv, s.lam);
+                s.reducedSlope = s.armijo * s.slope;
+                s.stage = ST_TRIAL;
+            } else if (s.pendingSpec) {
+                s.op = OP_SDONLY; s.spec(s.cur, s.dprev, s.beta, 0.0); s.stage = ST_SD;
             } else {
-                stage = ST_LS_DONE;
+                s.stage = ST_LS_DONE;
             }
             break;
         case ST_SD:        // s.F without a trial (max|F| = 0)
-            pendingSpec = false;
-            if (sdF <= 0) { dvec = FB(cur); lastFDotF = FFcur; slope = FFcur; }
-            else { dvec = Snew; slope = sdF; }
-            stage = ST_LS_DONE;
+            s.pendingSpec = 0;
+            s.sdF = s.xa;
+            if (s.sdF <= 0) s.reset();
+            else { s.dv = s.sNew; s.slope = s.sdF; }
+            s.stage = ST_LS_DONE;
             break;
         case ST_TRIAL: {   // one backtracking step
-            if (P.mode == PosAny::SPEC) {
-                pendingSpec = false;
-                sdF = ev.xa;
-                if (sdF <= 0) {   // resetCGParams: redo this trial along F
-                    dvec = FB(cur); lastFDotF = FFcur; slope = FFcur;
-                    reducedSlope = armijo * slope;
-                    op = OP_EVAL; P = PosAny::line(A.x, dvec, lam);
+            if (s.mode == PosAny::SPEC) {
+                s.pendingSpec = 0;
+                s.sdF = s.xa;
+                if (s.sdF <= 0) {   // resetCGParams: redo this trial along F
+                    s.reset();
+                    s.reducedSlope = s.armijo * s.slope;
+                    s.eval_line(s.dv, s.lam, ST_TRIAL);
                     break;
                 }
-                dvec = Snew; slope = sdF;
-                reducedSlope = armijo * slope;
+                s.dv = s.sNew; s.slope = s.sdF;
+                s.reducedSlope = s.armijo * s.slope;
             }
-            double Et = ev.E;
-            nEC++;
-            if (quadLS) {   // CGMethod.hpp:567-617: Armijo slope 0.4, every trial recorded
-                lamEval = lam; Eacc = Et;
-                qIter++;
-                const double idealq = -0.4 * lam * slope;
-                if (idealq > 0) { K.status = MDY_ERR_QUADRATIC; after = false; stage = ST_FINISH; break; }
+            double Et = s.E;
+            s.nEC++;
+            if (QUAD && s.quadLS) {   // CGMethod.hpp:567-617: Armijo slope 0.4, every trial recorded
+                s.lamEval = s.lam; s.Eacc = Et;
+                s.qIter++;
+                const double idealq = -0.4 * s.lam * s.slope;
+                if (idealq > 0) { s.stop(MDY_ERR_QUADRATIC); break; }
                 bool conv = false;
-                if (Et - E0 <= idealq) conv = true;
-                else { qPrevL = lam; qPrevE = Et; lam *= 0.5; }
+                if (Et - s.E0 <= idealq) conv = true;
+                else { s.qPrevL = s.lam; s.qPrevE = Et; s.lam *= 0.5; }
                 double recL, recE;
-                if (lam <= 0.0 || lam <= 1e-8) { conv = true; lam = 0.0; recL = 0.0; recE = E0; }
-                else if (conv) { recL = lam; recE = Et; }
-                else { recL = qPrevL; recE = qPrevE; }
-                if (qIter == 1) { qL0 = recL; qE0 = recE; }
-                else qMax = fmax(qMax, recE);
-                if (!conv) { op = OP_EVAL; P = PosAny::line(A.x, dvec, lam); break; }
-                newE = Et;
+                if (s.lam <= 0.0 || s.lam <= 1e-8) { conv = true; s.lam = 0.0; recL = 0.0; recE = s.E0; }
+                else if (conv) { recL = s.lam; recE = Et; }
+                else { recL = s.qPrevL; recE = s.qPrevE; }
+                if (s.qIter == 1) { s.qL0 = recL; s.qE0 = recE; }
+                else s.qMax = fmax(s.qMax, recE);
+                if (!conv) { s.eval_line(s.dv, s.lam, ST_TRIAL); break; }
+                s.newE = Et;
                 // CGMethod.hpp:621-645: refine when an earlier record lies above
                 // the accepted energy; the third point is the first record
-                if (lam > 0.0 && qIter > 1 && Et < E0 && Et < qMax) {
-                    qx0 = 0.0; qx1 = lam; qx2 = qL0; qy0 = E0; qy1 = Et; qy2 = qE0;
-                    qBt = lam; qRef = 0;
-                    stage = ST_QUAD;
+                if (s.lam > 0.0 && s.qIter > 1 && Et < s.E0 && Et < s.qMax) {
+                    s.qx0 = 0.0; s.qx1 = s.lam; s.qx2 = s.qL0; s.qy0 = s.E0; s.qy1 = Et; s.qy2 = s.qE0;
+                    s.qBt = s.lam; s.qRef = 0;
+                    s.stage = ST_QUAD;
                 } else {
-                    stage = ST_LS_DONE;
+                    s.stage = ST_LS_DONE;
                 }
                 break;
             }
-            const double ideal = -reducedSlope * lam;
+            const double ideal = -s.reducedSlope * s.lam;
             bool done = false;
-            if (lam < 0 || ideal > 0) { done = true; lam = 0.0; }
-            const double change = Et - E0;
+            if (s.lam < 0 || ideal > 0) { done = true; s.lam = 0.0; }
+            const double change = Et - s.E0;
             if (change <= ideal) done = true;
-            else lam *= 0.5;
-            if (lam <= 0.0 || lam <= 1e-8) { done = true; lam = 0.0; Et = E0; }
-            if (!done) { op = OP_EVAL; P = PosAny::line(A.x, dvec, lam); break; }
-            newE = Et;
-            if (lam != 0.0) {   // accepted: gather at once (ST_LS_DONE's accepting branch)
-                op = OP_GATHER; P = PosAny::line(A.x, dvec, lam);
-                gOut = FB(1 - cur); gPrev = FB(cur); gMove = true;
-                stage = ST_ACCEPT;
-            } else {
-                stage = ST_LS_DONE;
-            }
+            else s.lam *= 0.5;
+            if (s.lam <= 0.0 || s.lam <= 1e-8) { done = true; s.lam = 0.0; Et = s.E0; }
+            if (!done) { s.eval_line(s.dv, s.lam, ST_TRIAL); break; }
+            s.newE = Et;
+            s.stage = ST_LS_DONE;
             break;
         }
         case ST_QUAD: {   // quadraticoptimization, CGMethod.hpp:663-765 (at most 200 refinements)
             if constexpr (!QUAD) break;
-            if (qRef >= 200) { qLam = qx1; stage = ST_QUAD_DONE; break; }
-            qRef++;
-            const double d = (qx0 - qx1) * (qx0 - qx2) * (qx1 - qx2);
-            const double a = qy0 * (qx1 - qx2) - qy1 * (qx0 - qx2) + qy2 * (qx0 - qx1);
-            const double b = -(qy0 * (qx1 + qx2) * (qx1 - qx2) - qy1 * (qx0 + qx2) * (qx0 - qx2) +
-                               qy2 * (qx0 + qx1) * (qx0 - qx1));
-            qLam = -b / (2 * a);
-            if (fabs(qLam - qx1) / qx1 < 1e-3) { stage = ST_QUAD_DONE; break; }
-            if (a / d < 0) { qLam = qBt; stage = ST_QUAD_DONE; break; }
-            op = OP_EVAL; P = PosAny::line(A.x, dvec, qLam); stage = ST_QUAD_EVAL;
+            if (s.qRef >= 200) { s.qLam = s.qx1; s.stage = ST_QUAD_DONE; break; }
+            s.qRef++;
+            const double d = (s.qx0 - s.qx1) * (s.qx0 - s.qx2) * (s.qx1 - s.qx2);
+            const double a = s.qy0 * (s.qx1 - s.qx2) - s.qy1 * (s.qx0 - s.qx2) + s.qy2 * (s.qx0 - s.qx1);
+            const double b = -(s.qy0 * (s.qx1 + s.qx2) * (s.qx1 - s.qx2) - s.qy1 * (s.qx0 + s.qx2) * (s.qx0 - s.qx2) +
+                               s.qy2 * (s.qx0 + s.qx1) * (s.qx0 - s.qx1));
+            s.qLam = -b / (2 * a);
+            if (fabs(s.qLam - s.qx1) / s.qx1 < 1e-3) { s.stage = ST_QUAD_DONE; break; }
+            if (a / d < 0) { s.qLam = s.qBt; s.stage = ST_QUAD_DONE; break; }
+            s.eval_line(s.dv, s.qLam, ST_QUAD_EVAL);
             break;
         }
         case ST_QUAD_EVAL: {
             if constexpr (!QUAD) break;
-            const double eq = ev.E;
-            nEC++;
-            lamEval = qLam; Eacc = eq;
-            if (fabs(eq - qy1) / qy1 < 1e-3) { stage = ST_QUAD_DONE; break; }
-            if (qLam < qx1) {
-                if (eq < qy0 && eq < qy1) { qx1 = qLam; qy1 = eq; }
-                else { qx0 = qLam; qy0 = eq; }
-            } else if (qx1 < qLam) {
-                if (eq < qy1 && eq < qy2) { qx1 = qLam; qy1 = eq; }
-                else { qx2 = qLam; qy2 = eq; }
+            const double eq = s.E;
+            s.nEC++;
+            s.lamEval = s.qLam; s.Eacc = eq;
+            if (fabs(eq - s.qy1) / s.qy1 < 1e-3) { s.stage = ST_QUAD_DONE; break; }
+            if (s.qLam < s.qx1) {
+                if (eq < s.qy0 && eq < s.qy1) { s.qx1 = s.qLam; s.qy1 = eq; }
+                else { s.qx0 = s.qLam; s.qy0 = eq; }
+            } else if (s.qx1 < s.qLam) {
+                if (eq < s.qy1 && eq < s.qy2) { s.qx1 = s.qLam; s.qy1 = eq; }
+                else { s.qx2 = s.qLam; s.qy2 = eq; }
             } else {
-                qLam = qx1; stage = ST_QUAD_DONE; break;
+                s.qLam = s.qx1; s.stage = ST_QUAD_DONE; break;
             }
-            stage = ST_QUAD;
+            s.stage = ST_QUAD;
             break;
         }
         case ST_QUAD_DONE:   // newE stays the backtracking energy (CGMethod.hpp:655)
             if constexpr (!QUAD) break;
-            lam = (qLam <= 0.0 || qLam <= 1e-8) ? 0.0 : qLam;
-            if (lam != 0.0 && lam != lamEval) {   // forces and energy at the accepted point
-                op = OP_EVAL; P = PosAny::line(A.x, dvec, lam); stage = ST_QUAD_AT;
+            s.lam = (s.qLam <= 0.0 || s.qLam <= 1e-8) ? 0.0 : s.qLam;
+            if (s.lam != 0.0 && s.lam != s.lamEval) {   // forces and energy at the accepted point
+                s.eval_line(s.dv, s.lam, ST_QUAD_AT);
                 break;
             }
-            stage = ST_LS_DONE;
+            s.stage = ST_LS_DONE;
             break;
         case ST_QUAD_AT:
             if constexpr (!QUAD) break;
-            Eacc = ev.E;
-            stage = ST_LS_DONE;
+            s.Eacc = s.E;
+            s.stage = ST_LS_DONE;
             break;
         case ST_LS_DONE:
-            if (lam == 0.0) {
+            if (s.lam == 0.0) {
                 if (!A.try_recover) {
-                    flags |= MDY_ERROR_LINESEARCH;
-                    trace(0.0, newE, 0.0);
-                    after = false;   // the reference returns before energiesAfter / ptrOutForce
-                    stage = ST_FINISH;
-                } else if (safeMode) {
-                    op = OP_MINSTEP; stage = ST_REC_STEP;
+                    s.flags |= MDY_ERROR_LINESEARCH;
+                    trace(0.0, s.newE, 0.0);
+                    s.after = 0;   // the reference returns before energiesAfter / ptrOutForce
+                    s.stage = ST_FINISH;
+                } else if (s.safeMode) {
+                    s.op = OP_MINSTEP; s.stage = ST_REC_STEP;
                 } else {
-                    dvec = FB(cur); lastFDotF = FFcur; slope = FFcur;
-                    safeMode = 1;
-                    nSM++;
-                    trace(0.0, newE, 0.0);
-                    stage = ST_ITER;
+                    s.reset();
+                    s.safeMode = 1;
+                    s.nSM++;
+                    trace(0.0, s.newE, 0.0);
+                    s.stage = ST_ITER;
                 }
             } else {   // accepted: the force slots hold the forces at x + lam*d
-                op = OP_GATHER; P = PosAny::line(A.x, dvec, lam);
-                gOut = FB(1 - cur); gPrev = FB(cur); gMove = true;
-                stage = ST_ACCEPT;
+                s.line(s.dv, s.lam);
+                s.gather_step(ST_ACCEPT);
             }
             break;
         case ST_REC_STEP:
-            if (stepRec == INFINITY) { K.status = MDY_ERR_RECOVERY; after = false; stage = ST_FINISH; break; }
-            op = OP_EVAL; P = PosAny::line(A.x, dvec, stepRec); stage = ST_REC_EVAL;
+            if (s.stepRec == INFINITY) { s.stop(MDY_ERR_RECOVERY); break; }
+            s.eval_line(s.dv, s.stepRec, ST_REC_EVAL);
             break;
         case ST_REC_EVAL:
-            op = OP_GATHER; gOut = FB(1 - cur); gPrev = FB(cur); gMove = true; stage = ST_REC_GATHER;
+            s.gather_step(ST_REC_GATHER);
             break;
         case ST_REC_GATHER:
-            nFC++; nRec++;
-            gradInf = maxF;
-            if (__builtin_expect(!isfinite(gradInf), 0)) { K.status = MDY_ERR_NONFINITE; after = false; stage = ST_FINISH; break; }
-            cur = 1 - cur;
-            FFcur = FF;
-            dvec = FB(cur); lastFDotF = FF; slope = FF;
-            safeMode = 0;
-            E0 = ev.E;   // computeEnergy at the moved coordinates
-            trace(0.0, newE, 0.0);
-            stage = ST_ITER;
+            s.nFC++; s.nRec++;
+            s.gradInf = s.maxF;
+            if (__builtin_expect(!isfinite(s.gradInf), 0)) { s.stop(MDY_ERR_NONFINITE); break; }
+            s.cur = 1 - s.cur;
+            s.FFcur = s.FF;
+            s.reset();
+            s.safeMode = 0;
+            s.E0 = s.E;   // computeEnergy at the moved coordinates
+            trace(0.0, s.newE, 0.0);
+            s.stage = ST_ITER;
             break;
         case ST_ACCEPT: {
-            nFC++;
-            gradInf = maxF;
-            if (__builtin_expect(!isfinite(gradInf), 0)) { K.status = MDY_ERR_NONFINITE; after = false; stage = ST_FINISH; break; }
-            E0 = quadLS ? Eacc : newE;   // E(x) of the next line search
-            relE = fabs(newE - prevEnergy) / fabs(prevEnergy);
-            prevEnergy = newE;
-            const double newGrad = FF, prevGrad = FFp;
-            beta = 0.0;
-            if (A.method == MDY_CG_FLETCHER_RIEVES) beta = newGrad / lastFDotF;
-            else if (A.method == MDY_CG_POLAK_RIBIERE) beta = smax(0.0, (newGrad - prevGrad) / lastFDotF);
-            cur = 1 - cur;
-            FFcur = newGrad;
-            dprev = dvec; Snew = SB(1 - sidx); sidx = 1 - sidx;
-            pendingSpec = true;   // s = F + beta*d is formed with the next trial
+            s.nFC++;
+            s.gradInf = s.maxF;
+            if (__builtin_expect(!isfinite(s.gradInf), 0)) { s.stop(MDY_ERR_NONFINITE); break; }
+            s.E0 = QUAD && s.quadLS ? s.Eacc : s.newE;   // E(x) of the next line search
+            s.relE = fabs(s.newE - s.prevEnergy) / fabs(s.prevEnergy);
+            s.prevEnergy = s.newE;
+            const double newGrad = s.FF, prevGrad = s.FFp;
+            s.beta = 0.0;
+            if (A.method == MDY_CG_FLETCHER_RIEVES) s.beta = newGrad / s.lastFDotF;
+            else if (A.method == MDY_CG_POLAK_RIBIERE) s.beta = smax(0.0, (newGrad - prevGrad) / s.lastFDotF);
+            s.cur = 1 - s.cur;
+            s.FFcur = newGrad;
+            s.dprev = s.dv; s.sNew = 2 + (1 - s.sidx); s.sidx = 1 - s.sidx;
+            s.pendingSpec = 1;   // s = F + beta*d is formed with the next trial
             // forceBelowRelaxedTolerance(10) && numIter > forceCallLimit/2 -> keep lowest-energy coordinates
-            if (maxF <= 10 * A.grad_tol && nIter > A.force_call_limit / 2 && newE <= minimumE) {
-                minimumE = newE;
-                haveMin = true;
-                for (int o = K.gtid; o < A.D.ndof; o += K.gs) A.xmin[o] = A.x[o];
+            if (s.maxF <= 10 * A.grad_tol && s.nIter > A.force_call_limit / 2 && s.newE <= s.minimumE) {
+                s.minimumE = s.newE;
+                s.haveMin = 1;
+                s.saveMin = 1;   // copied before the next work moves anything
             }
-            if (A.method != MDY_CG_STEEPEST) lastFDotF = newGrad;
-            trace(lam, newE, beta);
-            stage = ST_ITER;
-            goto control;   // no device work in between
+            if (A.method != MDY_CG_STEEPEST) s.lastFDotF = newGrad;
+            trace(s.lam, s.newE, s.beta);
+            s.stage = ST_ITER;
+            break;
         }
         case ST_FINAL:
-            if (after) { op = OP_EVAL_FF; P = PosAny::at(A.x); ffout = R + R_EA; stage = ST_FINAL_DONE; }
-            else stage = ST_FINISH;
+            if (s.after) { s.op = OP_EVAL_FF; s.at_x(); s.ffAfter = 1; s.stage = ST_FINAL_DONE; }
+            else s.stage = ST_FINISH;
             break;
         case ST_FINAL_DONE:
-            nEC++; nEE++;
-            stage = ST_FINISH;
+            s.nEC++; s.nEE++;
+            s.stage = ST_FINISH;
             break;
-        default:
+        default:   // ST_FINISH
+            s.op = OP_EXIT;
             break;
         }
-        if (stage == ST_FINISH && op == OP_NONE) break;
+    }
+}
+
+// One minimization run by a cluster of G blocks (blk = index within it).
+// QUAD: compiled with the quadratic line-search stages.
+// BATCH: the batched launch's passes ended by completions.
+template <bool MIXED, bool QUAD, bool BATCH>
+__device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *lds, int blk, int G,
+                                                      int *done = nullptr, int suspend_done = 0) {
+    __shared__ unsigned long long accl[24];
+    __shared__ XBlock xb;
+    __shared__ CgState S;
+    xblock_zero(xb);
+    atan_table_fill();
+    Cg<MIXED> K(A, lds, xb, accl, blk, G);
+    if (BATCH) K.done_ctr = done;
+    double *R = A.out;
+    const int tid = K.tid;
+    const bool leader = (K.blk == 0 && tid == 0);
+    if (leader) { R[R_T0] = (double)wall_clock64(); R[R_SUSP] = 0.0; }
+    if (tid == 0) {
+        // everything the iterations carry from one to the next starts here, or
+        // from what a suspension saved; the vectors (x, forces, directions,
+        // minimum-energy backup, trace) stay in the network's buffers. The phase
+        // counter restarts at 0 with cleared accumulators, which changes no value.
+        S = CgState{};
+        S.op = OP_EVAL_FF; S.at_x(); S.stage = ST_INIT_FF;
+        S.gradInf = S.relE = S.minimumE = INFINITY;
+        S.after = 1;
+        S.dv = S.dprev = S.sNew = -1;
+        if (A.resume) {
+            const double *Q = R + R_RS;
+            S.flags = (unsigned)Q[0]; S.nEC = (int)Q[1]; S.nFC = (int)Q[2]; S.nIter = (int)Q[3]; S.nEE = (int)Q[4];
+            S.nSM = (int)Q[5]; S.nRec = (int)Q[6]; S.trn = (long long)Q[7]; S.gradInf = Q[8]; S.relE = Q[9];
+            S.cur = (int)Q[10]; S.sidx = (int)Q[11]; S.dv = (int)Q[12]; S.maxF = Q[13]; S.FFcur = Q[14]; S.E0 = Q[15];
+            S.prevEnergy = Q[16]; S.lastFDotF = Q[17]; S.slope = Q[18]; S.safeMode = (int)Q[19]; S.minimumE = Q[20];
+            S.haveMin = (int)Q[21]; S.beta = Q[22]; S.pendingSpec = (int)Q[23]; S.dprev = (int)Q[24];
+            S.sNew = (int)Q[25];
+            S.op = OP_NONE; S.stage = ST_ITER;
+        }
+    }
+    auto vec = [&](int id) -> double * {
+        return id == 0 ? A.F0 : id == 1 ? A.F1 : id == 2 ? A.S0 : id == 3 ? A.S1 : nullptr;
+    };
+    auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    auto unid = [](double v) {
+        return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                                __builtin_amdgcn_readfirstlane(__double2loint(v)));
+    };
+    for (;;) {
+        __syncthreads();
+        const int op = uni(S.op);
+        if (__builtin_expect(uni(S.saveMin), 0))   // read back by the same threads (OP_RESTORE)
+            for (int o = K.gtid; o < A.D.ndof; o += K.gs) A.xmin[o] = A.x[o];
+        if (op == OP_EXIT) break;
+        const PosAny P{A.x, vec(uni(S.pd)), vec(uni(S.pF)), unid(S.plam), unid(S.pbeta), uni(S.mode)};
+        bool ok = true, failed = false;
+        if (op == OP_GATHER) {
+            const int nqf = uni(S.nqf);
+            if (__builtin_expect(nqf != 0, 0)) {
+                ok = K.force_fallback(P, nqf, uni(S.qb));
+                if (!ok) break;
+                failed = K.status != 0;
+            }
+        }
+        if (__builtin_expect((op == OP_EVAL || op == OP_GATHER || op == OP_SDONLY) && !failed, 1)) {
+            if (op != OP_GATHER) {
+                if (P.mode == PosAny::SPEC) spec_direction(K, P.F, P.d, P.beta, vec(uni(S.sNew)));
+                if (op == OP_EVAL) K.eval(P);
+            } else {
+                K.template gather<BATCH>(vec(uni(S.gOut)), vec(uni(S.gPrev)), uni(S.gMove) != 0, P.d, P.lam);
+            }
+            // end of the phase: the block's sums, the barrier, and what the
+            // decision reads; the other waves wait at the top of the loop
+            const int p1 = K.ph;
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (tid < 64) {
+                K.acc_push(p1);
+                ok = K.barrier(op == OP_EVAL ? PK_EVAL : op == OP_GATHER ? PK_GATHER : PK_REDUCE);
+                const double v = K.acc_fetch(p1, A.qn + 4 * (p1 % 3), A.qn + 4 * (p1 % 3) + 1);
+                const double v1 = __shfl(v, 1, 64);
+                if (tid == 0) {
+                    if (op == OP_GATHER) {
+                        S.maxF = __longlong_as_double((long long)accl[kAccMax]);
+                        S.FF = v;
+                        S.FFp = S.gPrev >= 0 ? v1 : 0.0;
+                        if (BATCH) S.doneSeen = (int)accl[kAccDone];
+                    } else {
+                        S.xa = v1;
+                        if (op == OP_EVAL) {
+                            const int nqe = (int)accl[17], nqf = (int)accl[18];
+                            S.nEE++;
+                            S.E = v;
+                            S.nqe = nqe; S.nqf = nqf; S.qb = p1 % 3;
+                            if (__builtin_expect(nqe > kQueueCap || nqf > kQueueCap, 0)) S.status = MDY_ERR_CAPACITY;
+                            else if (__builtin_expect(nqe > 0, 0)) S.op = OP_EFALLBACK;
+                        }
+                    }
+                }
+            }
+            K.ph++;
+        } else if (op != OP_NONE && op != OP_GATHER) {
+            // collective work: every thread takes part beyond the barrier
+            double Eff = 0.0, Effp = 0.0, step = 0.0;
+            if (op == OP_EVAL_FF) {
+                ok = K.eval_ff(P, R + (uni(S.ffAfter) ? R_EA : R_EB), Eff, Effp);
+            } else if (op == OP_EFALLBACK) {
+                ok = K.energy_fallback(P, K.dv(uni(S.qb)), uni(S.nqe), uni(S.qb));
+            } else if (op == OP_MINSTEP) {
+                // MController::moveAlongDirectionLimitingBeadMove_: step = min maxDist/|d_i|
+                const double *dvec = vec(uni(S.dv));
+                double v[1] = {INFINITY};
+                for (int o = K.gtid; o < A.D.ndof; o += K.gs) v[0] = smin(v[0], A.max_dist / fabs(dvec[o]));
+                block_reduce<1>(v, lds, 0u, 0x1u);
+                const int p1 = K.ph;
+                if (tid == 0) K.red(p1)[(size_t)K.blk * kRed] = v[0];
+                ok = K.sync(PK_REDUCE);
+                if (ok) {
+                    grid_partials_reduce<1>(K.red(p1), K.G, v, lds, 0u, 0x1u);
+                    step = v[0];
+                }
+            } else {   // OP_RESTORE
+                for (int o = K.gtid; o < A.D.ndof; o += K.gs) A.x[o] = A.xmin[o];
+                ok = K.sync(PK_RESTORE);
+            }
+            if (tid == 0) {
+                S.Eff = Eff; S.Effp = Effp; S.stepRec = step;
+                if (op == OP_EFALLBACK) {
+                    double e[kNFF + 2];
+                    energy_finish(K.acc_local(kAcc0), nullptr, S.nqe, A.qe + S.qb * kQueueCap, K.qeu(S.qb), e);
+                    S.E = e[kNFF];
+                    S.op = OP_NONE;
+                }
+            }
+        }
+        if (tid == 0) {
+            S.saveMin = 0;
+            if (K.status) S.status = K.status;
+            if (__builtin_expect(!ok, 0)) { S.op = OP_EXIT; S.status = MDY_ERR_TIMEOUT; }
+            else if (S.op != OP_EFALLBACK) cg_control<QUAD, BATCH>(S, A, leader, suspend_done);
+        }
     }
     if (leader) {
-        R[R_FLAGS] = flags; R[R_NEC] = nEC; R[R_NFC] = nFC; R[R_NIT] = nIter; R[R_GIN] = gradInf; R[R_ERC] = relE;
-        R[R_NEE] = nEE; R[R_NSM] = nSM; R[R_NREC] = nRec; R[R_STATUS] = K.status; R[R_TRN] = (double)trn;
-        R[R_LAST] = after ? 1.0 : 0.0; R[R_FOUT] = (double)cur; R[R_NPH] = (double)K.ph;
+        if (S.status == MDY_ERR_TIMEOUT || S.op != OP_EXIT) { R[R_STATUS] = MDY_ERR_TIMEOUT; return; }
+        R[R_FLAGS] = S.flags; R[R_NEC] = S.nEC; R[R_NFC] = S.nFC; R[R_NIT] = S.nIter; R[R_GIN] = S.gradInf;
+        R[R_ERC] = S.relE; R[R_NEE] = S.nEE; R[R_NSM] = S.nSM; R[R_NREC] = S.nRec; R[R_STATUS] = S.status;
+        R[R_TRN] = (double)S.trn; R[R_LAST] = S.after ? 1.0 : 0.0; R[R_FOUT] = (double)S.cur; R[R_NPH] = (double)K.ph;
         // the reference shifts the direction right after an accepted step; here
         // that shift is pending until the next trial
-        R[R_DIR] = bufid(dvec); R[R_PEND] = pendingSpec ? 1.0 : 0.0; R[R_BETA] = beta; R[R_DPREV] = bufid(dprev);
+        R[R_DIR] = S.dv; R[R_PEND] = S.pendingSpec; R[R_BETA] = S.beta; R[R_DPREV] = S.dprev;
         R[R_T1] = (double)wall_clock64();
-        if (BATCH && done && !suspended) atomicAdd(done, 1);
+        if (BATCH && done && !S.suspended) atomicAdd(done, 1);
     }
-    return;
-aborted:
-    if (leader) R[R_STATUS] = MDY_ERR_TIMEOUT;
-#undef FB
-#undef SB
 }
 
 // The arguments come by value: pointers read from the kernel-argument segment
 // are known to be global, so every access is a global (not flat) access.
-// LDS: the shuffle-free exact reductions need block_combine_words(17) words
-constexpr int kCgLds = block_combine_words(17);
-static_assert(kCgLds >= 17 * 16, "LDS of the other block reductions");
+constexpr int kCgLds = 17 * 16;    // words of the block reductions
+constexpr int kCgBlock = 768;      // threads per block: three waves per SIMD
 
-template <bool MIXED, bool QUAD, bool WIDE>
-__global__ void __launch_bounds__(kBlock) k_cg(const CgArgs Av) {
+template <bool MIXED, bool QUAD>
+__global__ void __launch_bounds__(kCgBlock) k_cg(const CgArgs Av) {
     __shared__ double lds[kCgLds];
-    cg_run<MIXED, QUAD, WIDE, false>(Av, lds, blockIdx.x, gridDim.x);
+    cg_run<MIXED, QUAD, false>(Av, lds, blockIdx.x, gridDim.x);
 }
 
 // Batched form: independent minimizations in one cooperative launch. Block b
@@ -910,7 +894,7 @@ __global__ void __launch_bounds__(kBlock) k_cg(const CgArgs Av) {
 // done (nullable): the launch's count of finished minimizations; each
 // suspends at the top of an iteration once the count reaches suspend_done (>0).
 template <bool MIXED, bool QUAD>
-__global__ void __launch_bounds__(kBlock) k_cg_batch(const CgArgs *__restrict__ all, const int2 *__restrict__ map,
+__global__ void __launch_bounds__(kCgBlock) k_cg_batch(const CgArgs *__restrict__ all, const int2 *__restrict__ map,
                                                      int *done, int suspend_done) {
     __shared__ double lds[kCgLds];
     const int2 m = map[blockIdx.x];
@@ -920,18 +904,14 @@ __global__ void __launch_bounds__(kBlock) k_cg_batch(const CgArgs *__restrict__ 
 #else
     CgArgs A = all[m.x];
 #endif
-    cg_run<MIXED, QUAD, false, true>(A, lds, m.y, A.grid, done, suspend_done);
+    cg_run<MIXED, QUAD, true>(A, lds, m.y, A.grid, done, suspend_done);
 }
 
-template <bool WIDE>
-static const void *cg_kernel_w(bool mixed, bool quad) {
-    if (mixed) return quad ? reinterpret_cast<const void *>(k_cg<true, true, WIDE>)
-                           : reinterpret_cast<const void *>(k_cg<true, false, WIDE>);
-    return quad ? reinterpret_cast<const void *>(k_cg<false, true, WIDE>)
-                : reinterpret_cast<const void *>(k_cg<false, false, WIDE>);
-}
-static const void *cg_kernel(bool mixed, bool quad, bool wide) {
-    return wide ? cg_kernel_w<true>(mixed, quad) : cg_kernel_w<false>(mixed, quad);
+static const void *cg_kernel(bool mixed, bool quad) {
+    if (mixed) return quad ? reinterpret_cast<const void *>(k_cg<true, true>)
+                           : reinterpret_cast<const void *>(k_cg<true, false>);
+    return quad ? reinterpret_cast<const void *>(k_cg<false, true>)
+                : reinterpret_cast<const void *>(k_cg<false, false>);
 }
 static const void *cg_batch_kernel(bool mixed, bool quad) {
     if (mixed) return quad ? reinterpret_cast<const void *>(k_cg_batch<true, true>)
@@ -957,11 +937,11 @@ static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, hipStr
     MDY_TRY(ensure(c.tr_lam, c.trace_cap + 1)); MDY_TRY(ensure(c.tr_e, c.trace_cap + 1));
     MDY_TRY(ensure(c.tr_mf, c.trace_cap + 1)); MDY_TRY(ensure(c.tr_beta, c.trace_cap + 1));
     MDY_TRY(ensure(c.tr_safe, c.trace_cap + 1));
-    MDY_TRY(ensure(c.bar, 64 + 16 * (size_t)G));
+    MDY_TRY(ensure(c.bar, 32));
     MDY_TRY(ensure(c.acc, 3 * (size_t)kAccWords));
     MDY_TRY(ensure(c.red, (size_t)3 * G * kRed));
     MDY_TRY(ensure(c.simpson_part, (size_t)6 * G * kRed));
-    MDY_HIP(hipMemsetAsync(c.bar.p, 0, (64 + 16 * (size_t)G) * sizeof(unsigned long long), st));
+    MDY_HIP(hipMemsetAsync(c.bar.p, 0, 32 * sizeof(unsigned long long), st));
     MDY_HIP(hipMemsetAsync(c.qn.p, 0, 16 * sizeof(int), st));
     MDY_HIP(hipMemsetAsync(c.acc.p, 0, 3 * kAccWords * sizeof(unsigned long long), st));
     MDY_HIP(hipMemsetAsync(c.err.p, 0, sizeof(int), st));
@@ -982,6 +962,10 @@ static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, hipStr
     A.grid = G;
     A.suspend_calls = 0;
     A.resume = 0;
+    // Polls go past L2. Below 64 blocks their traffic is small and the shorter wait wins; at 256
+    // blocks 2k clocks measured best (40k cylinders: 81.7 / 79.7 / 85.8 us per iteration at 512 /
+    // 2k / 8k clocks)
+    A.poll_sleep = G > 64 ? 16 : 4;
     return MDY_OK;
 }
 
@@ -1076,17 +1060,20 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
     int per_cu = 0;
     const bool mixed = c.opts.precision == MDY_PREC_MIXED;
     const bool quad = p->line_search == MDY_LS_QUADRATIC;
-    const void *kern = cg_kernel(mixed, quad, false);
-    MDY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, 0));
+    const void *kern = cg_kernel(mixed, quad);
+    MDY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kCgBlock, 0));
     if (per_cu < 1) return MDY_ERR_LAUNCH;
     if (c.opts.blocks_per_cu > 0 && c.opts.blocks_per_cu < per_cu) per_cu = c.opts.blocks_per_cu;
-    const int G = per_cu * c.num_cu;
-    if ((long long)c.nb <= (long long)G * kBlock) {   // one bead per thread in the gather: the wide form
-        int per_cu_w = 0;
-        const void *kw = cg_kernel(mixed, quad, true);
-        MDY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_w, kw, kBlock, 0));
-        if (per_cu_w >= per_cu) kern = kw;
-    }
+    // One lane per thread where the network has fewer lanes than that: a phase's
+    // barrier, and the L2 write-back and invalidation that go with it, get slower
+    // with the block count (500 cylinders: 27 us per iteration on 8 blocks, 43 on
+    // 256; 4k: 43 on 48 blocks, 80 on 256; fewer blocks than lanes / 512 lose more
+    // than they save: 50 on 24). Blocks of 512 threads while one turn covers the
+    // lanes, of 768 (three waves per SIMD) beyond: 200k cylinders 191 against 195.
+    const int lanes = c.dev().n_lanes();
+    const int threads = lanes > c.num_cu * 512 ? kCgBlock : 512;
+    int G = per_cu * c.num_cu;
+    if (c.opts.blocks_per_cu <= 0) G = std::min(G, std::max(8, (lanes + threads - 1) / threads));
     c.coop_blocks = G;
     CgArgs A;
     MDY_TRY(prepare_cg(c, p, d_x, G, st, A));
@@ -1095,7 +1082,7 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
     MDY_HIP(hipEventCreate(&ev.b));
     MDY_HIP(hipEventRecord(ev.a, st));
     void *args[] = {&A};
-    if (hipLaunchCooperativeKernel(kern, dim3(G), dim3(kBlock), args, 0, st) != hipSuccess) return MDY_ERR_LAUNCH;
+    if (hipLaunchCooperativeKernel(kern, dim3(G), dim3(threads), args, 0, st) != hipSuccess) return MDY_ERR_LAUNCH;
     MDY_HIP(hipEventRecord(ev.b, st));
     double R[R_SIZE];
     MDY_HIP(hipMemcpyAsync(R, c.cg_out.p, sizeof(R), hipMemcpyDeviceToHost, st));
@@ -1109,16 +1096,15 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
     return res->status == MDY_ERR_TIMEOUT ? MDY_ERR_TIMEOUT : MDY_OK;
 }
 
-// Batched minimizations: the resident blocks (threads_per_block threads each)
-// are split into one cluster per network, in proportion to its weight (by
-// default its per-evaluation work, interactions + 2 x beads), at least one
-// block each; networks beyond the resident block count run in further
-// launches. With first_pass_calls > 0 the minimizations run in passes: pass
+// Batched minimizations: the resident blocks are split into one cluster per
+// network, in proportion to its weight (by default its per-evaluation work,
+// interactions + 2 x beads), at least one block each; networks beyond the
+// resident block count run in further launches. With first_pass_calls > 0 the minimizations run in passes: pass
 // k suspends every minimization at the top of its first iteration after
 // first_pass_calls * 4^(k-1) force calls (one below its own limit and not
 // converged), saving its state; the next pass resumes it exactly there, with
 // all the blocks shared among the networks still running; a pass in which
-// every network gets at least kUncappedShare blocks runs uncapped. A
+// every network gets at least kUncappedShare threads runs uncapped. A
 // minimization's trajectory does not depend on its cluster size, so the
 // results equal those of one uncapped pass; the passes only move the blocks
 // of finished networks to the slow ones. With first_pass_calls = -k < 0 the
@@ -1128,9 +1114,9 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
 // count once per iteration); the next pass re-splits all the blocks among
 // them, down to one network on the whole grid. cs[i] owns network i's
 // tables, neighbor lists and CG buffers; cs[0] the launch arrays.
-constexpr int kUncappedShare = 64;   // blocks per network at which a pass runs uncapped
-constexpr int kCapGrowth = 4;        // force-call cap growth from one pass to the next (x2 measured slower)
-constexpr int kMaxClusterThreads = 8192;    // threads of one network's cluster at most
+constexpr int kUncappedShare = 4096;   // threads per network at which a pass runs uncapped
+constexpr int kCapGrowth = 4;          // force-call cap growth from one pass to the next (x2 measured slower)
+constexpr int kBatchBlock = 512;       // threads per block while every network gets a block
 int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d_x, double *const *d_force_out,
                        mdy_min_result *res, double *net_ms, int threads_per_block, const double *weights,
                        int first_pass_calls, hipStream_t st, double *total_ms) {
@@ -1139,9 +1125,17 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
     bool quad = false;
     for (int i = 0; i < n; i++) quad = quad || p[i].line_search == MDY_LS_QUADRATIC;
     const void *kern = cg_batch_kernel(mixed, quad);
-    const int tpb = threads_per_block;
-    int per_cu = 0;
-    MDY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, tpb, 0));
+    // Blocks of 512 threads while every network gets one, then half as many, down
+    // to threads_per_block: every block of a launch writes its XCD's L2 back and
+    // invalidates it once per phase of its network, for all the others too, so
+    // fewer and larger ones win (32 networks of 500 to 5000 cylinders, kernel
+    // time: 156 ms with 64 threads, 67 with 256, 53 with 512; 256 networks: 333,
+    // 147, 112). The results do not depend on it.
+    int tpb = std::max(kBatchBlock, threads_per_block), per_cu = 0;
+    for (;; tpb /= 2) {
+        MDY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, tpb, 0));
+        if (tpb <= threads_per_block || per_cu * c0.num_cu >= n) break;
+    }
     if (per_cu < 1) return MDY_ERR_LAUNCH;
     const int Gmax = per_cu * c0.num_cu;
     std::vector<char> resume(n, 0);   // suspended in an earlier pass
@@ -1164,7 +1158,7 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
         const int nt = (int)todo.size();
         // few networks left: each gets enough blocks that a larger cluster
         // would not be faster, so this pass runs them to the end
-        if ((long long)nt * kUncappedShare <= Gmax) cap = 0;
+        if ((long long)nt * kUncappedShare <= (long long)Gmax * tpb) cap = 0;
         for (int lo = 0; lo < nt && rc == MDY_OK; lo += Gmax) {
             const int m = (nt - lo < Gmax) ? nt - lo : Gmax;
             // cluster sizes: proportional shares of the blocks left after one each
@@ -1193,10 +1187,9 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
                           return a.first > b.first || (a.first == b.first && a.second < b.second);
                       });
             for (int k = 0; k < spare - used && k < m; k++) gsz[frac[k].second]++;
-            // a cluster's barrier slows down with its block count: beyond
-            // kMaxClusterThreads threads a network gets no faster
-            const int gcap = std::max(1, kMaxClusterThreads / tpb);
-            for (int i = 0; i < m; i++) gsz[i] = std::min(gsz[i], gcap);
+            // one lane per thread: more blocks only slow a cluster's barrier down
+            for (int i = 0; i < m; i++)
+                gsz[i] = std::min(gsz[i], std::max(1, (cs[todo[lo + i]]->dev().n_lanes() + tpb - 1) / tpb));
             args.assign(m, CgArgs{});
             map.clear();
             for (int i = 0; i < m && rc == MDY_OK; i++) {

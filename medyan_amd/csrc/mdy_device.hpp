@@ -69,8 +69,46 @@ __device__ __forceinline__ Dual xsqrt(Dual a) {
 }
 __device__ __forceinline__ double xfabs(double a) { return fabs(a); }
 __device__ __forceinline__ Dual xfabs(Dual a) { return a.v < 0 ? -a : a; }
-__device__ __forceinline__ double xatan(double a) { return mdy_atan(a); }
-__device__ __forceinline__ Dual xatan(Dual a) { return Dual(mdy_atan(a.v), a.d / (1 + a.v * a.v)); }
+// mdy_atan (the same operations and bits) with its table of atan(k/8) = hi + lo
+// in LDS: one 16-byte read instead of 40 selects. Kernels fill the table first
+// (atan_table_fill, then a __syncthreads).
+struct AtanEntry { double hi, lo; };
+__device__ __forceinline__ AtanEntry *atan_table() {
+    __shared__ __align__(16) AtanEntry tab[9];
+    return tab;
+}
+__device__ __forceinline__ void atan_table_fill() {
+    constexpr AtanEntry t[9] = {{0.0, 0.0}, {MDY_ATAN_H1, MDY_ATAN_L1}, {MDY_ATAN_H2, MDY_ATAN_L2},
+                                {MDY_ATAN_H3, MDY_ATAN_L3}, {MDY_ATAN_H4, MDY_ATAN_L4}, {MDY_ATAN_H5, MDY_ATAN_L5},
+                                {MDY_ATAN_H6, MDY_ATAN_L6}, {MDY_ATAN_H7, MDY_ATAN_L7}, {MDY_ATAN_H8, MDY_ATAN_L8}};
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < 9; k++) atan_table()[k] = t[k];
+}
+__device__ __forceinline__ double xatan(double x) {
+    const double ax = fabs(x);
+    const bool inv = ax > 1.0;
+    const double y = inv ? 1.0 / ax : ax;
+    const int k = (y < 0.09375 || !(y <= 1.0)) ? 0 : (int)(y * 8.0 + 0.5);
+    const AtanEntry e = atan_table()[k];
+    const double c = (double)k * 0.125;
+    const double t = (y - c) / (1.0 + y * c);
+    const double t2 = t * t;
+    double p = -1.0 / 15.0;
+    p = p * t2 + 1.0 / 13.0;
+    p = p * t2 - 1.0 / 11.0;
+    p = p * t2 + 1.0 / 9.0;
+    p = p * t2 - 1.0 / 7.0;
+    p = p * t2 + 1.0 / 5.0;
+    p = p * t2 - 1.0 / 3.0;
+    p = t + t * (t2 * p);
+    double r = e.hi + (e.lo + p);
+    const double ri = (MDY_PIO2_HI - r) + MDY_PIO2_LO;
+    r = inv ? ri : r;
+    r = x < 0 ? -r : r;
+    return (x != x) ? x : r;
+}
+__device__ __forceinline__ Dual xatan(Dual a) { return Dual(xatan(a.v), a.d / (1 + a.v * a.v)); }
 __device__ __forceinline__ double xacos(double a) { return mdy_acos(a); }
 // d acos(v) = -dv / sqrt(1 - v^2); a constant argument (a clamped cosine) has
 // no derivative, also at v = +-1
@@ -523,7 +561,16 @@ __device__ __forceinline__ V3<T> bd_force(const double *__restrict__ pl, V3<T> p
 // areInPlane, MathFunctions.h:1101-1133
 __device__ __forceinline__ bool are_in_plane(d3 p1, d3 p2, d3 p3, d3 p4) {
     d3 v1 = sub(p2, p1), v2 = sub(p3, p1), v3 = sub(p4, p1);
-    d3 cp = normalize3(cross3(v1, v2));
+    d3 n = cross3(v1, v2);
+    // |cos| < 0.1 from the squares, without the two norms and six divisions,
+    // unless it is within rounding (margin 1e-12, rounding below 1e-14) of 0.1,
+    // degenerate or out of the squares' range
+    const double t = dot3(v3, n), t2 = t * t, lim = 0.01 * dot3(n, n) * dot3(v3, v3);
+    if (lim > 1e-200 && lim < 1e200) {
+        if (t2 < lim * (1.0 - 1e-12)) return true;
+        if (t2 > lim * (1.0 + 1e-12)) return false;
+    }
+    d3 cp = normalize3(n);
     v3 = normalize3(v3);
     return fabs(dot3(v3, cp) - 0.0) < 1e-1;
 }
@@ -533,148 +580,209 @@ __device__ __forceinline__ d3 moved_off_plane(d3 p1, d3 p2, d3 p3, d3 src, doubl
     return d3{(src.x + n.x * d), (src.y + n.y * d), (src.z + n.z * d)};
 }
 
-template <class T>
-struct EvInvT {
-    T a, b, c, d, e, F;
-    T AA, BB, CC, DD, EE, FF, GG, HH, JJ;
-    T ATG1, ATG2, ATG3, ATG4;
-};
-using EvInv = EvInvT<double>;
+// A pair is evaluated by two neighboring lanes, one per cylinder. The closed
+// form is a sum over the four edges of the parameter square [0,1]^2 (t = 0,
+// t = 1, s = 0, s = 1: the blocks A, E, B, F of the reference), and the edge
+// terms are the same expression of different scalars: lane 0 forms the terms
+// and derivative blocks of the edges A and E along the first cylinder, lane 1
+// those of B and F along the second, and each the forces on its cylinder's
+// beads. That halves a pair's chain of dependent instructions (a sweep waits
+// for its slowest thread), for about a quarter more instructions in all than
+// on one lane; on four lanes (an edge and a bead each) the scalars that every
+// lane forms again outweigh the shorter chain once the chip is full. Sums over
+// the edges run A, E, B, F in the reference's order, so the results keep their
+// bits.
+// Quotients by one divisor: with y = 1 / b rounded to nearest, q = a y and one
+// correction by the remainder a - q b (a fused multiply-add forms it exactly)
+// give a / b rounded to nearest (P. Markstein, IBM J. Res. Dev. 34, 1990;
+// N. Brisebarre, J.-M. Muller, S. K. Raina, IEEE Trans. Comput. 53, 2004),
+// in 3 instructions instead of a division's own reciprocal and scaling.
+template <class R> struct InvT;
+template <> struct InvT<double> { double b, y; };
+template <> struct InvT<float> { float b, y; };
+template <> struct InvT<Dual> { Dual b; double y; };
+__device__ __forceinline__ InvT<double> inv_of(double b) { return {b, 1.0 / b}; }
+__device__ __forceinline__ InvT<float> inv_of(float b) { return {b, 1.0f / b}; }
+__device__ __forceinline__ InvT<Dual> inv_of(Dual b) { return {b, 1.0 / b.v}; }
+__device__ __forceinline__ double div_by(double a, InvT<double> i) {
+    const double q = a * i.y;
+    return __builtin_fma(__builtin_fma(-q, i.b, a), i.y, q);
+}
+__device__ __forceinline__ float div_by(float a, InvT<float> i) {
+    const float q = a * i.y;
+    return __builtin_fmaf(__builtin_fmaf(-q, i.b, a), i.y, q);
+}
+__device__ __forceinline__ Dual div_by(Dual a, InvT<Dual> i) {
+    const InvT<double> iv{i.b.v, i.y};
+    const double q = div_by(a.v, iv);
+    return Dual(q, div_by(a.d - q * i.b.d, iv));
+}
 
+// the pair's lane H's value in both lanes (both are active or none is)
+template <int H> __device__ __forceinline__ int duo_get(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, H ? 0xF5 : 0xA0, 0xf, 0xf, true);   // lanes 1 1 3 3 or 0 0 2 2
+}
+template <int H> __device__ __forceinline__ float duo_get(float v) {
+    return __int_as_float(duo_get<H>(__float_as_int(v)));
+}
+template <int H> __device__ __forceinline__ double duo_get(double v) {
+    return __hiloint2double(duo_get<H>(__double2hiint(v)), duo_get<H>(__double2loint(v)));
+}
+template <int H> __device__ __forceinline__ Dual duo_get(Dual v) { return Dual(duo_get<H>(v.v), duo_get<H>(v.d)); }
+template <int H, class T> __device__ __forceinline__ V3<T> duo_get(V3<T> v) {
+    return V3<T>{duo_get<H>(v.x), duo_get<H>(v.y), duo_get<H>(v.z)};
+}
+// true in both lanes if true in one
+__device__ __forceinline__ bool duo_any(bool b) {
+    const int v = b ? 1 : 0;
+    return (v | __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true)) != 0;   // lanes 1 0 3 2
+}
+template <class T> __device__ __forceinline__ T pick(bool c, T a, T b) { return c ? a : b; }
+template <> __device__ __forceinline__ Dual pick(bool c, Dual a, Dual b) { return Dual(c ? a.v : b.v, c ? a.d : b.d); }
+
+template <class T> __device__ __forceinline__ V3<T> pick3(bool c, V3<T> a, V3<T> b) {
+    return V3<T>{pick(c, a.x, b.x), pick(c, a.y, b.y), pick(c, a.z, b.z)};
+}
+
+// sum over the edges of t0 and t1
+template <class T> __device__ __forceinline__ T duo_sum(T t0, T t1) {
+    const T s = duo_get<0>(T(t0 + t1));
+    return duo_get<1>(T(s + t0 + t1));
+}
+// the pair's scalars (in both lanes) and this lane's two edges, A and E or B
+// and F: X the edge's AA, EE, BB or FF, C its CC, GG, DD or HH, u and w the
+// arctangents' numerators
+template <class T> struct EvEdgeT { T X, C, ATG; };
 template <class T>
-__device__ __forceinline__ void ev_invariants(V3<T> c1, V3<T> c2, V3<T> c3, V3<T> c4, EvInvT<T> &v) {
+struct EvDuoT {
+    T a, b, c, d, e, F, JJ;
+    EvEdgeT<T> g0, g1;
+};
+template <class T>
+__device__ __forceinline__ void ev_duo_uw(bool h, T a, T b, T d, T e, T F, T &u0, T &w0, T &u1, T &w1) {
+    u0 = pick(h, F, T(a + e));
+    w0 = pick(h, T(F - b), e);
+    u1 = pick(h, T(d + F), T(a + e - d));
+    w1 = pick(h, T(d + F - b), T(e - d));
+}
+// X = sqrt(max(0, (ac + o)(ac - o))), ac = sqrt(m n)
+template <class T>
+__device__ __forceinline__ void ev_edge(T m, T n, T o, T u, T w, EvEdgeT<T> &g, T &term) {
+    const T ac = xsqrt(m * n);
+    g.X = xsqrt(smax(T(0.0), (ac + o) * (ac - o)));
+    const InvT<T> iX = inv_of(g.X);
+    g.ATG = xatan(div_by(u, iX)) - xatan(div_by(w, iX));
+    term = div_by(g.C, iX) * g.ATG;
+}
+template <class T>
+__device__ __forceinline__ void ev_duo_invariants(bool h, V3<T> c1, V3<T> c2, V3<T> c3, V3<T> c4, EvDuoT<T> &v,
+                                                  T &block) {
     v.a = sprod(c1, c2, c1, c2);
     v.b = sprod(c3, c4, c3, c4);
     v.c = sprod(c3, c1, c3, c1);
     v.d = sprod(c1, c2, c3, c4);
     v.e = sprod(c1, c2, c3, c1);
     v.F = sprod(c3, c4, c3, c1);
-    T g = sprod(c1, c2, c1, c4);
-    T h = sprod(c3, c4, c3, c2);
-    T I = sprod(c3, c4, c1, c4);
-    T sqD, sqE;
-    {
-        T x = c1.x - c4.x, y = c1.y - c4.y, z = c1.z - c4.z;
-        sqD = (x * x + y * y + z * z);
-        x = c3.x - c2.x; y = c3.y - c2.y; z = c3.z - c2.z;
-        sqE = (x * x + y * y + z * z);
-    }
+    const T g = sprod(c1, c2, c1, c4);
+    const T I = sprod(c3, c4, c1, c4);
     const T a = v.a, b = v.b, c = v.c, d = v.d, e = v.e, F = v.F;
-    T ac = xsqrt(a * c), bc = xsqrt(b * c), aD = xsqrt(a * sqD), bE = xsqrt(b * sqE);
-    v.AA = xsqrt(smax(T(0.0), (ac + e) * (ac - e)));
-    v.BB = xsqrt(smax(T(0.0), (bc + F) * (bc - F)));
-    v.CC = d * e - a * F;
-    v.DD = b * e - d * F;
-    v.EE = xsqrt(smax(T(0.0), (aD + g) * (aD - g)));
-    v.FF = xsqrt(smax(T(0.0), (bE + h) * (bE - h)));
-    v.GG = d * g - a * I;
-    v.HH = v.CC + v.GG - v.DD;
-    V3<T> cp = cross3(sub(c1, c2), sub(c3, c4));
-    T JJ = dot3(cp, sub(c3, c1));
+    // the far edge's distance: c4 from c1, or c2 from c3
+    const V3<T> f0 = pick3(h, c3, c1), f1 = pick3(h, c2, c4);
+    const T x = f0.x - f1.x, y = f0.y - f1.y, z = f0.z - f1.z;
+    const T sq = (x * x + y * y + z * z);
+    const T hh = sprod(c3, c4, c3, c2);
+    const T CC = d * e - a * F, DD = b * e - d * F, GG = d * g - a * I, HH = CC + GG - DD;
+    v.g0.C = pick(h, DD, CC);
+    v.g1.C = pick(h, HH, GG);
+    const V3<T> cp = cross3(sub(c1, c2), sub(c3, c4));
+    const T JJ = dot3(cp, sub(c3, c1));
     v.JJ = -JJ * JJ;
-    v.ATG1 = xatan((a + e) / v.AA) - xatan(e / v.AA);
-    v.ATG2 = xatan((a + e - d) / v.EE) - xatan((e - d) / v.EE);
-    v.ATG3 = xatan((F) / v.BB) - xatan((F - b) / v.BB);
-    v.ATG4 = xatan((d + F) / v.FF) - xatan((d + F - b) / v.FF);
+    T u0, w0, u1, w1, t0, t1;
+    ev_duo_uw(h, a, b, d, e, F, u0, w0, u1, w1);
+    const T m = pick(h, b, a);
+    ev_edge(m, c, pick(h, F, e), u0, w0, v.g0, t0);
+    ev_edge(m, sq, pick(h, hh, g), u1, w1, v.g1, t1);
+    block = duo_sum(t0, t1);
 }
-
-template <class T> __device__ __forceinline__ T ev_energy_inv(const EvInvT<T> &v, double kr) {
-    return 0.5 * kr / v.JJ * (v.CC / v.AA * v.ATG1 + v.GG / v.EE * v.ATG2 + v.DD / v.BB * v.ATG3 + v.HH / v.FF * v.ATG4);
-}
-__device__ __forceinline__ double ev_energy(d3 c1, d3 c2, d3 c3, d3 c4, double kr) {
-    EvInv v;
-    ev_invariants(c1, c2, c3, c4, v);
-    return ev_energy_inv(v, kr);
+template <class T> __device__ __forceinline__ T ev_duo_energy(const EvDuoT<T> &v, T block, double kr) {
+    return 0.5 * kr / v.JJ * block;
 }
 __device__ __forceinline__ bool ev_energy_bad(double U) { return fabs(U) == INFINITY || U != U || U < -1.0; }
 
-// Analytic pair force; f[0..3] = forces on c1..c4. Direction vectors use the
-// c2 passed in (the moved one in the coplanar case), as the reference does.
+// derivative block of an edge: by C, by X, by the common shift of u and w, by u
+template <class R> struct EvBlockT { R pC, pX, pm, pa; InvT<R> iX; };
+template <class R>
+__device__ __forceinline__ EvBlockT<R> ev_block(R X, R C, R u, R w, R ATG, R &term) {
+    EvBlockT<R> g;
+    g.iX = inv_of(X);
+    term = div_by(C, g.iX) * ATG;
+    const R X2 = X * X;
+    const InvT<R> iX2 = inv_of(X2);
+    const R A1 = X2 / (X2 + u * u);
+    const R A2 = X2 / (X2 + w * w);
+    g.pC = div_by(ATG, g.iX);
+    g.pX = div_by(R(-(ATG * C)), iX2) + (-A1 * u + A2 * w) * C / (X2 * X);
+    g.pm = div_by(R((A1 - A2) * C), iX2);
+    g.pa = div_by(R(A1 * C), iX2);
+    return g;
+}
+// Analytic pair force on this lane's cylinder's beads. Direction vectors use
+// the c2 passed in (the moved one in the coplanar case), as the reference does.
 // R = T: the FP64 path (T = double) and the Hessian-vector product (T = Dual);
 // T = double, R = float: the mixed-precision form, whose derivative blocks run
 // in FP32 from the FP64 invariants.
 template <class R, class T>
-__device__ __forceinline__ void ev_force_inv_t(const EvInvT<T> &v, V3<T> c1, V3<T> c2, V3<T> c3, V3<T> c4,
-                                               double kr_, V3<R> f[4]) {
+__device__ __forceinline__ void ev_duo_force(bool h, const EvDuoT<T> &v, V3<T> c1, V3<T> c2, V3<T> c3, V3<T> c4,
+                                             double kr_, V3<R> f[2]) {
     const R a = cvt<R>(v.a), b = cvt<R>(v.b), c = cvt<R>(v.c), d = cvt<R>(v.d), e = cvt<R>(v.e), F = cvt<R>(v.F);
-    const R AA = cvt<R>(v.AA), BB = cvt<R>(v.BB), CC = cvt<R>(v.CC), DD = cvt<R>(v.DD), EE = cvt<R>(v.EE),
-            FF = cvt<R>(v.FF), GG = cvt<R>(v.GG), HH = cvt<R>(v.HH);
-    const R ATG1 = cvt<R>(v.ATG1), ATG2 = cvt<R>(v.ATG2), ATG3 = cvt<R>(v.ATG3), ATG4 = cvt<R>(v.ATG4);
     const R kr = R(kr_);
     const R invJJ = 1 / cvt<R>(v.JJ);
-    const R sumBlock = CC / AA * ATG1 + GG / EE * ATG2 + DD / BB * ATG3 + HH / FF * ATG4;
+    R u0, w0, u1, w1, t0, t1;
+    ev_duo_uw(h, a, b, d, e, F, u0, w0, u1, w1);
+    const EvBlockT<R> p = ev_block(cvt<R>(v.g0.X), cvt<R>(v.g0.C), u0, w0, cvt<R>(v.g0.ATG), t0);
+    const EvBlockT<R> q = ev_block(cvt<R>(v.g1.X), cvt<R>(v.g1.C), u1, w1, cvt<R>(v.g1.ATG), t1);
+    const R sumBlock = duo_sum(t0, t1);
     const R enFactor = kr * invJJ / 2;
-    const R A1 = AA * AA / (AA * AA + (a + e) * (a + e));
-    const R A2 = AA * AA / (AA * AA + e * e);
-    const R E1 = EE * EE / (EE * EE + (a + e - d) * (a + e - d));
-    const R E2 = EE * EE / (EE * EE + (e - d) * (e - d));
-    const R B1 = BB * BB / (BB * BB + F * F);
-    const R B2 = BB * BB / (BB * BB + (F - b) * (F - b));
-    const R F1 = FF * FF / (FF * FF + (d + F) * (d + F));
-    const R F2 = FF * FF / (FF * FF + (d + F - b) * (d + F - b));
-    const R pA_C = ATG1 / AA;
-    const R pA_A = -(ATG1 * CC) / (AA * AA) + (-A1 * (a + e) + A2 * e) * CC / (AA * AA * AA);
-    const R pA_e = ((A1 - A2) * CC) / (AA * AA);
-    const R pA_a = (A1 * CC) / (AA * AA);
-    const R pE_G = ATG2 / EE;
-    const R pE_E = -(ATG2 * GG) / (EE * EE) + (-E1 * (a + e - d) + E2 * (e - d)) * GG / (EE * EE * EE);
-    const R pE_emd = ((E1 - E2) * GG) / (EE * EE);
-    const R pE_a = (E1 * GG) / (EE * EE);
-    const R pB_D = ATG3 / BB;
-    const R pB_B = -(ATG3 * DD) / (BB * BB) + (-B1 * F + B2 * (F - b)) * DD / (BB * BB * BB);
-    const R pB_fmb = ((B1 - B2) * DD) / (BB * BB);
-    const R pB_b = (B1 * DD) / (BB * BB);
-    const R pF_H = ATG4 / FF;
-    const R pF_F = -(ATG4 * HH) / (FF * FF) + (-F1 * (d + F) + F2 * (d + F - b)) * HH / (FF * FF * FF);
-    const R pF_dfb = ((F1 - F2) * HH) / (FF * FF);
-    const R pF_b = (F1 * HH) / (FF * FF);
-    const R k11 = pA_C * (-2 * F) + pA_A * (c / AA) + pA_a * 2 + pE_G * (2 * (F - b)) +
-                  pE_E * ((b + c - 2 * F) / EE) + pE_a * 2 + pF_H * (-2 * b) + pF_F * (b / FF);
-    const R k12 = pA_C * e + pE_G * (2 * d - e) + pE_E * ((e - d) / EE) + pE_emd * (-1) + pB_D * (-F) +
-                  pF_H * (2 * d + F) + pF_F * (-(d + F) / FF) + pF_dfb;
-    const R k13 = pA_C * d + pA_A * (-e / AA) + pA_e + pE_G * (-d) + pE_E * (-(e - d) / EE) + pE_emd +
-                  pB_D * b + pF_H * (-b) + pF_F * (b / FF);
-    const R k22 = pE_G * (-2 * a) + pE_E * (a / EE) + pB_D * (2 * e) + pB_B * (c / BB) + pB_fmb * (-2) +
-                  pB_b * 2 + pF_H * (-2 * (a + e)) + pF_F * ((a + c + 2 * e) / FF) + pF_dfb * (-2) + pF_b * 2;
-    const R k23 = pA_C * (-a) + pE_G * a + pE_E * (-a / EE) + pB_D * (-d) + pB_B * (-F / BB) + pB_fmb +
-                  pF_H * d + pF_F * (-(d + F) / FF) + pF_dfb;
-    const R k33 = pA_A * (a / AA) + pE_E * (a / EE) + pB_B * (b / BB) + pF_F * (b / FF);
-    const R k21 = k12, k31 = k13, k32 = k23;
+    // quotients by X: A c, -e, a; E b + c - 2F, e - d, a; B c, -F, b; F b, -(d + F), a + c + 2e
+    const R p1 = div_by(c, p.iX), p2 = div_by(pick(h, R(-F), R(-e)), p.iX), p3 = div_by(pick(h, b, a), p.iX);
+    const R q1 = div_by(pick(h, b, R(b + c - 2 * F)), q.iX), q2 = div_by(pick(h, R(-(d + F)), R(e - d)), q.iX),
+            q3 = div_by(pick(h, R(a + c + 2 * e), a), q.iX);
+
+    // lane 0 starts the sums with the edges A and E
+    R k11 = p.pC * (-2 * F) + p.pX * p1 + p.pa * 2 + q.pC * (2 * (F - b)) + q.pX * q1 + q.pa * 2;
+    R k12 = p.pC * e + q.pC * (2 * d - e) + q.pX * q2 + q.pm * (-1);
+    R k13 = p.pC * d + p.pX * p2 + p.pm + q.pC * (-d) + q.pX * (-q2) + q.pm;
+    R k22 = q.pC * (-2 * a) + q.pX * q3;
+    R k23 = p.pC * (-a) + q.pC * a + q.pX * (-q3);
+    R k33 = p.pX * p3 + q.pX * q3;
+    k11 = duo_get<0>(k11); k12 = duo_get<0>(k12); k13 = duo_get<0>(k13);
+    k22 = duo_get<0>(k22); k23 = duo_get<0>(k23); k33 = duo_get<0>(k33);
+    // lane 1 goes on with B and F
+    k11 = k11 + q.pC * (-2 * b) + q.pX * q1;
+    k12 = k12 + p.pC * (-F) + q.pC * (2 * d + F) + q.pX * q2 + q.pm;
+    k13 = k13 + p.pC * b + q.pC * (-b) + q.pX * q1;
+    k22 = k22 + p.pC * (2 * e) + p.pX * p1 + p.pm * (-2) + p.pa * 2 + q.pC * (-2 * (a + e)) + q.pX * q3 + q.pm * (-2) +
+          q.pa * 2;
+    k23 = k23 + p.pC * (-d) + p.pX * p2 + p.pm + q.pC * d + q.pX * q2 + q.pm;
+    k33 = k33 + p.pX * p3 + q.pX * q1;
+    k11 = duo_get<1>(k11); k12 = duo_get<1>(k12); k13 = duo_get<1>(k13);
+    k22 = duo_get<1>(k22); k23 = duo_get<1>(k23); k33 = duo_get<1>(k33);
     const R J11 = 2 * (-b * c + F * F), J12 = 2 * (c * d - e * F), J13 = 2 * (b * e - d * F);
-    const R J21 = 2 * (c * d - e * F), J22 = 2 * (-a * c + e * e), J23 = 2 * (-d * e + a * F);
-    const R J31 = 2 * (b * e - d * F), J32 = 2 * (-d * e + a * F), J33 = 2 * (d * d - a * b);
+    const R J22 = 2 * (-a * c + e * e), J23 = 2 * (-d * e + a * F), J33 = 2 * (d * d - a * b);
     const R sb = -invJJ * sumBlock;
-    R dv[4][3];
-    dv[0][0] = enFactor * (sb * (J31 - J11) + (k31 - k11));
-    dv[0][1] = enFactor * (sb * (J32 - J12) + (k32 - k12));
-    dv[0][2] = enFactor * (sb * (J33 - J13) + (k33 - k13));
-    dv[1][0] = enFactor * (sb * (J11) + (k11));
-    dv[1][1] = enFactor * (sb * (J12) + (k12));
-    dv[1][2] = enFactor * (sb * (J13) + (k13));
-    dv[2][0] = enFactor * (sb * (-J31 - J21) + (-k31 - k21));
-    dv[2][1] = enFactor * (sb * (-J32 - J22) + (-k32 - k22));
-    dv[2][2] = enFactor * (sb * (-J33 - J23) + (-k33 - k23));
-    dv[3][0] = enFactor * (sb * (J21) + (k21));
-    dv[3][1] = enFactor * (sb * (J22) + (k22));
-    dv[3][2] = enFactor * (sb * (J23) + (k23));
     const V3<T> u1d = sub(c2, c1), u2d = sub(c4, c3), u3d = sub(c1, c3);
-    const R u1x = cvt<R>(u1d.x), u1y = cvt<R>(u1d.y), u1z = cvt<R>(u1d.z);
-    const R u2x = cvt<R>(u2d.x), u2y = cvt<R>(u2d.y), u2z = cvt<R>(u2d.z);
-    const R u3x = cvt<R>(u3d.x), u3y = cvt<R>(u3d.y), u3z = cvt<R>(u3d.z);
-#pragma unroll
-    for (int bi = 0; bi < 4; bi++) {
-        f[bi].x = -(dv[bi][0] * u1x + dv[bi][1] * u2x + dv[bi][2] * u3x);
-        f[bi].y = -(dv[bi][0] * u1y + dv[bi][1] * u2y + dv[bi][2] * u3y);
-        f[bi].z = -(dv[bi][0] * u1z + dv[bi][1] * u2z + dv[bi][2] * u3z);
-    }
-}
-__device__ __forceinline__ void ev_force_inv(const EvInv &v, d3 c1, d3 c2, d3 c3, d3 c4, double kr, d3 f[4]) {
-    ev_force_inv_t<double>(v, c1, c2, c3, c4, kr, f);
-}
-__device__ __forceinline__ void ev_force(d3 c1, d3 c2, d3 c3, d3 c4, double kr, d3 f[4]) {
-    EvInv v;
-    ev_invariants(c1, c2, c3, c4, v);
-    ev_force_inv(v, c1, c2, c3, c4, kr, f);
+    auto bead = [&](R x1, R x2, R x3) {
+        return V3<R>{-(x1 * cvt<R>(u1d.x) + x2 * cvt<R>(u2d.x) + x3 * cvt<R>(u3d.x)),
+                     -(x1 * cvt<R>(u1d.y) + x2 * cvt<R>(u2d.y) + x3 * cvt<R>(u3d.y)),
+                     -(x1 * cvt<R>(u1d.z) + x2 * cvt<R>(u2d.z) + x3 * cvt<R>(u3d.z))};
+    };
+    // plus bead: row 1 or 2; minus bead: row 3 - row 1 or -row 3 - row 2
+    const R r1 = pick(h, J12, J11), r2 = pick(h, J22, J12), r3 = pick(h, J23, J13);
+    const R s1 = pick(h, k12, k11), s2 = pick(h, k22, k12), s3 = pick(h, k23, k13);
+    auto minus = [&](R row3, R row) { return R(pick(h, R(-row3), row3) - row); };
+    f[0] = bead(enFactor * (sb * minus(J13, r1) + minus(k13, s1)), enFactor * (sb * minus(J23, r2) + minus(k23, s2)),
+                enFactor * (sb * minus(J33, r3) + minus(k33, s3)));
+    f[1] = bead(enFactor * (sb * r1 + s1), enFactor * (sb * r2 + s2), enFactor * (sb * r3 + s3));
 }
 template <class T> __device__ __forceinline__ bool finite_d3(V3<T> v) {
     return xfinite(v.x) && xfinite(v.y) && xfinite(v.z);

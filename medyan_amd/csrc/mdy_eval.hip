@@ -14,18 +14,18 @@ namespace mdy {
 template <class P, bool QUAD = false>
 __global__ void __launch_bounds__(kBlock, 3) k_energy(Dev D, P pos, double *red) {
     __shared__ double lds[17 * kNFF + 8];
+    __shared__ XBlock xb;
+    xblock_zero(xb);
+    atan_table_fill();
     double acc[kNFF];
 #pragma unroll
     for (int k = 0; k < kNFF; k++) acc[k] = 0.0;
-    mdy_xsum xs;
-    mdy_xs_zero(&xs);
-    const int total = D.n_items(), gs = gridDim.x * blockDim.x;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gs)
-        item<false, QUAD>(D, i, pos, acc, xs, nullptr, true, false);
+    __syncthreads();
+    sweep<false, QUAD>(D, pos, blockIdx.x, gridDim.x, acc, &xb, nullptr, true, false);
     block_reduce<kNFF>(acc, lds);
-    block_reduce_xsum(xs, reinterpret_cast<long long *>(lds));
     if (threadIdx.x < kNFF) red[(size_t)blockIdx.x * kRed + threadIdx.x] = acc[threadIdx.x];
-    if (threadIdx.x == 0) store_xsum(red, blockIdx.x, kXsE, xs);
+    const unsigned long long w = xblock_take(xb);
+    if (threadIdx.x < 8) reinterpret_cast<unsigned long long *>(red)[(size_t)blockIdx.x * kRed + kXsE + threadIdx.x] = w;
 }
 
 // One block per queued pair: 2-D Simpson energy (energyN, 400 x 400 intervals).
@@ -66,12 +66,9 @@ __global__ void __launch_bounds__(kBlock) k_energy_final(Dev D, const double *re
 template <bool MIXED, class P, bool QUAD = false>
 __global__ void __launch_bounds__(kBlock) k_force(Dev D, P pos, double *contrib_) {
     auto *contrib = reinterpret_cast<typename SlotT<MIXED>::T *>(contrib_);
-    const int total = D.n_items(), gs = gridDim.x * blockDim.x;
-    double acc[kNFF];
-    mdy_xsum xs;
-    mdy_xs_zero(&xs);
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gs)
-        item<MIXED, QUAD>(D, i, pos, acc, xs, contrib, false, true);
+    atan_table_fill();
+    __syncthreads();
+    sweep<MIXED, QUAD>(D, pos, blockIdx.x, gridDim.x, nullptr, nullptr, contrib, false, true);
 }
 
 // Quadrature force (forceN, 10^4 x 10^4 intervals) of one queued pair,
@@ -137,19 +134,12 @@ __global__ void __launch_bounds__(kBlock) k_force_simpson_final(Dev D, const dou
     }
 }
 
-// WIDE: the wide per-bead form (fewer beads than one block per CU has
-// threads: at 200k cylinders the narrow form's occupancy wins); same sums
-// either way
-template <bool MIXED, bool WIDE>
+template <bool MIXED>
 __global__ void __launch_bounds__(kBlock) k_gather(Dev D, const double *contrib_, double *force, int accumulate) {
     const auto *contrib = reinterpret_cast<const typename SlotT<MIXED>::T *>(contrib_);
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < D.nb; b += gridDim.x * blockDim.x) {
-        d3 f = WIDE ? gather_bead_w<12, 24>(D, contrib, b) : gather_bead(D, contrib, b);
-        if (accumulate) {
-            force[3 * b] += f.x; force[3 * b + 1] += f.y; force[3 * b + 2] += f.z;
-        } else {
-            force[3 * b] = f.x; force[3 * b + 1] = f.y; force[3 * b + 2] = f.z;
-        }
+    for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < D.ndof; o += gridDim.x * blockDim.x) {
+        const double f = gather_coord(D, contrib, o);
+        force[o] = accumulate ? force[o] + f : f;
     }
 }
 
@@ -170,7 +160,7 @@ static int grid_for(const Ctx &c, long long n) {
 
 int launch_energy(Ctx &c, const double *d_x, double *d_out, hipStream_t st) {
     Dev D = c.dev();
-    const int nblk = grid_for(c, D.n_items());
+    const int nblk = grid_for(c, D.n_lanes());
     const bool quad = quad_on(c);
     const int nqb = quad ? quad_blocks(c) : 0;   // the quadrature pairs' block records follow the others
     MDY_TRY(ensure(c.red, (size_t)kRed * (nblk + nqb)));
@@ -233,7 +223,7 @@ int launch_energy_noalloc(Ctx &c, const double *d_x, double *d_out, hipStream_t 
     }
     if (!sc) return MDY_ERR_STATE;
     Dev D = c.dev();
-    const int nblk = grid_for(c, D.n_items());
+    const int nblk = grid_for(c, D.n_lanes());
     if (nblk > kScratchBlocks) return MDY_ERR_CAPACITY;
     double *red = reinterpret_cast<double *>(sc + kScRed);
     int *qn = reinterpret_cast<int *>(sc + kScQn);
@@ -254,7 +244,7 @@ int launch_energy_noalloc(Ctx &c, const double *d_x, double *d_out, hipStream_t 
 
 int launch_forces(Ctx &c, const double *d_x, double *d_force, int accumulate, hipStream_t st) {
     Dev D = c.dev();
-    const int nblk = grid_for(c, D.n_items());
+    const int nblk = grid_for(c, D.n_lanes());
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, c.qn.p, 4);
     const bool mixed = c.opts.precision == MDY_PREC_MIXED;
     if (quad_on(c)) {   // FP64 only (the mode is refused for mixed-precision contexts)
@@ -294,11 +284,8 @@ int launch_forces(Ctx &c, const double *d_x, double *d_force, int accumulate, hi
             if (moved || !fl[1]) return MDY_ERR_FORCE;  // the reference exits here
         }
     }
-    const int gg = grid_for(c, D.nb);
-    const bool wide = (long long)D.nb <= (long long)c.num_cu * kBlock;
-    auto kern = mixed ? (wide ? k_gather<true, true> : k_gather<true, false>)
-                      : (wide ? k_gather<false, true> : k_gather<false, false>);
-    hipLaunchKernelGGL(kern, dim3(gg), dim3(kBlock), 0, st, D, c.contrib.p, d_force, accumulate);
+    hipLaunchKernelGGL(mixed ? k_gather<true> : k_gather<false>, dim3(grid_for(c, D.ndof)), dim3(kBlock), 0, st, D,
+                       c.contrib.p, d_force, accumulate);
     return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
 }
 

@@ -9,32 +9,22 @@
 namespace mdy {
 
 // ---- where bead positions come from ---------------------------------------
+// get: the positions of N beads, every load issued before the first use, so N
+// beads cost one memory round trip.
 struct PosX {  // x
     const double *__restrict__ x;
     __device__ __forceinline__ d3 operator()(int o) const { return d3{x[o], x[o + 1], x[o + 2]}; }
-};
-struct PosLine {  // x + lam * d   (CGMethod::calcCoordLineSearch, CGMethod.cpp:43-46)
-    const double *__restrict__ x;
-    const double *__restrict__ d;
-    double lam;
-    __device__ __forceinline__ d3 operator()(int o) const {
-        return d3{x[o] + lam * d[o], x[o + 1] + lam * d[o + 1], x[o + 2] + lam * d[o + 2]};
+    template <int N> __device__ __forceinline__ void get(const int (&o)[N], d3 (&c)[N]) const {
+#pragma unroll
+        for (int k = 0; k < N; k++) c[k] = (*this)(o[k]);
     }
 };
-struct PosSpec {  // x + lam * (F + beta * d): trial along the not-yet-stored new direction
-    const double *__restrict__ x;
-    const double *__restrict__ F;
-    const double *__restrict__ d;
-    double beta, lam;
-    __device__ __forceinline__ double c(int o) const {
-        double s = F[o] + beta * d[o];
-        return x[o] + lam * s;
-    }
-    __device__ __forceinline__ d3 operator()(int o) const { return d3{c(o), c(o + 1), c(o + 2)}; }
-};
-
-// one functor for all three (uniform runtime mode): a single inlined copy of
-// the interaction code serves every evaluation of the persistent kernel
+// One functor for the minimizer's three kinds (uniform runtime mode), so that a
+// single inlined copy of the interaction code serves every evaluation: x,
+// x + lam * d (CGMethod::calcCoordLineSearch, CGMethod.cpp:43-46), or
+// x + lam * (F + beta * d), the trial along the not-yet-stored new direction.
+// One branch per item: with one per component each was a dependent round trip
+// (a linker's four beads took 21 us of a 50 us sweep at 40k cylinders).
 struct PosAny {
     enum { X = 0, LINE = 1, SPEC = 2 };
     const double *__restrict__ x;
@@ -42,18 +32,28 @@ struct PosAny {
     const double *__restrict__ F;
     double lam, beta;
     int mode;
-    __device__ __forceinline__ double c(int o) const {
-        if (mode == X) return x[o];
-        const double s = (mode == SPEC) ? F[o] + beta * d[o] : d[o];
-        return x[o] + lam * s;
+    template <int N> __device__ __forceinline__ void get(const int (&o)[N], d3 (&c)[N]) const {
+        const PosX px{x};
+        px.get(o, c);
+        if (mode == X) return;
+        d3 s[N];
+        PosX{d}.get(o, s);
+        if (mode == SPEC) {
+            d3 f[N];
+            PosX{F}.get(o, f);
+#pragma unroll
+            for (int k = 0; k < N; k++)
+                s[k] = d3{f[k].x + beta * s[k].x, f[k].y + beta * s[k].y, f[k].z + beta * s[k].z};
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            c[k] = d3{c[k].x + lam * s[k].x, c[k].y + lam * s[k].y, c[k].z + lam * s[k].z};
     }
-    __device__ __forceinline__ d3 operator()(int o) const { return d3{c(o), c(o + 1), c(o + 2)}; }
-    static __device__ PosAny at(const double *x) { return PosAny{x, nullptr, nullptr, 0.0, 0.0, X}; }
-    static __device__ PosAny line(const double *x, const double *d, double lam) {
-        return PosAny{x, d, nullptr, lam, 0.0, LINE};
-    }
-    static __device__ PosAny spec(const double *x, const double *F, const double *d, double beta, double lam) {
-        return PosAny{x, d, F, lam, beta, SPEC};
+    __device__ __forceinline__ d3 operator()(int o) const {
+        const int q[1] = {o};
+        d3 c[1];
+        get(q, c);
+        return c[0];
     }
 };
 
@@ -75,30 +75,136 @@ __device__ __forceinline__ void put3(float *__restrict__ c, int slot, d3 v) {
 __device__ __forceinline__ void put3(float *__restrict__ c, int slot, f3 v) {
     c[3 * slot] = v.x; c[3 * slot + 1] = v.y; c[3 * slot + 2] = v.z;
 }
+template <class S> __device__ __forceinline__ V3<S> vec3_none() { return V3<S>{S(-0.0), S(-0.0), S(-0.0)}; }
 // force-record element type of each form
 template <bool MIXED> struct SlotT { using T = double; };
 template <> struct SlotT<true> { using T = float; };
 
+// ---- exact block sums in LDS -------------------------------------------------
+// Two exact sums (mdy_xsum's digits) and a maximum per block, accumulated as the
+// terms arise: each term adds its two or three digits with LDS integer atomics,
+// in any order with the same result, so no thread carries an accumulator (14
+// registers each) through the sweep and the end of a phase combines 16 copies
+// of 17 words instead of every thread's. Copy = thread % 16.
+// A block of at most 1024 threads may add kXTurns terms per thread and sum
+// between two calls of xblock_norm: 1024 * 16 terms below 2^48 stay below 2^63.
+constexpr int kXRep = 16, kXTurns = 16;
+struct XBlock {
+    unsigned long long w[17][kXRep];   // sum 0: digits 0..6, flags; sum 1: the same; maximum
+};
+struct XAdd {   // this thread's copy of sum 0 or 1
+    XBlock *x;
+    int row;
+    __device__ __forceinline__ void put(int k, unsigned long long v) const {
+        __hip_atomic_fetch_add(&x->w[row + k][threadIdx.x & (kXRep - 1)], v, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __device__ __forceinline__ void flag(int v) const {
+        __hip_atomic_fetch_or(&x->w[row + 7][threadIdx.x & (kXRep - 1)], (unsigned long long)v, __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    // mdy_xs_add
+    __device__ __forceinline__ void operator()(double v) const {
+        const unsigned long long b = mdy_dbits(v);
+        const bool neg = (b >> 63) != 0;
+        const int ex = (int)((b >> 52) & 0x7ff);
+        unsigned long long m = b & 0xFFFFFFFFFFFFFull;
+        if (__builtin_expect(ex == 0x7ff, 0)) {
+            flag(m ? MDY_XS_NAN : (neg ? MDY_XS_NINF : MDY_XS_PINF));
+            return;
+        }
+        if (ex) m |= 0x10000000000000ull;
+        int p = (ex ? ex - 1075 : -1074) + MDY_XS_BIAS;
+        if (p < 0) {
+            m = (-p >= 64) ? 0 : (m >> (-p));
+            p = 0;
+        }
+        if (m == 0) return;
+        if (__builtin_expect(p + 53 > 48 * (MDY_XS_N - 1) + 47, 0)) {
+            flag(neg ? MDY_XS_NINF : MDY_XS_PINF);
+            return;
+        }
+        const int j = p / 48, sh = p - 48 * j;
+        const unsigned long long lo = (m << sh) & (unsigned long long)MDY_XS_MASK;
+        const unsigned long long mid = (sh == 0 ? (m >> 48) : (m >> (48 - sh))) & (unsigned long long)MDY_XS_MASK;
+        const unsigned long long hi = (96 - sh < 64) ? m >> (96 - sh) : 0;   // 0 in the last digits: the sum's bound
+        put(j, neg ? 0 - lo : lo);
+        put(j + 1, neg ? 0 - mid : mid);
+        if (hi) put(j + 2, neg ? 0 - hi : hi);
+    }
+};
+__device__ __forceinline__ void xblock_zero(XBlock &x) {
+    for (int k = threadIdx.x; k < 17 * kXRep; k += blockDim.x) (&x.w[0][0])[k] = 0;
+}
+__device__ __forceinline__ void xblock_max(XBlock &x, double m) {   // m >= 0 or NaN: ordered as integers
+    __hip_atomic_fetch_max(&x.w[16][threadIdx.x & (kXRep - 1)], (unsigned long long)__double_as_longlong(m),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// carries of every copy into [0, 2^48) digits (all threads of the block)
+__device__ __forceinline__ void xblock_norm(XBlock &x) {
+    __syncthreads();
+    if (threadIdx.x < 2 * kXRep) {
+        const int row = 8 * (threadIdx.x / kXRep), r = threadIdx.x % kXRep;
+        long long c = 0;
+        for (int k = 0; k < MDY_XS_N; k++) {
+            const long long d = (long long)x.w[row + k][r] + c;
+            c = d >> 48;
+            x.w[row + k][r] = k < MDY_XS_N - 1 ? (unsigned long long)(d & MDY_XS_MASK) : (unsigned long long)d;
+        }
+    }
+    __syncthreads();
+}
+// Word t (t = 0..16, one per thread of the first wave) of the block's sums, its
+// copies cleared for the next phase: digits below 2^49, so that the words of
+// 2^14 blocks can be added. Every thread calls it after a __syncthreads();
+// threads t >= 17 get 0.
+__device__ __forceinline__ unsigned long long xblock_take(XBlock &x) {
+    const int t = threadIdx.x;
+    if (t >= 64) return 0;
+    unsigned long long r = 0;
+    if (t < 17) {
+        const bool isor = (t & 7) == 7, ismax = t == 16;
+#pragma unroll
+        for (int k = 0; k < kXRep; k++) {   // rotated: the lanes read different banks
+            unsigned long long &e = x.w[t][(k + t) & (kXRep - 1)];
+            const unsigned long long v = e;
+            e = 0;
+            r = isor ? (r | v) : ismax ? (v > r ? v : r) : r + v;
+        }
+    }
+    // one carry step: each digit keeps its low 48 bits and takes its neighbor's rest
+    const long long carry = (long long)r >> 48, up = __shfl_up(carry, 1, 64);
+    const int k = t & 7;
+    if (t < 16 && k < 7) {
+        if (k < MDY_XS_N - 1) r &= (unsigned long long)MDY_XS_MASK;
+        if (k > 0) r += (unsigned long long)up;
+    }
+    return r;
+}
+
 // ---- the interaction sweep -------------------------------------------------
-// Every interaction is an item of the index space [EV | FS | FB | LM | BS | BB |
-// BD]. An item's record (its bead offsets and parameters) and its beads'
-// coordinates are fetched one item ahead of the one being computed, so each
-// thread's chain of dependent memory accesses overlaps with its arithmetic.
-// IT_EVM: an excluded-volume pair of the monomer-sum form (same table and slots as IT_EV)
-enum { IT_EV = 0, IT_FS, IT_FB, IT_LM, IT_BS, IT_BB, IT_BDH, IT_BP, IT_BD, IT_EVM, IT_NONE };
+// The sweep's index space is one of lanes: two for every excluded-volume pair
+// of the integral form, then one for every other interaction,
+// [EV x 2 | FS | FB | LM | BS | BB | BDH | BP | BD]. Starts and strides are
+// multiples of the wave, so a pair's lanes are neighbors in one.
+// IT_EVM: an excluded-volume pair of the monomer-sum form (one lane, same table and slots)
+enum { IT_EVM = 0, IT_FS, IT_FB, IT_LM, IT_BS, IT_BB, IT_BDH, IT_BP, IT_BD, IT_NONE };
 struct ItemRec {
     int type, j;      // kind and index within its table
     int4 b;           // bead offsets (x3); unused entries repeat the first
     double p0, p1, p2, p3;
 };
+// record of lane i >= n_duo_lanes()
 __device__ __forceinline__ ItemRec fetch_rec(const Dev &D, int i) {
     ItemRec r;
     r.p0 = r.p1 = r.p2 = r.p3 = 0.0;
-    if (i < D.n_ev) {
-        r.type = D.ev_mon ? IT_EVM : IT_EV; r.j = i;
+    i -= D.n_duo_lanes();
+    const int n_evm = D.ev_mon ? D.n_ev : 0;
+    if (i < n_evm) {
+        r.type = IT_EVM; r.j = i;
         r.b = D.ev_bs[i];
         r.p0 = D.ev_kr[i];
-    } else if ((i -= D.n_ev) < D.n_fs) {
+    } else if ((i -= n_evm) < D.n_fs) {
         r.type = IT_FS; r.j = i;
         const int2 b = D.fs_bs[i];
         r.b = make_int4(b.x, b.y, b.x, b.x);
@@ -142,21 +248,10 @@ __device__ __forceinline__ ItemRec fetch_rec(const Dev &D, int i) {
     return r;
 }
 __device__ __forceinline__ int rec_nbeads(int type) {
-    return type == IT_EV || type == IT_EVM || type == IT_LM || type == IT_BB || type == IT_BDH ? 4
+    return type == IT_EVM || type == IT_LM || type == IT_BB || type == IT_BDH ? 4
          : type == IT_FB || type == IT_BS || type == IT_BP ? 3
          : type == IT_FS ? 2 : type == IT_BD ? 1 : 0;
 }
-// bead k's position (the unused entries of a record repeat its first bead)
-__device__ __forceinline__ d3 rec_pos(const PosAny &P, const ItemRec &r, int k) {
-    const int o = k == 0 ? r.b.x : k == 1 ? (r.type == IT_BD ? r.b.x : r.b.y) : k == 2 ? r.b.z : r.b.w;
-    return P(o);
-}
-
-// ---- one interaction from its record and positions: energy (into the exact
-// total and, if PER_FF, into the per-force-field double sums) and, if FORCES,
-// its per-bead force slots. One accumulation site and one copy of the
-// excluded-volume invariants and force keep the inlined code small (it runs
-// from the instruction cache of every CU).
 // Mixed-precision form: a pair's force runs in FP32 only when the squared
 // normalized triple product q = -JJ / (a b c) of the two cylinders is at
 // least this; nearer-coplanar pairs amplify FP32 rounding as ~6e-8 / q (at
@@ -164,66 +259,85 @@ __device__ __forceinline__ d3 rec_pos(const PosAny &P, const ItemRec &r, int k) 
 // the pairs of a random network qualify).
 constexpr double kMixedMinQ = 0.03;
 
+// ---- an excluded-volume pair on its two lanes, each having loaded its
+// cylinder's beads: energy (counted by lane 0) and, if FORCES, the four slots.
 // QUAD: the pairs flagged in D.evq are skipped (the quadrature kernels evaluate them).
-template <bool MIXED = false, bool QUAD = false>
+template <bool MIXED, bool QUAD, class P>
+__device__ __forceinline__ void ev_duo_item(const Dev &D, int i, const P &pos, double acc[kNFF], const XAdd &xs,
+                                            typename SlotT<MIXED>::T *__restrict__ contrib, const bool PER_FF,
+                                            const bool FORCES) {
+    const int j = i >> 1;
+    const bool h = (i & 1) != 0;
+    if (QUAD && D.evq[j]) return;
+    const int2 o = reinterpret_cast<const int2 *>(D.ev_bs)[i];
+    const double kr = D.ev_kr[j];
+    const int oo[2] = {o.x, o.y};
+    d3 mm[2];
+    pos.get(oo, mm);
+    const d3 m0 = mm[0];
+    d3 m1 = mm[1];
+    EvDuoT<double> v;
+    double U = 0.0;
+    // pass 0: the pair as given (energy, and force unless coplanar);
+    // pass 1: the coplanar perturbation of the reference force path,
+    // c2 moved off the plane (CylinderExclVolRepulsion.cpp:610-626)
+#pragma clang loop unroll(disable)
+    for (int pass = 0; pass < 2; pass++) {
+        const d3 c1 = duo_get<0>(m0), c2 = duo_get<0>(m1), c3 = duo_get<1>(m0), c4 = duo_get<1>(m1);
+        double block;
+        ev_duo_invariants(h, c1, c2, c3, c4, v, block);
+        if (pass == 0) {
+            U = ev_duo_energy(v, block, kr);
+            if (!FORCES || !(D.coplanar_mode == MDY_COPLANAR_REFERENCE && are_in_plane(c1, c2, c3, c4))) break;
+            const d3 c2e = moved_off_plane(c1, c2, c3, c2, 0.01);
+            m1 = pick3(h, m1, c2e);
+        }
+    }
+    if (!h) {
+        if (ev_energy_bad(U)) {
+            enqueue(D.qe, D.qe_n, j, D.err);
+        } else {
+            if (xs.x) xs(U);
+            if (PER_FF) acc[MDY_FF_EV] += U;
+        }
+    }
+    if (FORCES) {
+        const int s = D.slot_ev + 2 * i;
+        const d3 c1 = duo_get<0>(m0), c2 = duo_get<0>(m1), c3 = duo_get<1>(m0), c4 = duo_get<1>(m1);
+        if constexpr (MIXED) {
+            if (-v.JJ / (v.a * v.b * v.c) >= kMixedMinQ) {
+                // well-conditioned pair: derivative blocks in FP32
+                f3 f[2];
+                ev_duo_force<float>(h, v, c1, c2, c3, c4, kr, f);
+                if (!duo_any(!(finite_d3(f[0]) && finite_d3(f[1])))) {
+                    put3(contrib, s, f[0]); put3(contrib, s + 1, f[1]);
+                    return;
+                }
+            }
+        }
+        d3 f[2];
+        ev_duo_force<double>(h, v, c1, c2, c3, c4, kr, f);
+        if (duo_any(!(finite_d3(f[0]) && finite_d3(f[1])))) {
+            if (!h) enqueue(D.qf, D.qf_n, j, D.err);
+        } else {
+            put3(contrib, s, f[0]); put3(contrib, s + 1, f[1]);
+        }
+    }
+}
+
+// ---- one other interaction from its record and positions: energy (into the
+// exact total and, if PER_FF, into the per-force-field double sums) and, if
+// FORCES, its per-bead force slots. One accumulation site keeps the inlined
+// code small (it runs from the instruction cache of every CU).
+template <bool MIXED = false>
 __device__ __forceinline__ void item_compute(const Dev &D, const ItemRec &r, const d3 c[4], double acc[kNFF],
-                                             mdy_xsum &xs, typename SlotT<MIXED>::T *__restrict__ contrib,
+                                             const XAdd &xs, typename SlotT<MIXED>::T *__restrict__ contrib,
                                              const bool PER_FF, const bool FORCES) {
     double U = 0.0;
     int ff = 0;
     bool add = true;
     const int j = r.j;
-    if (QUAD && r.type == IT_EV && D.evq[j]) {
-        add = false;
-    } else if (r.type == IT_EV) {
-        const double kr = r.p0;
-        const d3 c1 = c[0], c2 = c[1], c3 = c[2], c4 = c[3];
-        ff = MDY_FF_EV;
-        EvInv v;
-        d3 c2e = c2;
-        // pass 0: the pair as given (energy, and force unless coplanar);
-        // pass 1: the coplanar perturbation of the reference force path,
-        // c2 moved off the plane (CylinderExclVolRepulsion.cpp:610-626)
-#pragma clang loop unroll(disable)
-        for (int pass = 0; pass < 2; pass++) {
-            ev_invariants(c1, c2e, c3, c4, v);
-            if (pass == 0) {
-                U = ev_energy_inv(v, kr);
-                if (!FORCES || !(D.coplanar_mode == MDY_COPLANAR_REFERENCE && are_in_plane(c1, c2, c3, c4))) break;
-                c2e = moved_off_plane(c1, c2, c3, c2, 0.01);
-            }
-        }
-        if (ev_energy_bad(U)) {
-            enqueue(D.qe, D.qe_n, j, D.err);
-            add = false;
-        }
-        if (FORCES) {
-            bool done = false;
-            if constexpr (MIXED) {
-                if (-v.JJ / (v.a * v.b * v.c) >= kMixedMinQ) {
-                    // well-conditioned pair: derivative blocks in FP32
-                    f3 f[4];
-                    ev_force_inv_t<float>(v, c1, c2e, c3, c4, kr, f);
-                    if (finite_d3(f[0]) && finite_d3(f[1]) && finite_d3(f[2]) && finite_d3(f[3])) {
-                        int s = D.slot_ev + 4 * j;
-                        put3(contrib, s, f[0]); put3(contrib, s + 1, f[1]);
-                        put3(contrib, s + 2, f[2]); put3(contrib, s + 3, f[3]);
-                        done = true;
-                    }
-                }
-            }
-            if (!done) {
-                d3 f[4];
-                ev_force_inv(v, c1, c2e, c3, c4, kr, f);
-                if (!(finite_d3(f[0]) && finite_d3(f[1]) && finite_d3(f[2]) && finite_d3(f[3]))) {
-                    enqueue(D.qf, D.qf_n, j, D.err);
-                } else {
-                    int s = D.slot_ev + 4 * j;
-                    put3(contrib, s, f[0]); put3(contrib, s + 1, f[1]); put3(contrib, s + 2, f[2]); put3(contrib, s + 3, f[3]);
-                }
-            }
-        }
-    } else if (r.type == IT_EVM) {   // monomer-pair sum, in FP64 in both forms; no fallbacks
+    if (r.type == IT_EVM) {   // monomer-pair sum, in FP64 in both forms; no fallbacks
         ff = MDY_FF_EV;
         const int2 cc = D.ev_cyl[j];
         const int4 m1 = D.cyl_mon[cc.x], m2 = D.cyl_mon[cc.y];
@@ -308,7 +422,7 @@ __device__ __forceinline__ void item_compute(const Dev &D, const ItemRec &r, con
         add = false;
     }
     if (add) {
-        mdy_xs_add(&xs, U);
+        if (xs.x) xs(U);
         if (PER_FF) {
 #pragma unroll
             for (int k = 0; k < kNFF; k++) acc[k] += (k == ff) ? U : 0.0;
@@ -316,114 +430,90 @@ __device__ __forceinline__ void item_compute(const Dev &D, const ItemRec &r, con
     }
 }
 
-// All items i = start, start + stride, ... below D.n_items() at positions P.
-// (Fetching the next record ahead of the arithmetic was measured slower: the
-// extra live registers cost more than the memory round trip they hide.)
-template <bool MIXED = false>
-__device__ __forceinline__ void sweep(const Dev &D, const PosAny &P, int start, int stride, double acc[kNFF],
-                                      mdy_xsum &xs, typename SlotT<MIXED>::T *__restrict__ contrib,
-                                      const bool PER_FF, const bool FORCES) {
-    const int total = D.n_items();
-    for (int i = start; i < total; i += stride) {
-        const ItemRec r = fetch_rec(D, i);
-        const int nb = rec_nbeads(r.type);
-        d3 c[4];
-        c[0] = rec_pos(P, r, 0);
-        c[1] = nb > 1 ? rec_pos(P, r, 1) : c[0];
-        c[2] = nb > 2 ? rec_pos(P, r, 2) : c[0];
-        c[3] = nb > 3 ? rec_pos(P, r, 3) : c[0];
-        item_compute<MIXED>(D, r, c, acc, xs, contrib, PER_FF, FORCES);
-    }
-}
-
-// single item (one-shot kernels)
+// lane i of the sweep's index space
 template <bool MIXED = false, bool QUAD = false, class P>
-__device__ __forceinline__ void item(const Dev &D, int i, const P &pos, double acc[kNFF], mdy_xsum &xs,
+__device__ __forceinline__ void item(const Dev &D, int i, const P &pos, double acc[kNFF], const XAdd &xs,
                                      typename SlotT<MIXED>::T *__restrict__ contrib, const bool PER_FF,
                                      const bool FORCES) {
-    ItemRec r = fetch_rec(D, i);
-    const int nb = rec_nbeads(r.type);
-    d3 c[4];
-    c[0] = pos(r.b.x);
-    c[1] = nb > 1 ? pos(r.b.y) : c[0];
-    c[2] = nb > 2 ? pos(r.b.z) : c[0];
-    c[3] = nb > 3 ? pos(r.b.w) : c[0];
-    item_compute<MIXED, QUAD>(D, r, c, acc, xs, contrib, PER_FF, FORCES);
-}
-
-// Slots k0..k1-1 of a bead's row (after the ones loaded with the row's
-// first), added in order. CHUNKED: kTail indices, then their kTail values, at
-// a time, so a bead with many slots (up to ~60 in a 200k-cylinder network)
-// costs two dependent round trips per kTail slots rather than per slot;
-// otherwise one slot at a time (fewer instructions where rows rarely go past
-// their first loads).
-constexpr int kTail = 8;
-template <bool CHUNKED, class S>
-__device__ __forceinline__ void gather_tail(const int *__restrict__ idx, int k0, int k1, const S *__restrict__ contrib,
-                                            double &fx, double &fy, double &fz) {
-    if (!CHUNKED) {
-        for (int k = k0; k < k1; k++) {
-            const int s = idx[k];
-            fx += contrib[3 * s]; fy += contrib[3 * s + 1]; fz += contrib[3 * s + 2];
-        }
+    if (i < D.n_duo_lanes()) {
+        ev_duo_item<MIXED, QUAD>(D, i, pos, acc, xs, contrib, PER_FF, FORCES);
         return;
     }
-#pragma clang loop unroll(disable)
-    for (int k = k0; k < k1; k += kTail) {
-        int ix[kTail];
-#pragma unroll
-        for (int j = 0; j < kTail; j++) ix[j] = (k + j < k1) ? idx[k + j] : 0;
-        S v[kTail][3];
-#pragma unroll
-        for (int j = 0; j < kTail; j++)
-            if (k + j < k1) { v[j][0] = contrib[3 * ix[j]]; v[j][1] = contrib[3 * ix[j] + 1]; v[j][2] = contrib[3 * ix[j] + 2]; }
-#pragma unroll
-        for (int j = 0; j < kTail; j++)
-            if (k + j < k1) { fx += v[j][0]; fy += v[j][1]; fz += v[j][2]; }
+    const ItemRec r = fetch_rec(D, i);
+    d3 c[4];
+    const int o1 = r.type == IT_BD ? r.b.x : r.b.y;   // a boundary record's second entry is its plane
+    if (__any(rec_nbeads(r.type) > 2)) {
+        const int o[4] = {r.b.x, o1, r.b.z, r.b.w};
+        pos.get(o, c);
+    } else {   // a wave of stretching or boundary terms
+        const int o[2] = {r.b.x, o1};
+        d3 q[2];
+        pos.get(o, q);
+        c[0] = c[2] = c[3] = q[0];
+        c[1] = q[1];
+    }
+    item_compute<MIXED>(D, r, c, acc, xs, contrib, PER_FF, FORCES);
+}
+
+// Block blk of nblk's lanes of the index space at positions pos. Chunks of 64
+// lanes (a wave) go to the blocks in turn, chunk c to block c % nblk, so that
+// every CU gets its share of each kind of item: the kinds are contiguous in the
+// index space and differ by a factor of five in time. The terms go into sum 0
+// of x (null: forces only).
+template <bool MIXED, bool QUAD, class P>
+__device__ __forceinline__ void sweep(const Dev &D, const P &pos, int blk, int nblk, double acc[kNFF], XBlock *x,
+                                      typename SlotT<MIXED>::T *__restrict__ contrib, const bool PER_FF,
+                                      const bool FORCES) {
+    const int total = D.n_lanes(), stride = nblk * (int)blockDim.x;
+    const int first = (((int)threadIdx.x >> 6) * nblk + blk) * 64 + ((int)threadIdx.x & 63);
+    if (FORCES && first == 0) put_none(D, contrib);
+    int turn = 0;
+    for (int base = 0; base < total; base += stride) {
+        if (x && turn == kXTurns) { xblock_norm(*x); turn = 0; }
+        turn++;
+        const int i = base + first;
+        if (i < total) item<MIXED, QUAD>(D, i, pos, acc, XAdd{x, 0}, contrib, PER_FF, FORCES);
+        if (total - base <= stride) break;   // base + stride may pass the range of int
     }
 }
-// Per-bead force: the slots of bead b in reference order, starting from 0.0
-// (ForceFieldManager::computeForces zero-fills, then each force field adds).
-// The first kGS static and kGD dynamic slot indices and values are loaded
-// together before any addition, so a bead costs three dependent memory round
-// trips (offsets, indices, values) instead of two per slot; slots beyond
-// those follow in chunks in the narrow form (gather_tail). Every phase waits
-// for its slowest bead, so when a
-// thread gathers one bead (the minimizer on networks with fewer beads than
-// threads) the wide form (12 static, 24 dynamic) covers the beads with the
-// most slots; with several beads per thread the narrow form's fewer
-// instructions per bead win.
-template <int kGS, int kGD, class S>
-__device__ __forceinline__ d3 gather_bead_w(const Dev &D, const S *__restrict__ contrib, int b) {
-    const int s0 = D.st_off[b], s1 = D.st_off[b + 1], d0 = D.dy_off[b], d1 = D.dy_off[b + 1];
-    int is[kGS], id[kGD];
-#pragma unroll
-    for (int j = 0; j < kGS; j++) is[j] = (s0 + j < s1) ? D.st_idx[s0 + j] : 0;
-#pragma unroll
-    for (int j = 0; j < kGD; j++) id[j] = (d0 + j < d1) ? D.dy_idx[d0 + j] : 0;
-    S vs[kGS][3], vd[kGD][3];
-#pragma unroll
-    for (int j = 0; j < kGS; j++) {
-        if (s0 + j < s1) { vs[j][0] = contrib[3 * is[j]]; vs[j][1] = contrib[3 * is[j] + 1]; vs[j][2] = contrib[3 * is[j] + 2]; }
-    }
-#pragma unroll
-    for (int j = 0; j < kGD; j++) {
-        if (d0 + j < d1) { vd[j][0] = contrib[3 * id[j]]; vd[j][1] = contrib[3 * id[j] + 1]; vd[j][2] = contrib[3 * id[j] + 2]; }
-    }
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-#pragma unroll
-    for (int j = 0; j < kGS; j++)
-        if (s0 + j < s1) { fx += vs[j][0]; fy += vs[j][1]; fz += vs[j][2]; }
-    gather_tail<(kGS <= 8)>(D.st_idx, s0 + kGS, s1, contrib, fx, fy, fz);
-#pragma unroll
-    for (int j = 0; j < kGD; j++)
-        if (d0 + j < d1) { fx += vd[j][0]; fy += vd[j][1]; fz += vd[j][2]; }
-    gather_tail<(kGS <= 8)>(D.dy_idx, d0 + kGD, d1, contrib, fx, fy, fz);
-    return d3{fx, fy, fz};
-}
+
+// Force on one coordinate, o = 3 * bead + axis: its bead's slots in reference
+// order, starting from 0.0 (ForceFieldManager::computeForces zero-fills, then
+// each force field adds). One lane per coordinate: three lanes share a bead's
+// row and read neighboring words of its records, so a wave's loads touch
+// about 21 beads' lines instead of 64, and the vectors that the caller reads
+// and writes next to it are contiguous. The row comes in groups of four slot
+// offsets, filled up with the offset of a record of -0.0, the addition that
+// changes nothing; sixteen values are in flight at a time.
+constexpr int kRowGroups = 4;
 template <class S>
-__device__ __forceinline__ d3 gather_bead(const Dev &D, const S *__restrict__ contrib, int b) {
-    return gather_bead_w<8, 8>(D, contrib, b);
+__device__ __forceinline__ double gather_coord(const Dev &D, const S *__restrict__ contrib, int o) {
+    const int b = o / 3, c = o - 3 * b;
+    const int g1 = D.row_off[b + 1];
+    double f = 0.0;
+    for (int g = D.row_off[b]; g < g1; g += kRowGroups) {
+        int4 id[kRowGroups];
+        const int none = 3 * D.n_slots;
+#pragma unroll
+        for (int m = 0; m < kRowGroups; m++) {
+            id[m] = D.row_idx[min(g + m, g1 - 1)];
+            if (g + m >= g1) id[m] = make_int4(none, none, none, none);
+        }
+        S v[4 * kRowGroups];
+#pragma unroll
+        for (int m = 0; m < kRowGroups; m++) {
+            v[4 * m] = contrib[id[m].x + c]; v[4 * m + 1] = contrib[id[m].y + c];
+            v[4 * m + 2] = contrib[id[m].z + c]; v[4 * m + 3] = contrib[id[m].w + c];
+        }
+#pragma unroll
+        for (int m = 0; m < 4 * kRowGroups; m++) f += v[m];
+    }
+    return f;
+}
+// the record that fills up the rows
+template <class S>
+__device__ __forceinline__ void put_none(const Dev &D, S *__restrict__ contrib) {
+    put3(contrib, D.n_slots, vec3_none<S>());
 }
 
 // ---- block reductions (fixed butterfly + fixed wave order: deterministic) ----
@@ -503,104 +593,6 @@ __device__ __forceinline__ void block_reduce_xsum(mdy_xsum &s, long long *lds) {
     s.flags = (int)lds[128 + 7];
     mdy_xs_norm(&s);
     __syncthreads();
-}
-// Two block sums in one pass (one set of barriers, interleaved shuffles).
-// lds: >= 17 * 16 int64.
-__device__ __forceinline__ void block_reduce_xsum2(mdy_xsum &s, mdy_xsum &t, long long *lds) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    mdy_xs_norm(&s);
-    mdy_xs_norm(&t);
-#pragma unroll
-    for (int k = 0; k < MDY_XS_N; k++) {
-        const long long r = wave_sum_i64(s.d[k]), q = wave_sum_i64(t.d[k]);
-        if (lane == 0) { lds[wave * 16 + k] = r; lds[wave * 16 + 8 + k] = q; }
-    }
-    const int f = wave_or(s.flags), g = wave_or(t.flags);
-    if (lane == 0) { lds[wave * 16 + 7] = f; lds[wave * 16 + 15] = g; }
-    __syncthreads();
-    if (threadIdx.x < 16) {
-        const int k = threadIdx.x;
-        long long r = lds[k];
-        for (int w = 1; w < nw; w++) r = ((k & 7) == 7) ? (r | lds[w * 16 + k]) : r + lds[w * 16 + k];
-        lds[256 + k] = r;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < MDY_XS_N; k++) { s.d[k] = lds[256 + k]; t.d[k] = lds[256 + 8 + k]; }
-    s.flags = (int)lds[256 + 7];
-    t.flags = (int)lds[256 + 15];
-    mdy_xs_norm(&s);
-    mdy_xs_norm(&t);
-    __syncthreads();
-}
-// Block-wide combination of NW 64-bit words per thread through LDS: word k
-// is summed, or OR-ed where bit k of or_mask is set, or unsigned-max-ed where
-// bit k of max_mask is set. Every thread writes its words; one thread per
-// 16-entry chunk combines it; one thread per word combines the chunks; every
-// thread reads the results. Exact for integers, so the result does not depend
-// on the order, and it takes three short LDS round trips instead of the
-// dependent shuffle chains of a butterfly. blockDim.x must be a multiple of 16.
-// lds: >= block_combine_words(NW) 64-bit words.
-__host__ __device__ constexpr int block_combine_words(int nw, int nthreads = kBlock) {
-    return nw * (nthreads + nthreads / 16 + 1);
-}
-template <int NW>
-__device__ __forceinline__ void block_combine(long long w[NW], long long *lds, unsigned or_mask, unsigned max_mask) {
-    const int n = blockDim.x, t = threadIdx.x, nch = n >> 4;
-    long long *part = lds + NW * n;
-    long long *res = part + NW * nch;
-#pragma unroll
-    for (int k = 0; k < NW; k++) lds[k * n + t] = w[k];
-    __syncthreads();
-    for (int job = t; job < NW * nch; job += n) {
-        const int k = job / nch, c = job - k * nch;
-        const bool isor = (or_mask >> k) & 1u, ismax = (max_mask >> k) & 1u;
-        const long long *src = lds + k * n + c * 16;
-        long long r = src[0];
-#pragma unroll
-        for (int j = 1; j < 16; j++) {
-            const long long v = src[j];
-            r = isor ? (r | v) : ismax ? ((unsigned long long)v > (unsigned long long)r ? v : r) : r + v;
-        }
-        part[k * nch + c] = r;
-    }
-    __syncthreads();
-    if (t < NW) {
-        const bool isor = (or_mask >> t) & 1u, ismax = (max_mask >> t) & 1u;
-        long long r = part[t * nch];
-        for (int c = 1; c < nch; c++) {
-            const long long v = part[t * nch + c];
-            r = isor ? (r | v) : ismax ? ((unsigned long long)v > (unsigned long long)r ? v : r) : r + v;
-        }
-        res[t] = r;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < NW; k++) w[k] = res[k];
-    __syncthreads();
-}
-// Exact block sums of two per-thread accumulators through block_combine;
-// with_max: also the maximum of a non-negative double m (all threads get it).
-__device__ __forceinline__ void block_reduce_xsum2_lds(mdy_xsum &s, mdy_xsum &t, long long *lds, double *m = nullptr) {
-    mdy_xs_norm(&s);   // digits below 2^48: a block's sum of them cannot overflow
-    mdy_xs_norm(&t);
-    long long w[17];
-#pragma unroll
-    for (int k = 0; k < MDY_XS_N; k++) { w[k] = s.d[k]; w[8 + k] = t.d[k]; }
-    w[7] = s.flags;
-    w[15] = t.flags;
-    w[16] = m ? __double_as_longlong(*m) : 0;
-    if (m) block_combine<17>(w, lds, (1u << 7) | (1u << 15), 1u << 16);
-    else block_combine<16>(w, lds, (1u << 7) | (1u << 15), 0u);
-#pragma unroll
-    for (int k = 0; k < MDY_XS_N; k++) { s.d[k] = w[k]; t.d[k] = w[8 + k]; }
-    s.flags = (int)w[7];
-    t.flags = (int)w[15];
-    s.cnt = 0;
-    t.cnt = 0;
-    mdy_xs_norm(&s);
-    mdy_xs_norm(&t);
-    if (m) *m = __longlong_as_double(w[16]);
 }
 // per-block partial records: [blk * kRed + off .. off+7] hold a normalized accumulator
 __device__ __forceinline__ void store_xsum(double *red, int blk, int off, const mdy_xsum &s) {

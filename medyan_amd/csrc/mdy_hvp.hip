@@ -18,13 +18,7 @@ namespace mdy {
 // returns the force-field index, or -1 for an empty record.
 template <class T>
 __device__ __forceinline__ int item_forces(const Dev &D, const ItemRec &r, const V3<T> c[4], V3<T> f[4]) {
-    if (r.type == IT_EV) {
-        if (D.evq && D.evq[r.j]) return -1;   // quadrature mode: evaluated by the quadrature kernels
-        EvInvT<T> inv;
-        ev_invariants(c[0], c[1], c[2], c[3], inv);
-        ev_force_inv_t<T>(inv, c[0], c[1], c[2], c[3], r.p0, f);
-        return MDY_FF_EV;
-    } else if (r.type == IT_EVM) {
+    if (r.type == IT_EVM) {
         const int2 cc = D.ev_cyl[r.j];
         (void)evm_eval<T, true>(c[0], c[1], c[2], c[3], D.cyl_mon[cc.x], D.cyl_mon[cc.y], r.p0, f);
         return MDY_FF_EV;
@@ -59,7 +53,6 @@ __device__ __forceinline__ int item_forces(const Dev &D, const ItemRec &r, const
 
 __device__ __forceinline__ int item_slot(const Dev &D, const ItemRec &r) {
     switch (r.type) {
-        case IT_EV:
         case IT_EVM: return D.slot_ev + 4 * r.j;
         case IT_FS: return D.slot_fs + 2 * r.j;
         case IT_FB: return D.slot_fb + 3 * r.j;
@@ -80,8 +73,33 @@ __device__ __forceinline__ int bead_off(const ItemRec &r, int k) {
 // lane spilled; at one wave the kernel needed 286): 13 % faster at 50k.
 __global__ void __launch_bounds__(kBlock, 2) k_hvp(Dev D, const double *__restrict__ x, const double *__restrict__ v,
                                                  double *__restrict__ contrib) {
-    const int total = D.n_items(), gs = gridDim.x * blockDim.x;
+    const int total = D.n_lanes(), gs = gridDim.x * blockDim.x;
+    atan_table_fill();
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x == 0) put_none(D, contrib);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gs) {
+        if (i < D.n_duo_lanes()) {   // an excluded-volume pair's two lanes, one per cylinder
+            if (D.evq && D.evq[i >> 1]) continue;   // evaluated by the quadrature kernels
+            const bool h = (i & 1) != 0;
+            const int2 o = reinterpret_cast<const int2 *>(D.ev_bs)[i];
+            auto at = [&](int k) {
+                return V3<Dual>{Dual(x[k], v[k]), Dual(x[k + 1], v[k + 1]), Dual(x[k + 2], v[k + 2])};
+            };
+            const V3<Dual> m0 = at(o.x), m1 = at(o.y);
+            const V3<Dual> c1 = duo_get<0>(m0), c2 = duo_get<0>(m1), c3 = duo_get<1>(m0), c4 = duo_get<1>(m1);
+            EvDuoT<Dual> inv;
+            Dual block;
+            ev_duo_invariants(h, c1, c2, c3, c4, inv, block);
+            V3<Dual> f[2];
+            ev_duo_force<Dual>(h, inv, c1, c2, c3, c4, D.ev_kr[i >> 1], f);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const d3 hv{-f[k].x.d, -f[k].y.d, -f[k].z.d};
+                if (!finite_d3(hv)) set_err(D.err, MDY_ERR_FORCE);
+                put3(contrib, D.slot_ev + 2 * i + k, hv);
+            }
+            continue;
+        }
         const ItemRec r = fetch_rec(D, i);
         const int nb = rec_nbeads(r.type);
         V3<Dual> c[4], f[4];
@@ -106,15 +124,10 @@ __global__ void __launch_bounds__(kBlock, 2) k_hvp(Dev D, const double *__restri
     }
 }
 
-// WIDE: the wide per-bead form (fewer beads than one block per CU has
-// threads); same sums either way
-template <bool WIDE>
 __global__ void __launch_bounds__(kBlock) k_hvp_gather(Dev D, const double *__restrict__ contrib,
                                                         double *__restrict__ hv) {
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < D.nb; b += gridDim.x * blockDim.x) {
-        const d3 h = WIDE ? gather_bead_w<12, 24>(D, contrib, b) : gather_bead(D, contrib, b);
-        hv[3 * b] = h.x; hv[3 * b + 1] = h.y; hv[3 * b + 2] = h.z;
-    }
+    for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < D.ndof; o += gridDim.x * blockDim.x)
+        hv[o] = gather_coord(D, contrib, o);
 }
 
 // per-block partial sums of grad E_k . w = -sum over an interaction's beads of F . w
@@ -124,9 +137,27 @@ __global__ void __launch_bounds__(kBlock) k_energy_jvp(Dev D, const double *__re
     double acc[kNFF];
 #pragma unroll
     for (int k = 0; k < kNFF; k++) acc[k] = 0.0;
-    const int total = D.n_items(), gs = gridDim.x * blockDim.x;
+    const int total = D.n_lanes(), gs = gridDim.x * blockDim.x;
     bool ok = true;
+    atan_table_fill();
+    __syncthreads();
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gs) {
+        if (i < D.n_duo_lanes()) {   // an excluded-volume pair's two lanes, one per cylinder
+            if (D.evq && D.evq[i >> 1]) continue;   // evaluated by the quadrature kernels
+            const bool h = (i & 1) != 0;
+            const int2 o = reinterpret_cast<const int2 *>(D.ev_bs)[i];
+            const d3 m0 = ld3(x + o.x), m1 = ld3(x + o.y);
+            const d3 c1 = duo_get<0>(m0), c2 = duo_get<0>(m1), c3 = duo_get<1>(m0), c4 = duo_get<1>(m1);
+            EvDuoT<double> inv;
+            double block;
+            ev_duo_invariants(h, c1, c2, c3, c4, inv, block);
+            d3 f[2];
+            ev_duo_force<double>(h, inv, c1, c2, c3, c4, D.ev_kr[i >> 1], f);
+            ok = ok && finite_d3(f[0]) && finite_d3(f[1]);
+            acc[MDY_FF_EV] -= f[0].x * w[o.x] + f[0].y * w[o.x + 1] + f[0].z * w[o.x + 2] + f[1].x * w[o.y] +
+                              f[1].y * w[o.y + 1] + f[1].z * w[o.y + 2];
+            continue;
+        }
         const ItemRec r = fetch_rec(D, i);
         const int nb = rec_nbeads(r.type);
         d3 c[4], f[4];
@@ -193,17 +224,16 @@ int launch_hvp(Ctx &c, const double *d_x, const double *d_v, double *d_hv, hipSt
     Dev D = c.dev();
     const bool quad = quad_on(c);
     if (quad) MDY_TRY(quad_classify(c, D, d_x, st));
-    hipLaunchKernelGGL(k_hvp, dim3(grid_of(c, D.n_items())), dim3(kBlock), 0, st, D, d_x, d_v, c.contrib.p);
+    hipLaunchKernelGGL(k_hvp, dim3(grid_of(c, D.n_lanes())), dim3(kBlock), 0, st, D, d_x, d_v, c.contrib.p);
     if (quad) MDY_TRY(launch_quad(c, D, 2, d_x, d_v, c.contrib.p, 0, st));
-    hipLaunchKernelGGL(D.nb <= c.num_cu * kBlock ? k_hvp_gather<true> : k_hvp_gather<false>, dim3(grid_of(c, D.nb)),
-                       dim3(kBlock), 0, st, D, c.contrib.p, d_hv);
+    hipLaunchKernelGGL(k_hvp_gather, dim3(grid_of(c, D.ndof)), dim3(kBlock), 0, st, D, c.contrib.p, d_hv);
     if (!sync) return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
     return sync_errors(c, st);
 }
 
 int launch_energy_jvp(Ctx &c, const double *d_x, const double *d_w, double *d_out, hipStream_t st) {
     Dev D = c.dev();
-    const int nblk = grid_of(c, D.n_items());
+    const int nblk = grid_of(c, D.n_lanes());
     const bool quad = quad_on(c);
     const int nqb = quad ? quad_blocks(c) : 0;   // the quadrature pairs' block records follow the others
     MDY_TRY(ensure(c.red, (size_t)kRed * (nblk + nqb)));

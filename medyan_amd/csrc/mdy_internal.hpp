@@ -16,8 +16,8 @@ constexpr int kQueueCap = 4096;      // excluded-volume quadrature fallback queu
 constexpr int kRed = 32;             // 8-byte words per block in a reduction record
 
 // Interaction tables on the device. The evaluation index space is
-// [EV | FS | FB | LM | BS | BB | BD]: excluded volume first so its costly
-// items are packed densely into the first waves of the grid.
+// [EV | FS | FB | LM | BS | BB | BDH | BP | BD]: excluded volume first so its
+// costly items are packed densely into the first waves of the grid.
 // Force slots (3 doubles each) follow the reference force-field order
 // FS, FB, LS, MS, BS, BB, EV, BD, so the per-bead gather adds contributions in
 // the order ForceFieldManager::computeForces would.
@@ -38,8 +38,9 @@ struct Dev {
     const int *bp_bs; const double *bp_k, *bp_pos;               // branching position
     const int *bd_bead; const int *bd_plane; const double *bd_k, *bd_sl; const double *planes;
     int slot_fs, slot_fb, slot_lm, slot_bs, slot_bb, slot_bdh, slot_bp, slot_ev, slot_bd, n_slots;
-    const int *st_off, *st_idx;   // static CSR: bead -> bonded/cross-link slots
-    const int *dy_off, *dy_idx;   // dynamic CSR: bead -> excluded-volume/boundary slots
+    // bead -> its slots in slot order, as offsets 3 * slot in groups of four (the last one filled
+    // up with 3 * n_slots): bead b's groups are row_off[b] .. row_off[b + 1] - 1
+    const int *row_off; const int4 *row_idx;
     int coplanar_mode;
     const unsigned char *evq;     // quadrature mode: per excluded-volume pair, 1 = evaluated by quadrature
     double cq, sq;                // cos and sin of pi/2 (C library), branching position
@@ -48,6 +49,9 @@ struct Dev {
     int *qf, *qf_n;               // force
     int *err;                     // sticky device error word (MDY_ERR_*)
     __host__ __device__ int n_items() const { return n_ev + n_fs + n_fb + n_lm + n_bs + n_bb + n_bdh + n_bp + n_bd; }
+    // lanes of a sweep: two per excluded-volume pair of the integral form, one per other interaction
+    __host__ __device__ int n_duo_lanes() const { return ev_mon ? 0 : 2 * n_ev; }
+    __host__ __device__ int n_lanes() const { return n_items() + (ev_mon ? 0 : n_ev); }
 };
 
 template <class T>
@@ -76,7 +80,7 @@ struct Ctx {
     DBuf<int4> bb_bs; DBuf<double> bb_k, bb_th, bb_ct, bb_st;
     DBuf<int4> bdh_bs; DBuf<double> bdh_k, bdh_pos;
     DBuf<int> bp_bs; DBuf<double> bp_k, bp_pos;
-    DBuf<int> st_off, st_idx;
+    DBuf<int> st_off, st_idx;   // bead -> bonded / cross-link slots
     int n_fs = 0, n_fb = 0, n_ls = 0, n_ms = 0, n_bs = 0, n_bb = 0, n_bdh = 0, n_bp = 0;
     // cylinders
     DBuf<int> c_b1, c_b2, c_fil, c_pos, c_child; DBuf<long long> c_id; DBuf<short> c_type;
@@ -99,7 +103,8 @@ struct Ctx {
     DBuf<int2> ev_cyl;            // monomer-sum form: cylinders of each pair
     DBuf<int> bd_flag, bd_off, bd_bead, bd_plane; DBuf<double> bd_k, bd_sl; int n_bd = 0;
     std::vector<int> h_bd_nneigh;
-    DBuf<int> dy_cnt, dy_off, dy_cur, dy_idx;
+    DBuf<int> row_cnt4, row_off4, row_cur; DBuf<int4> row_idx, row_tmp;   // bead -> all slots (Dev::row_idx)
+    int n_static = 0;             // entries of st_idx
     DBuf<unsigned char> evq;      // quadrature mode: per-pair flags of the current evaluation
     DBuf<int> qpan, qcnt, qoff, qmap; // quadrature mode: panels, chunk counts, first chunks, chunk -> pair
     DBuf<int> qtot;               // quadrature mode: running chunk total (zero between calls)

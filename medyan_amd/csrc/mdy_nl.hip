@@ -213,42 +213,59 @@ __global__ void k_bd_emit(int ncyl, int np, const int *b1, const int *b2, const 
     }
 }
 
-// dynamic CSR: bead -> excluded-volume / boundary slots, rows sorted by slot
+// The gather's rows (Dev::row_idx): a bead's bonded slots, then its
+// excluded-volume and boundary slots in slot order.
 __device__ __forceinline__ int dyn_slot_bead(const Dev &D, int j, int &slot) {
-    int nev4 = 4 * D.n_ev;
+    const int nev4 = 4 * D.n_ev;
     if (j < nev4) {
-        int4 b = D.ev_bs[j >> 2];
-        int o = (j & 3) == 0 ? b.x : (j & 3) == 1 ? b.y : (j & 3) == 2 ? b.z : b.w;
         slot = D.slot_ev + j;
-        return o / 3;
+        return reinterpret_cast<const int *>(D.ev_bs)[j] / 3;
     }
     j -= nev4;
     slot = D.slot_bd + j;
     return D.bd_bead[j] / 3;
 }
-__global__ void k_dy_count(Dev D, int *cnt) {
+__global__ void k_row_count(Dev D, int *cur) {
     const int tot = 4 * D.n_ev + D.n_bd;
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < tot; j += gridDim.x * blockDim.x) {
         int s;
-        atomicAdd(cnt + dyn_slot_bead(D, j, s), 1);
+        atomicAdd(cur + dyn_slot_bead(D, j, s), 1);
     }
 }
-__global__ void k_dy_fill(Dev D, const int *off, int *cur, int *idx) {
+// groups of four per row; the counters restart for the fill
+__global__ void k_row_groups(int nb, const int *__restrict__ st_off, int *cur, int *cnt4) {
+    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b <= nb; b += gridDim.x * blockDim.x) {
+        cnt4[b] = b < nb ? (st_off[b + 1] - st_off[b] + cur[b] + 3) / 4 : 0;
+        if (b < nb) cur[b] = 0;
+    }
+}
+// dynamic slots in any order, after the room of the bonded ones
+__global__ void k_row_fill(Dev D, const int *__restrict__ st_off, int *cur, int *tmp) {
     const int tot = 4 * D.n_ev + D.n_bd;
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < tot; j += gridDim.x * blockDim.x) {
         int s;
-        int b = dyn_slot_bead(D, j, s);
-        idx[off[b] + atomicAdd(cur + b, 1)] = s;
+        const int b = dyn_slot_bead(D, j, s);
+        tmp[4 * D.row_off[b] + (st_off[b + 1] - st_off[b]) + atomicAdd(cur + b, 1)] = s;
     }
 }
-__global__ void k_dy_sort(int nb, const int *off, int *idx) {
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x) {
-        int s0 = off[b], e = off[b + 1];
-        for (int a = s0 + 1; a < e; a++) {
-            int v = idx[a], k = a - 1;
-            while (k >= s0 && idx[k] > v) { idx[k + 1] = idx[k]; k--; }
-            idx[k + 1] = v;
+// Eight lanes per bead: the bonded slots copied, each dynamic slot placed by
+// counting the smaller ones of its row (rows hold ~10, all in cache), the last
+// group filled up.
+__global__ void k_row_place(Dev D, const int *__restrict__ st_off, const int *__restrict__ st_idx,
+                            const int *__restrict__ cur, const int *__restrict__ tmp, int *__restrict__ out) {
+    const int q = threadIdx.x & 7;
+    for (int b = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; b < D.nb; b += (gridDim.x * blockDim.x) >> 3) {
+        const int s0 = st_off[b], ns = st_off[b + 1] - s0, nd = cur[b];
+        const int r0 = 4 * D.row_off[b], r1 = 4 * D.row_off[b + 1];
+        for (int k = q; k < ns; k += 8) out[r0 + k] = 3 * st_idx[s0 + k];
+        const int *row = tmp + r0 + ns;
+        for (int k = q; k < nd; k += 8) {
+            const int v = row[k];
+            int rank = 0;
+            for (int m = 0; m < nd; m++) rank += row[m] < v ? 1 : 0;
+            out[r0 + ns + rank] = 3 * v;
         }
+        for (int k = r0 + ns + nd + q; k < r1; k += 8) out[k] = 3 * D.n_slots;
     }
 }
 
@@ -377,19 +394,24 @@ int build_neighbors(Ctx &c, const double *d_x) {
     Dev D = c.dev();
     const int nb = c.nb;
     const int ndyn = 4 * c.n_ev + c.n_bd;
-    MDY_TRY(ensure(c.dy_cnt, (size_t)nb + 1));
-    MDY_TRY(ensure(c.dy_cur, (size_t)nb + 1));
-    MDY_TRY(ensure(c.dy_off, (size_t)nb + 2));
-    MDY_TRY(ensure(c.dy_idx, (size_t)ndyn + 1));
-    hipLaunchKernelGGL(k_fill_int, dim3(grid1(c, nb + 1)), dim3(kBlock), 0, st, c.dy_cnt.p, nb + 1, 0);
-    hipLaunchKernelGGL(k_fill_int, dim3(grid1(c, nb + 1)), dim3(kBlock), 0, st, c.dy_cur.p, nb + 1, 0);
+    MDY_TRY(ensure(c.row_cur, (size_t)nb + 1));
+    MDY_TRY(ensure(c.row_cnt4, (size_t)nb + 1));
+    MDY_TRY(ensure(c.row_off4, (size_t)nb + 2));
+    // every row's last group may be filled up with three entries
+    const size_t groups = ((size_t)c.n_static + ndyn) / 4 + nb + 1;
+    MDY_TRY(ensure(c.row_idx, groups));
+    MDY_TRY(ensure(c.row_tmp, groups));
+    hipLaunchKernelGGL(k_fill_int, dim3(grid1(c, nb + 1)), dim3(kBlock), 0, st, c.row_cur.p, nb + 1, 0);
     D = c.dev();
-    if (ndyn > 0) hipLaunchKernelGGL(k_dy_count, dim3(grid1(c, ndyn)), dim3(kBlock), 0, st, D, c.dy_cnt.p);
-    MDY_TRY(exclusive_scan(c, c.dy_cnt.p, c.dy_off.p, nb, st));
-    if (ndyn > 0) {
-        hipLaunchKernelGGL(k_dy_fill, dim3(grid1(c, ndyn)), dim3(kBlock), 0, st, D, c.dy_off.p, c.dy_cur.p, c.dy_idx.p);
-        hipLaunchKernelGGL(k_dy_sort, dim3(grid1(c, nb)), dim3(kBlock), 0, st, nb, c.dy_off.p, c.dy_idx.p);
-    }
+    if (ndyn > 0) hipLaunchKernelGGL(k_row_count, dim3(grid1(c, ndyn)), dim3(kBlock), 0, st, D, c.row_cur.p);
+    hipLaunchKernelGGL(k_row_groups, dim3(grid1(c, nb + 1)), dim3(kBlock), 0, st, nb, c.st_off.p, c.row_cur.p,
+                       c.row_cnt4.p);
+    MDY_TRY(exclusive_scan(c, c.row_cnt4.p, c.row_off4.p, nb, st));
+    if (ndyn > 0)
+        hipLaunchKernelGGL(k_row_fill, dim3(grid1(c, ndyn)), dim3(kBlock), 0, st, D, c.st_off.p, c.row_cur.p,
+                           reinterpret_cast<int *>(c.row_tmp.p));
+    hipLaunchKernelGGL(k_row_place, dim3(grid1(c, 8LL * nb)), dim3(kBlock), 0, st, D, c.st_off.p, c.st_idx.p,
+                       c.row_cur.p, reinterpret_cast<const int *>(c.row_tmp.p), reinterpret_cast<int *>(c.row_idx.p));
     MDY_HIP(hipGetLastError());
     // evaluation scratch sized for the new slot count
     MDY_TRY(ensure(c.contrib, (size_t)3 * D.n_slots + 3));

@@ -424,7 +424,8 @@ def minimize_batch(ctxs, params, d_coords, d_forces=None, threads_per_block=64, 
     """Batched minimization (mdy_minimize_batch): ctxs[i] holds network i with
     its neighbor lists; d_coords[i] its device coordinates (updated in place).
     params: one CGParams / ConjugateGradientParams for all, or one per
-    network. weights (optional): block shares. first_pass_calls > 0: passes
+    network. threads_per_block: the smallest block the launch may use (it takes
+    larger ones while every network gets a block; same results). weights (optional): block shares. first_pass_calls > 0: passes
     with force-call caps growing 4x; a capped network is suspended and resumed
     on more blocks. first_pass_calls = -k: passes end by completions (once
     max(1, m / k) of a pass's m networks have finished, the others are
