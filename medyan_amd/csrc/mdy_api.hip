@@ -40,7 +40,7 @@ Dev Ctx::dev() const {
     D.slot_ev = D.slot_bp + 3 * n_bp;
     D.slot_bd = D.slot_ev + 4 * D.n_ev;
     D.n_slots = D.slot_bd + D.n_bd;
-    D.row_off = row_off4.p; D.row_idx = row_idx.p;
+    D.row = row.p; D.row_idx = row_idx.p;
     D.coplanar_mode = opts.coplanar_mode;
     D.evq = nullptr;   // set by the one-shot launchers in quadrature mode
     D.cq = std::cos(0.5 * M_PI);   // BranchingPositionCosine.cpp:235, 372 (posheta = pi/2)
@@ -137,7 +137,7 @@ int mdy_create(mdy_ctx **out, int device, const mdy_opts *opts) {
     c.num_cu = prop.multiProcessorCount;
     if (!prop.cooperativeLaunch) { delete ctx; return MDY_ERR_LAUNCH; }
     if (hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking) != hipSuccess) { delete ctx; return MDY_ERR_HIP; }
-    if (ensure(c.qn, 16) || ensure(c.err, 4) || ensure(c.out, 16) || ensure(c.bbox, 8) || ensure(c.qe, 3 * kQueueCap) ||
+    if (ensure(c.qn, 16) || ensure(c.err, 4) || ensure(c.out, 16) || ensure(c.qe, 3 * kQueueCap) ||
         ensure(c.qf, 3 * kQueueCap) || ensure(c.qe_u, 3 * kQueueCap) || ensure(c.red, (size_t)kRed * c.num_cu * 64) ||
         ensure(c.simpson_part, (size_t)kRed * c.num_cu * 8)) {
         mdy_destroy(ctx);
@@ -167,11 +167,11 @@ void mdy_destroy(mdy_ctx *ctx) {
     release(c.c_type); release(c.c_eq); release(c.c_ek); release(c.c_minus); release(c.c_plus);
     release(c.c_mon); release(c.c_seg); release(c.ev_cyl);
     release(c.planes); release(c.plane_k); release(c.plane_sl);
-    release(c.mid); release(c.cell_of); release(c.cell_cnt); release(c.cell_off); release(c.cell_cur);
-    release(c.cell_list); release(c.row_cnt); release(c.row_keep); release(c.row_off); release(c.row_keep_off);
+    release(c.mid); release(c.cell_cnt); release(c.cell_range); release(c.near); release(c.cell_rank);
+    release(c.cell_list); release(c.row_cnt); release(c.row_off); release(c.pair_tmp); release(c.nl_out);
     release(c.pairs); release(c.ev_bs); release(c.ev_kr); release(c.bd_flag); release(c.bd_off); release(c.bd_bead);
-    release(c.bd_plane); release(c.bd_k); release(c.bd_sl); release(c.row_cnt4); release(c.row_off4);
-    release(c.row_cur); release(c.row_idx); release(c.row_tmp); release(c.scan_tmp); release(c.bbox); release(c.x); release(c.xt); release(c.f);
+    release(c.bd_plane); release(c.bd_k); release(c.bd_sl); release(c.row);
+    release(c.row_cur); release(c.row_idx); release(c.row_tmp); release(c.scan_tmp); release(c.x); release(c.xt); release(c.f);
     release(c.batch_args); release(c.batch_map); release(c.batch_done); release(c.evq); release(c.qpan); release(c.qcnt); release(c.qoff);
     release(c.qmap); release(c.qpart); release(c.qpe); release(c.qtot);
     release(c.contrib); release(c.red); release(c.out); release(c.qe); release(c.qf); release(c.qn); release(c.err);

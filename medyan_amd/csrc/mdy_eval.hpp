@@ -489,9 +489,10 @@ constexpr int kRowGroups = 4;
 template <class S>
 __device__ __forceinline__ double gather_coord(const Dev &D, const S *__restrict__ contrib, int o) {
     const int b = o / 3, c = o - 3 * b;
-    const int g1 = D.row_off[b + 1];
+    const int2 r = D.row[b];
+    const int g1 = r.y;
     double f = 0.0;
-    for (int g = D.row_off[b]; g < g1; g += kRowGroups) {
+    for (int g = r.x; g < g1; g += kRowGroups) {
         int4 id[kRowGroups];
         const int none = 3 * D.n_slots;
 #pragma unroll

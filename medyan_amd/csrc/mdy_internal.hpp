@@ -39,8 +39,8 @@ struct Dev {
     const int *bd_bead; const int *bd_plane; const double *bd_k, *bd_sl; const double *planes;
     int slot_fs, slot_fb, slot_lm, slot_bs, slot_bb, slot_bdh, slot_bp, slot_ev, slot_bd, n_slots;
     // bead -> its slots in slot order, as offsets 3 * slot in groups of four (the last one filled
-    // up with 3 * n_slots): bead b's groups are row_off[b] .. row_off[b + 1] - 1
-    const int *row_off; const int4 *row_idx;
+    // up with 3 * n_slots): bead b's groups are row[b].x .. row[b].y - 1
+    const int2 *row; const int4 *row_idx;
     int coplanar_mode;
     const unsigned char *evq;     // quadrature mode: per excluded-volume pair, 1 = evaluated by quadrature
     double cq, sq;                // cos and sin of pi/2 (C library), branching position
@@ -94,23 +94,23 @@ struct Ctx {
     int n_planes = 0;
     DBuf<double> planes, plane_k, plane_sl;
     // neighbor-list work
-    DBuf<double> mid;             // 3 * ncyl
-    DBuf<int> cell_of, cell_cnt, cell_off, cell_cur, cell_list;
-    DBuf<int> row_cnt, row_keep, row_off, row_keep_off;
-    DBuf<int> pairs;              // 2 * npairs (NL, before mother-daughter filtering)
+    DBuf<double> mid;       // 3 * ncyl: midpoints
+    DBuf<int> cell_cnt, cell_rank, near; DBuf<int2> cell_range; DBuf<int4> cell_list;
+    DBuf<unsigned long long> row_cnt, row_off;   // per cylinder: pairs << 32 | kept pairs
+    DBuf<int> pairs, pair_tmp;    // 2 * npairs (NL, before mother-daughter filtering); npairs
+    DBuf<long long> nl_out;       // totals for the host
     long long n_pairs = 0;
     DBuf<int4> ev_bs; DBuf<double> ev_kr; int n_ev = 0;
     DBuf<int2> ev_cyl;            // monomer-sum form: cylinders of each pair
     DBuf<int> bd_flag, bd_off, bd_bead, bd_plane; DBuf<double> bd_k, bd_sl; int n_bd = 0;
     std::vector<int> h_bd_nneigh;
-    DBuf<int> row_cnt4, row_off4, row_cur; DBuf<int4> row_idx, row_tmp;   // bead -> all slots (Dev::row_idx)
+    DBuf<int> row_cur; DBuf<int2> row; DBuf<int4> row_idx, row_tmp;   // bead -> all slots (Dev::row_idx)
     int n_static = 0;             // entries of st_idx
     DBuf<unsigned char> evq;      // quadrature mode: per-pair flags of the current evaluation
     DBuf<int> qpan, qcnt, qoff, qmap; // quadrature mode: panels, chunk counts, first chunks, chunk -> pair
     DBuf<int> qtot;               // quadrature mode: running chunk total (zero between calls)
     DBuf<double> qpart, qpe;      // quadrature mode: chunk records, per-pair values
     DBuf<int> scan_tmp;
-    DBuf<double> bbox;            // 6
     // evaluation scratch
     DBuf<double> x, xt, f, contrib;
     DBuf<double> red;             // per-block partials

@@ -13,7 +13,6 @@ size_t noalloc_scratch_bytes();
 int launch_energy_noalloc(Ctx &c, const double *d_x, double *d_out, hipStream_t st);
 // mdy_nl.hip
 int build_neighbors(Ctx &c, const double *d_x);
-int exclusive_scan(Ctx &c, const int *in, int *out, int n, hipStream_t st);  // out has n+1 entries
 // mdy_cg.hip
 int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_out, mdy_min_result *res);
 // CGMethod::searchDir after the context's last minimization, to host memory (3 n_beads doubles)

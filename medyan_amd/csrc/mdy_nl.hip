@@ -20,60 +20,81 @@
 
 namespace mdy {
 
-__global__ void k_fill_int(int *p, int n, int v) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
-
-__global__ void __launch_bounds__(kBlock) k_mid_bbox(int ncyl, const int *b1, const int *b2, const double *x,
-                                                     double *mid, double *red) {
-    __shared__ double lds[17 * 6];
-    double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncyl; c += gridDim.x * blockDim.x) {
-        const double *p1 = x + b1[c], *p2 = x + b2[c];
-        for (int k = 0; k < 3; k++) {
-            double m = 0.5 * (p1[k] + p2[k]);   // Cylinder::updateCoordinate (Cylinder.cpp:45-49)
-            mid[3 * c + k] = m;
-            v[k] = fmin(v[k], m);
-            v[3 + k] = fmax(v[3 + k], m);
-        }
+// start of the n entries that this thread takes from *total, one atomic per
+// block of 1024 threads (same-address atomics are served every 11 ns: one per
+// wave took 95 us at 200k cylinders). Every thread of the block calls it.
+constexpr int kRoomBlock = 1024;
+__device__ __forceinline__ int block_room(int n, int *total) {
+    __shared__ int part[kRoomBlock / 64], base;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
     }
-    block_reduce<6>(v, lds, 0x38u, 0x07u);
-    if (threadIdx.x < 6) red[(size_t)blockIdx.x * kRed + threadIdx.x] = v[threadIdx.x];
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int s = 0;
+        for (int w = 0; w < kRoomBlock / 64; w++) { const int v = part[w]; part[w] = s; s += v; }
+        base = s ? atomicAdd(total, s) : 0;
+    }
+    __syncthreads();
+    return base + part[wave] + incl - n;
 }
 
-__global__ void __launch_bounds__(kBlock) k_bbox_final(const double *red, int nblk, double *bbox) {
-    __shared__ double lds[17 * 6];
-    double v[6];
-    grid_partials_reduce<6>(red, nblk, v, lds, 0x38u, 0x07u);
-    if (threadIdx.x < 6) bbox[threadIdx.x] = v[threadIdx.x];
-}
-
-struct Grid {
-    double ox, oy, oz, h;
-    int nx, ny, nz;
-    __device__ __forceinline__ int clampi(int v, int n) const { return v < 0 ? 0 : (v >= n ? n - 1 : v); }
-    __device__ __forceinline__ void cell3(const double *m, int &cx, int &cy, int &cz) const {
-        cx = clampi((int)floor((m[0] - ox) / h), nx);
-        cy = clampi((int)floor((m[1] - oy) / h), ny);
-        cz = clampi((int)floor((m[2] - oz) / h), nz);
+// Cells of edge h in a hash table of nb = 2^k buckets, at least two per
+// cylinder: no bounding box, so the host does not wait for one, and the table
+// does not grow with the box. A bucket's cylinders are contiguous in `list`
+// with their cells; a reader skips those of other cells in the same bucket.
+// Cells that follow one another in x have neighbouring buckets: the 27 around a
+// cylinder lie in nine lines instead of 27.
+struct Cells {
+    double h;
+    unsigned mask;
+    __device__ __forceinline__ int3 cell(const double *m) const {
+        return make_int3((int)floor(m[0] / h), (int)floor(m[1] / h), (int)floor(m[2] / h));   // saturates
+    }
+    __device__ __forceinline__ unsigned bucket(int3 c) const {
+        const unsigned u = ((unsigned)c.y * 0x9E3779B1u) ^ ((unsigned)c.z * 0x85EBCA6Bu);
+        return ((u ^ (u >> 15)) * 0xC2B2AE35u + (unsigned)c.x) & mask;
     }
 };
 
-__global__ void k_cell_assign(int ncyl, const double *mid, Grid g, int *cell_of, int *cell_cnt) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncyl; c += gridDim.x * blockDim.x) {
-        int cx, cy, cz;
-        g.cell3(mid + 3 * c, cx, cy, cz);
-        int cell = (cz * g.ny + cy) * g.nx + cx;
-        cell_of[c] = cell;
-        atomicAdd(cell_cnt + cell, 1);
-    }
+__global__ void k_nl_zero(int *a, int na, int *b, int nb) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < na + nb; i += gridDim.x * blockDim.x)
+        if (i < na) a[i] = 0;
+        else b[i - na] = 0;
 }
 
-__global__ void k_cell_fill(int ncyl, const int *cell_of, const int *cell_off, int *cell_cur, int *cell_list) {
+// flags[0]: an infinite midpoint; flags[1..3]: a number on that axis (plain
+// stores of 1: nothing to order, no atomics on one word)
+__global__ void __launch_bounds__(kBlock) k_nl_cells(int ncyl, const int *__restrict__ b1, const int *__restrict__ b2,
+                                                     const double *__restrict__ x, Cells g, double *__restrict__ mid,
+                                                     int *__restrict__ rank, int *cnt, int *flags) {
+    int f = 0;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncyl; c += gridDim.x * blockDim.x) {
-        int cell = cell_of[c];
-        cell_list[cell_off[cell] + atomicAdd(cell_cur + cell, 1)] = c;
+        const double *p1 = x + b1[c], *p2 = x + b2[c];
+        double m[3];
+        for (int k = 0; k < 3; k++) {
+            m[k] = 0.5 * (p1[k] + p2[k]);   // Cylinder::updateCoordinate (Cylinder.cpp:45-49)
+            mid[3 * c + k] = m[k];
+            if (m[k] == m[k]) f |= 2 << k;
+            if (fabs(m[k]) == INFINITY) f |= 1;
+        }
+        rank[c] = atomicAdd(cnt + g.bucket(g.cell(m)), 1);
     }
+    f = wave_or(f);
+    if ((threadIdx.x & 63) < 4 && ((f >> (threadIdx.x & 63)) & 1)) flags[threadIdx.x & 63] = 1;
+}
+
+// a bucket's range, start and end (the buckets' order in the list does not matter)
+__global__ void __launch_bounds__(kRoomBlock) k_nl_ranges(const int *__restrict__ cnt, int2 *__restrict__ range,
+                                                          int *total) {
+    const int i = blockIdx.x * kRoomBlock + threadIdx.x;   // the bucket count is a multiple of the block
+    const int n = cnt[i], at = block_room(n, total);
+    range[i] = make_int2(at, at + n);
 }
 
 struct CylView {
@@ -85,132 +106,257 @@ struct CylView {
     int mon;             // monomer-sum excluded volume
 };
 
+// What the search reads of a cylinder, 64 bytes each, in the order of
+// the buckets: candidates of a bucket are read in full lines.
+struct CellEntry {
+    double m[3];
+    int c, fil;
+    long long id;
+    int pos, child;
+    int3 cell;
+    int pad;
+};
+static_assert(sizeof(CellEntry) == 64, "");
+__device__ __forceinline__ CellEntry cell_entry(const CylView &C, const Cells &g, const double *__restrict__ mid, int c) {
+    CellEntry e;
+    for (int k = 0; k < 3; k++) e.m[k] = mid[3 * c + k];
+    e.c = c; e.fil = C.fil[c]; e.id = C.id[c]; e.pos = C.pos[c]; e.child = C.child[c];
+    e.cell = g.cell(e.m);
+    e.pad = 0;
+    return e;
+}
+
+__global__ void k_nl_fill(int ncyl, CylView C, Cells g, const double *__restrict__ mid, const int *__restrict__ rank,
+                          const int2 *__restrict__ range, CellEntry *__restrict__ list) {
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncyl; c += gridDim.x * blockDim.x) {
+        const CellEntry e = cell_entry(C, g, mid, c);
+        list[range[g.bucket(e.cell)].x + rank[c]] = e;
+    }
+}
+
 // Pairs the excluded-volume force field drops: the integral form skips a
 // neighbour that is the cylinder's branching mother
 // (cin->getBranchingCylinder() == ci, CylinderExclVolume.cpp:85, 116); the
 // monomer-sum form skips mother-daughter pairs in either order
 // (CylinderVolumeMon.hpp:134-136).
-__device__ __forceinline__ bool ev_dropped(const CylView &C, int c, int n) {
-    return C.child[n] == c || (C.mon && C.child[c] == n);
+__device__ __forceinline__ bool ev_dropped(const CylView &C, const CellEntry &c, const CellEntry &n) {
+    return n.child == c.c || (C.mon && c.child == n.c);
 }
 
-// the reference predicate for candidate n of cylinder c
-__device__ __forceinline__ bool nl_pred(const CylView &C, const double *mid, int c, int n, double rminsq,
-                                        double rmaxsq) {
-    if (C.id[c] <= C.id[n]) return false;
-    if (C.fil[c] == C.fil[n]) {
-        int ds = C.pos[c] - C.pos[n];
-        if (ds < 0) ds = -ds;
-        if (ds <= 2) return false;   // ChemParams::minCylinderDistanceSameFilament (SysParams.h:315)
-    }
-    const double *m1 = mid + 3 * c, *m2 = mid + 3 * n;
-    double d2 = (m2[0] - m1[0]) * (m2[0] - m1[0]);
-    d2 += (m2[1] - m1[1]) * (m2[1] - m1[1]);
-    d2 += (m2[2] - m1[2]) * (m2[2] - m1[2]);
-    if (d2 < rminsq || d2 > rmaxsq) return false;
-    return true;
-}
-
+// The candidates of cylinder c that pass the reference predicate, found by the
+// kGroup lanes of a group, each looking into its share of the 27 cells around
+// c. fn(n) is called by the lane that finds n. One lane per cylinder followed
+// 27 cells' dependent loads in a row (113 us at 40k cylinders for the count).
+constexpr int kGroup = 16;
 template <class F>
-__device__ __forceinline__ void for_candidates(const Grid &g, const double *mid, const int *cell_off,
-                                               const int *cell_list, int c, F &&fn) {
-    int cx, cy, cz;
-    g.cell3(mid + 3 * c, cx, cy, cz);
-    for (int dz = -1; dz <= 1; dz++) {
-        int z = cz + dz;
-        if (z < 0 || z >= g.nz) continue;
-        for (int dy = -1; dy <= 1; dy++) {
-            int y = cy + dy;
-            if (y < 0 || y >= g.ny) continue;
-            for (int dx = -1; dx <= 1; dx++) {
-                int xx = cx + dx;
-                if (xx < 0 || xx >= g.nx) continue;
-                int cell = (z * g.ny + y) * g.nx + xx;
-                for (int k = cell_off[cell], e = cell_off[cell + 1]; k < e; k++) fn(cell_list[k]);
+__device__ __forceinline__ void for_neighbors(const Cells &g, const int2 *__restrict__ range,
+                                              const CellEntry *__restrict__ list, const CellEntry &me, double rminsq,
+                                              double rmaxsq, F &&fn) {
+    constexpr int kCells = (27 + kGroup - 1) / kGroup;   // cells per lane
+    int3 cell[kCells];
+    int2 r[kCells];
+#pragma unroll
+    for (int j = 0; j < kCells; j++) {   // every range is on its way before the first is used
+        const int k = (int)(threadIdx.x & (kGroup - 1)) + j * kGroup;
+        cell[j] = make_int3(me.cell.x + k % 3 - 1, me.cell.y + (k / 3) % 3 - 1, me.cell.z + k / 9 - 1);
+        r[j] = k < 27 ? range[g.bucket(cell[j])] : make_int2(0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < kCells; j++) {
+        for (int a = r[j].x; a < r[j].y; a++) {
+            const CellEntry &n = list[a];
+            double d2 = (n.m[0] - me.m[0]) * (n.m[0] - me.m[0]);
+            d2 += (n.m[1] - me.m[1]) * (n.m[1] - me.m[1]);
+            d2 += (n.m[2] - me.m[2]) * (n.m[2] - me.m[2]);
+            if (d2 < rminsq || d2 > rmaxsq) continue;
+            if (n.cell.x != cell[j].x || n.cell.y != cell[j].y || n.cell.z != cell[j].z) continue;
+            if (me.id <= n.id) continue;
+            if (me.fil == n.fil) {
+                const int ds = me.pos - n.pos;
+                if ((ds < 0 ? -ds : ds) <= 2) continue;   // ChemParams::minCylinderDistanceSameFilament (SysParams.h:315)
             }
+            fn(n);
         }
     }
 }
 
-__global__ void k_pair_count(int ncyl, CylView C, const double *mid, Grid g, const int *cell_off,
-                             const int *cell_list, double rminsq, double rmaxsq, int *row_cnt, int *row_keep) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncyl; c += gridDim.x * blockDim.x) {
-        int cnt = 0, keep = 0;
-        for_candidates(g, mid, cell_off, cell_list, c, [&](int n) {
-            if (!nl_pred(C, mid, c, n, rminsq, rmaxsq)) return;
-            cnt++;
-            if (!ev_dropped(C, c, n)) keep++;
+// Row counts, pairs in the upper and kept pairs in the lower half (row[ncyl] =
+// 0), and the first kNear neighbours found (2 n, + 1 if dropped) in any order.
+// Cylinders are taken in the order of the cells' list, so that the groups of a
+// block share their cells' lines: 77 us at 200k cylinders (105 in cylinder
+// order with every field from its own array), bound by the reads of the buckets.
+constexpr int kNear = kGroup;
+__global__ void __launch_bounds__(kBlock) k_pair_count(int ncyl, CylView C, Cells g, const int2 *range,
+                                                       const CellEntry *list, double rminsq, double rmaxsq,
+                                                       unsigned long long *row, int *near) {
+    __shared__ int found[kBlock / kGroup];
+    const int i = blockIdx.x * (kBlock / kGroup) + threadIdx.x / kGroup, lane = threadIdx.x & (kGroup - 1);
+    const int grp = threadIdx.x / kGroup;
+    if (lane == 0) found[grp] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // the group's lanes are one wave's
+    __builtin_amdgcn_wave_barrier();
+    if (i < ncyl) {
+        const CellEntry me = list[i];
+        const int c = me.c;
+        int keep = 0;
+        for_neighbors(g, range, list, me, rminsq, rmaxsq, [&](const CellEntry &n) {
+            const int drop = ev_dropped(C, me, n) ? 1 : 0, at = atomicAdd(found + grp, 1);
+            if (at < kNear) near[(size_t)kNear * c + at] = 2 * n.c + drop;
+            keep += 1 - drop;
         });
-        row_cnt[c] = cnt;
-        row_keep[c] = keep;
+#pragma unroll
+        for (int o = 1; o < kGroup; o <<= 1) keep += __shfl_xor(keep, o, kGroup);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) row[c] = ((unsigned long long)(unsigned)found[grp] << 32) | (unsigned)keep;
+    } else if (i == ncyl && lane == 0) {
+        row[i] = 0;
     }
 }
 
-__global__ void k_pair_emit(int ncyl, CylView C, const double *mid, Grid g, const int *cell_off,
-                            const int *cell_list, double rminsq, double rmaxsq, const int *row_off,
-                            const int *row_keep_off, int2 *pairs, int4 *ev_bs, double *ev_kr, int2 *ev_cyl) {
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncyl; c += gridDim.x * blockDim.x) {
-        int2 *row = pairs + row_off[c];
-        int len = 0;
-        for_candidates(g, mid, cell_off, cell_list, c, [&](int n) {
-            if (!nl_pred(C, mid, c, n, rminsq, rmaxsq)) return;
-            row[len++] = make_int2(c, n);
-        });
-        for (int a = 1; a < len; a++) {  // insertion sort by neighbour index
-            int2 v = row[a];
-            int b = a - 1;
-            while (b >= 0 && row[b].y > v.y) { row[b + 1] = row[b]; b--; }
-            row[b + 1] = v;
+// The rows: each entry placed by counting the smaller ones of its row. Rows of
+// up to kNear come from the count; the longer ones are searched again, into
+// tmp. beads: slots per bead so far. 23 us at 200k cylinders; 93
+// with every row searched again.
+__global__ void __launch_bounds__(kBlock) k_pair_emit(int ncyl, CylView C, Cells g, const double *mid, const int2 *range,
+                                                      const CellEntry *list, double rminsq, double rmaxsq,
+                                                      const unsigned long long *row_off, const int *near,
+                                                      int *tmp, int2 *pairs, int4 *ev_bs, double *ev_kr, int2 *ev_cyl,
+                                                      int *beads) {
+    __shared__ int found[kBlock / kGroup];
+    const int q = threadIdx.x & (kGroup - 1), grp = threadIdx.x / kGroup;
+    const int c = blockIdx.x * (kBlock / kGroup) + grp;
+    if (c < ncyl) {
+        const unsigned long long r0 = row_off[c], r1 = row_off[c + 1];
+        const int o = (int)(r0 >> 32), len = (int)(r1 >> 32) - o, ok = (int)(unsigned)r0;
+        const int *keys = near + (size_t)kNear * c;
+        if (len > kNear) {
+            if (q == 0) found[grp] = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // the group's lanes are one wave's
+            __builtin_amdgcn_wave_barrier();
+            const CellEntry me = cell_entry(C, g, mid, c);
+            for_neighbors(g, range, list, me, rminsq, rmaxsq, [&](const CellEntry &n) {
+                tmp[o + atomicAdd(found + grp, 1)] = 2 * n.c + (ev_dropped(C, me, n) ? 1 : 0);
+            });
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            keys = tmp + o;
         }
-        int o = row_keep_off[c];
-        for (int a = 0; a < len; a++) {
-            int n = row[a].y;
-            if (ev_dropped(C, c, n)) continue;
-            ev_bs[o] = make_int4(C.b1[c], C.b2[c], C.b1[n], C.b2[n]);
+        for (int e = q; e < len; e += kGroup) {
+            const int key = keys[e];
+            int rank = 0, krank = 0;
+            for (int m = 0; m < len; m++) {
+                const int k = keys[m];
+                if (k < key) { rank++; krank += 1 - (k & 1); }
+            }
+            const int n = key >> 1;
+            pairs[o + rank] = make_int2(c, n);
+            if (key & 1) continue;
+            const int4 bs = make_int4(C.b1[c], C.b2[c], C.b1[n], C.b2[n]);
+            const int at = ok + krank;
+            ev_bs[at] = bs;
             if (C.mon) {
                 // kvol = max of the two constants; coeff = kvol * segEqLen1 * segEqLen2
                 // (CylinderVolumeMon.hpp:43, 160-163)
-                ev_kr[o] = smax(C.ek[c], C.ek[n]) * C.seg[c] * C.seg[n];
-                ev_cyl[o] = make_int2(c, n);
+                ev_kr[at] = smax(C.ek[c], C.ek[n]) * C.seg[c] * C.seg[n];
+                ev_cyl[at] = make_int2(c, n);
             } else {
-                double krep = (C.type[c] != C.type[n]) ? smax(C.ek[c], C.ek[n]) : C.ek[c];
-                ev_kr[o] = krep * C.eq[c] * C.eq[n];
+                const double krep = (C.type[c] != C.type[n]) ? smax(C.ek[c], C.ek[n]) : C.ek[c];
+                ev_kr[at] = krep * C.eq[c] * C.eq[n];
             }
-            o++;
+            atomicAdd(beads + bs.x / 3, 1); atomicAdd(beads + bs.y / 3, 1);
+            atomicAdd(beads + bs.z / 3, 1); atomicAdd(beads + bs.w / 3, 1);
         }
     }
 }
 
 // BoundaryCylinderNL (NeighborListImpl.cpp:738-751): plane distance of
 // Cylinder::coordinate = midPointCoordinate(b1, b2, 0.5) below the float cutoff.
-__global__ void k_bd_flag(int ncyl, int np, const int *b1, const int *b2, const unsigned char *minus,
-                          const double *x, const double *planes, float cutoff, int *flag) {
-    const long long tot = (long long)np * ncyl;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < tot;
-         i += (long long)gridDim.x * blockDim.x) {
-        int p = (int)(i / ncyl), c = (int)(i % ncyl);
+// One block per plane and kBlock cylinders; cnt: its terms (two for a minus end).
+__global__ void __launch_bounds__(kBlock) k_bd_flag(int ncyl, int nchunk, const int *__restrict__ b1,
+                                                    const int *__restrict__ b2, const unsigned char *__restrict__ minus,
+                                                    const double *__restrict__ x, const double *__restrict__ planes,
+                                                    float cutoff, int *__restrict__ flag, int *__restrict__ cnt) {
+    __shared__ int part[kBlock / 64];
+    const int p = blockIdx.x / nchunk, c = (blockIdx.x % nchunk) * kBlock + threadIdx.x;
+    int f = 0;
+    if (c < ncyl) {
         const double *p1 = x + b1[c], *p2 = x + b2[c];
         d3 m = d3{p1[0] * (1.0 - 0.5) + 0.5 * p2[0], p1[1] * (1.0 - 0.5) + 0.5 * p2[1],
                   p1[2] * (1.0 - 0.5) + 0.5 * p2[2]};
-        double dist = plane_dist(planes + 4 * p, m);
-        flag[i] = (dist < (double)cutoff) ? (minus[c] ? 2 : 1) : 0;
+        const double dist = plane_dist(planes + 4 * p, m);
+        f = (dist < (double)cutoff) ? (minus[c] ? 2 : 1) : 0;
+        flag[(size_t)p * ncyl + c] = f;
+    }
+    const int n = __popcll(__ballot(f > 0)) + __popcll(__ballot(f > 1));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+        for (int w = 0; w < kBlock / 64; w++) t += part[w];
+        cnt[blockIdx.x] = t;
     }
 }
 
-// BoundaryCylinderRepulsion::vectorize (BoundaryCylinderRepulsion.cpp:33-88)
-__global__ void k_bd_emit(int ncyl, int np, const int *b1, const int *b2, const int *flag, const int *off,
-                          const double *pk, const double *psl, int *bd_bead, int *bd_plane, double *bd_k,
-                          double *bd_sl) {
-    const long long tot = (long long)np * ncyl;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < tot;
-         i += (long long)gridDim.x * blockDim.x) {
-        int f = flag[i];
-        if (!f) continue;
-        int p = (int)(i / ncyl), c = (int)(i % ncyl);
-        int o = off[i];
-        if (f == 2) { bd_bead[o] = b1[c]; bd_plane[o] = p; bd_k[o] = pk[p]; bd_sl[o] = psl[p]; o++; }
-        bd_bead[o] = b2[c]; bd_plane[o] = p; bd_k[o] = pk[p]; bd_sl[o] = psl[p];
+// One block: the chunks' offsets, in place, and what the host needs to size the
+// tables: out = pair totals (packed as in row), midpoints fit for cells, then the offset
+// of each plane's first term and their total.
+__global__ void __launch_bounds__(1024) k_nl_totals(int nplanes, int nchunk, int *cnt, const unsigned long long *pairs,
+                                                    const int *flags, long long *out) {
+    __shared__ int part[16];
+    const int n = nplanes * nchunk, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int run = 0;
+    if (threadIdx.x == 0) {
+        out[0] = pairs ? (long long)*pairs : 0;
+        out[1] = flags ? (!flags[0] && flags[1] && flags[2] && flags[3] ? 1 : 0) : 1;
     }
+    for (int i0 = 0; i0 < n; i0 += 1024) {
+        const int i = i0 + threadIdx.x;
+        const int v = i < n ? cnt[i] : 0;
+        int incl = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += u;
+        }
+        if (lane == 63) part[wave] = incl;
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < 16; w++) { before += w < wave ? part[w] : 0; all += part[w]; }
+        const int at = run + before + incl - v;
+        if (i < n) {
+            cnt[i] = at;
+            if (i % nchunk == 0) out[2 + i / nchunk] = at;
+        }
+        run += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[2 + nplanes] = run;
+}
+
+// BoundaryCylinderRepulsion::vectorize (BoundaryCylinderRepulsion.cpp:33-88)
+__global__ void __launch_bounds__(kBlock) k_bd_emit(int ncyl, int nchunk, const int *__restrict__ b1,
+                                                    const int *__restrict__ b2, const int *__restrict__ flag,
+                                                    const int *__restrict__ off, const double *__restrict__ pk,
+                                                    const double *__restrict__ psl, int *bd_bead, int *bd_plane,
+                                                    double *bd_k, double *bd_sl, int *beads) {
+    __shared__ int part[kBlock / 64];
+    const int p = blockIdx.x / nchunk, c = (blockIdx.x % nchunk) * kBlock + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int f = c < ncyl ? flag[(size_t)p * ncyl + c] : 0;
+    const unsigned long long one = __ballot(f > 0), two = __ballot(f > 1), below = (1ull << lane) - 1;
+    if (lane == 0) part[wave] = __popcll(one) + __popcll(two);
+    __syncthreads();
+    if (!f) return;
+    int o = off[blockIdx.x] + __popcll(one & below) + __popcll(two & below);
+    for (int w = 0; w < wave; w++) o += part[w];
+    auto put = [&](int bead) {
+        bd_bead[o] = bead; bd_plane[o] = p; bd_k[o] = pk[p]; bd_sl[o] = psl[p];
+        atomicAdd(beads + bead / 3, 1);
+        o++;
+    };
+    if (f == 2) put(b1[c]);
+    put(b2[c]);
 }
 
 // The gather's rows (Dev::row_idx): a bead's bonded slots, then its
@@ -225,18 +371,16 @@ __device__ __forceinline__ int dyn_slot_bead(const Dev &D, int j, int &slot) {
     slot = D.slot_bd + j;
     return D.bd_bead[j] / 3;
 }
-__global__ void k_row_count(Dev D, int *cur) {
-    const int tot = 4 * D.n_ev + D.n_bd;
-    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < tot; j += gridDim.x * blockDim.x) {
-        int s;
-        atomicAdd(cur + dyn_slot_bead(D, j, s), 1);
-    }
-}
-// groups of four per row; the counters restart for the fill
-__global__ void k_row_groups(int nb, const int *__restrict__ st_off, int *cur, int *cnt4) {
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b <= nb; b += gridDim.x * blockDim.x) {
-        cnt4[b] = b < nb ? (st_off[b + 1] - st_off[b] + cur[b] + 3) / 4 : 0;
-        if (b < nb) cur[b] = 0;
+// room for the rows, in groups of four (their order does not matter); the
+// counters restart for the fill
+__global__ void __launch_bounds__(kRoomBlock) k_row_ranges(int nb, const int *__restrict__ st_off, int *__restrict__ cur,
+                                                       int2 *__restrict__ row, int *total) {
+    const int b = blockIdx.x * kRoomBlock + threadIdx.x;
+    const int n = b < nb ? (st_off[b + 1] - st_off[b] + cur[b] + 3) / 4 : 0;
+    const int base = block_room(n, total);
+    if (b < nb) {
+        row[b] = make_int2(base, base + n);
+        cur[b] = 0;
     }
 }
 // dynamic slots in any order, after the room of the bonded ones
@@ -245,7 +389,7 @@ __global__ void k_row_fill(Dev D, const int *__restrict__ st_off, int *cur, int 
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < tot; j += gridDim.x * blockDim.x) {
         int s;
         const int b = dyn_slot_bead(D, j, s);
-        tmp[4 * D.row_off[b] + (st_off[b + 1] - st_off[b]) + atomicAdd(cur + b, 1)] = s;
+        tmp[4 * D.row[b].x + (st_off[b + 1] - st_off[b]) + atomicAdd(cur + b, 1)] = s;
     }
 }
 // Eight lanes per bead: the bonded slots copied, each dynamic slot placed by
@@ -256,7 +400,7 @@ __global__ void k_row_place(Dev D, const int *__restrict__ st_off, const int *__
     const int q = threadIdx.x & 7;
     for (int b = (blockIdx.x * blockDim.x + threadIdx.x) >> 3; b < D.nb; b += (gridDim.x * blockDim.x) >> 3) {
         const int s0 = st_off[b], ns = st_off[b + 1] - s0, nd = cur[b];
-        const int r0 = 4 * D.row_off[b], r1 = 4 * D.row_off[b + 1];
+        const int r0 = 4 * D.row[b].x, r1 = 4 * D.row[b].y;
         for (int k = q; k < ns; k += 8) out[r0 + k] = 3 * st_idx[s0 + k];
         const int *row = tmp + r0 + ns;
         for (int k = q; k < nd; k += 8) {
@@ -276,142 +420,105 @@ static int grid1(const Ctx &c, long long n) {
     return (int)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
-int exclusive_scan(Ctx &c, const int *in, int *out, int n, hipStream_t st) {
-    // out[0..n]: exclusive prefix of in[0..n-1] followed by the total
-    size_t tmp = 0;
-    MDY_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, in, out, n + 1, st));
-    MDY_TRY(ensure(c.scan_tmp, tmp / sizeof(int) + 1));
-    size_t cap = c.scan_tmp.n * sizeof(int);
-    // the (n+1)-th input is read past `in`; callers allocate n+1 entries and zero the last
-    MDY_HIP(hipcub::DeviceScan::ExclusiveSum(c.scan_tmp.p, cap, in, out, n + 1, st));
-    return MDY_OK;
-}
-
 int build_neighbors(Ctx &c, const double *d_x) {
     hipStream_t st = c.stream;
-    const int ncyl = c.ncyl;
+    const int ncyl = c.ncyl, nb = c.nb;
     c.n_ev = 0;
     c.n_bd = 0;
     c.n_pairs = 0;
     CylView C{c.c_b1.p, c.c_b2.p, c.c_fil.p, c.c_pos.p, c.c_child.p, c.c_id.p, c.c_type.p, c.c_eq.p, c.c_ek.p,
               c.c_seg.p, c.ev_mon};
-    if (c.ev_on && ncyl > 1) {
-        MDY_TRY(ensure(c.mid, (size_t)3 * ncyl));
-        const int g = grid1(c, ncyl);
-        MDY_TRY(ensure(c.red, (size_t)kRed * c.num_cu * 64));
-        hipLaunchKernelGGL(k_mid_bbox, dim3(g), dim3(kBlock), 0, st, ncyl, c.c_b1.p, c.c_b2.p, d_x, c.mid.p, c.red.p);
-        hipLaunchKernelGGL(k_bbox_final, dim3(1), dim3(kBlock), 0, st, c.red.p, g, c.bbox.p);
-        double bb[6];
-        MDY_HIP(hipMemcpyAsync(bb, c.bbox.p, sizeof(bb), hipMemcpyDeviceToHost, st));
-        MDY_HIP(hipStreamSynchronize(st));
-        for (int k = 0; k < 6; k++)
-            if (!std::isfinite(bb[k])) return MDY_ERR_NONFINITE;
-        const float rmaxsq_f = c.ev_cut * c.ev_cut;   // float, HybridNeighborListImpl.h:78-80
-        const float rminsq_f = 0.0f * 0.0f;
-        Grid gr;
-        gr.h = std::sqrt((double)rmaxsq_f) * (1.0 + 1e-6) + 1e-6;
-        double ext[3] = {bb[3] - bb[0], bb[4] - bb[1], bb[5] - bb[2]};
-        for (;;) {
-            gr.nx = (int)std::floor(ext[0] / gr.h) + 1;
-            gr.ny = (int)std::floor(ext[1] / gr.h) + 1;
-            gr.nz = (int)std::floor(ext[2] / gr.h) + 1;
-            if ((double)gr.nx * gr.ny * gr.nz <= 4.0e6) break;
-            gr.h *= 1.25;   // larger cells stay correct, just prune less
-        }
-        gr.ox = bb[0]; gr.oy = bb[1]; gr.oz = bb[2];
-        const int ncell = gr.nx * gr.ny * gr.nz;
-        MDY_TRY(ensure(c.cell_of, ncyl));
-        MDY_TRY(ensure(c.cell_cnt, (size_t)ncell + 1));
-        MDY_TRY(ensure(c.cell_cur, (size_t)ncell + 1));
-        MDY_TRY(ensure(c.cell_off, (size_t)ncell + 2));
-        MDY_TRY(ensure(c.cell_list, ncyl));
-        hipLaunchKernelGGL(k_fill_int, dim3(grid1(c, ncell + 1)), dim3(kBlock), 0, st, c.cell_cnt.p, ncell + 1, 0);
-        hipLaunchKernelGGL(k_fill_int, dim3(grid1(c, ncell + 1)), dim3(kBlock), 0, st, c.cell_cur.p, ncell + 1, 0);
-        hipLaunchKernelGGL(k_cell_assign, dim3(g), dim3(kBlock), 0, st, ncyl, c.mid.p, gr, c.cell_of.p, c.cell_cnt.p);
-        MDY_TRY(exclusive_scan(c, c.cell_cnt.p, c.cell_off.p, ncell, st));
-        hipLaunchKernelGGL(k_cell_fill, dim3(g), dim3(kBlock), 0, st, ncyl, c.cell_of.p, c.cell_off.p, c.cell_cur.p,
-                           c.cell_list.p);
-        MDY_TRY(ensure(c.row_cnt, (size_t)ncyl + 1));
-        MDY_TRY(ensure(c.row_keep, (size_t)ncyl + 1));
-        MDY_TRY(ensure(c.row_off, (size_t)ncyl + 2));
-        MDY_TRY(ensure(c.row_keep_off, (size_t)ncyl + 2));
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, c.row_cnt.p + ncyl, 1, 0);
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, c.row_keep.p + ncyl, 1, 0);
-        hipLaunchKernelGGL(k_pair_count, dim3(g), dim3(kBlock), 0, st, ncyl, C, c.mid.p, gr, c.cell_off.p,
-                           c.cell_list.p, (double)rminsq_f, (double)rmaxsq_f, c.row_cnt.p, c.row_keep.p);
-        MDY_TRY(exclusive_scan(c, c.row_cnt.p, c.row_off.p, ncyl, st));
-        MDY_TRY(exclusive_scan(c, c.row_keep.p, c.row_keep_off.p, ncyl, st));
-        int tot[2];
-        MDY_HIP(hipMemcpyAsync(&tot[0], c.row_off.p + ncyl, sizeof(int), hipMemcpyDeviceToHost, st));
-        MDY_HIP(hipMemcpyAsync(&tot[1], c.row_keep_off.p + ncyl, sizeof(int), hipMemcpyDeviceToHost, st));
-        MDY_HIP(hipStreamSynchronize(st));
-        c.n_pairs = tot[0];
-        c.n_ev = tot[1];
-        MDY_TRY(ensure(c.pairs, (size_t)2 * tot[0] + 2));
-        MDY_TRY(ensure(c.ev_bs, (size_t)tot[1] + 1));
-        MDY_TRY(ensure(c.ev_kr, (size_t)tot[1] + 1));
-        if (c.ev_mon) MDY_TRY(ensure(c.ev_cyl, (size_t)tot[1] + 1));
-        hipLaunchKernelGGL(k_pair_emit, dim3(g), dim3(kBlock), 0, st, ncyl, C, c.mid.p, gr, c.cell_off.p,
-                           c.cell_list.p, (double)rminsq_f, (double)rmaxsq_f, c.row_off.p, c.row_keep_off.p,
-                           (int2 *)c.pairs.p, c.ev_bs.p, c.ev_kr.p, c.ev_mon ? c.ev_cyl.p : nullptr);
-        MDY_HIP(hipGetLastError());
-    }
-    if (c.bd_on && c.n_planes > 0 && ncyl > 0) {
-        const long long tot = (long long)c.n_planes * ncyl;
-        MDY_TRY(ensure(c.bd_flag, (size_t)tot + 1));
-        MDY_TRY(ensure(c.bd_off, (size_t)tot + 2));
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, st, c.bd_flag.p + tot, 1, 0);
-        hipLaunchKernelGGL(k_bd_flag, dim3(grid1(c, tot)), dim3(kBlock), 0, st, ncyl, c.n_planes, c.c_b1.p, c.c_b2.p,
-                           c.c_minus.p, d_x, c.planes.p, c.bd_cut, c.bd_flag.p);
-        MDY_TRY(exclusive_scan(c, c.bd_flag.p, c.bd_off.p, (int)tot, st));
-        std::vector<int> offs(c.n_planes + 1);
-        for (int p = 0; p <= c.n_planes; p++)
-            MDY_HIP(hipMemcpyAsync(&offs[p], c.bd_off.p + (size_t)p * ncyl, sizeof(int), hipMemcpyDeviceToHost, st));
-        MDY_HIP(hipStreamSynchronize(st));
-        c.n_bd = offs[c.n_planes];
-        c.h_bd_nneigh.assign(c.n_planes, 0);
-        for (int p = 0; p < c.n_planes; p++) c.h_bd_nneigh[p] = offs[p + 1] - offs[p];
-        MDY_TRY(ensure(c.bd_bead, (size_t)c.n_bd + 1));
-        MDY_TRY(ensure(c.bd_plane, (size_t)c.n_bd + 1));
-        MDY_TRY(ensure(c.bd_k, (size_t)c.n_bd + 1));
-        MDY_TRY(ensure(c.bd_sl, (size_t)c.n_bd + 1));
-        hipLaunchKernelGGL(k_bd_emit, dim3(grid1(c, tot)), dim3(kBlock), 0, st, ncyl, c.n_planes, c.c_b1.p, c.c_b2.p,
-                           c.bd_flag.p, c.bd_off.p, c.plane_k.p, c.plane_sl.p, c.bd_bead.p, c.bd_plane.p, c.bd_k.p,
-                           c.bd_sl.p);
-        MDY_HIP(hipGetLastError());
-    } else {
-        c.h_bd_nneigh.assign(c.n_planes, 0);
-    }
-    // dynamic CSR over the new slots
-    MDY_TRY(ensure(c.ev_bs, 1));
-    MDY_TRY(ensure(c.ev_kr, 1));
-    if (c.ev_mon) MDY_TRY(ensure(c.ev_cyl, 1));
-    MDY_TRY(ensure(c.bd_bead, 1));
-    MDY_TRY(ensure(c.bd_plane, 1));
-    MDY_TRY(ensure(c.bd_k, 1));
-    MDY_TRY(ensure(c.bd_sl, 1));
-    c.have_nl = true;
-    Dev D = c.dev();
-    const int nb = c.nb;
-    const int ndyn = 4 * c.n_ev + c.n_bd;
+    const bool ev = c.ev_on && ncyl > 1, bd = c.bd_on && c.n_planes > 0 && ncyl > 0;
+    // counters that start at zero: bucket counts, then list total, row total, four midpoint flags
+    int nbuckets = 1024;
+    while (nbuckets < 2LL * ncyl && nbuckets < (1 << 29)) nbuckets *= 2;
+    const int nzero = (ev ? nbuckets : 0) + 6;
+    MDY_TRY(ensure(c.cell_cnt, (size_t)nzero));
     MDY_TRY(ensure(c.row_cur, (size_t)nb + 1));
-    MDY_TRY(ensure(c.row_cnt4, (size_t)nb + 1));
-    MDY_TRY(ensure(c.row_off4, (size_t)nb + 2));
+    int *misc = c.cell_cnt.p + (nzero - 6);
+    hipLaunchKernelGGL(k_nl_zero, dim3(grid1(c, (long long)nzero + nb)), dim3(kBlock), 0, st, c.cell_cnt.p, nzero,
+                       c.row_cur.p, nb);
+    const float rmaxsq_f = c.ev_cut * c.ev_cut;   // float, HybridNeighborListImpl.h:78-80
+    const float rminsq_f = 0.0f * 0.0f;
+    const double rmin2 = (double)rminsq_f, rmax2 = (double)rmaxsq_f;
+    const Cells g{std::sqrt(rmax2) * (1.0 + 1e-6) + 1e-6, (unsigned)nbuckets - 1};
+    // a group per cylinder without a cap: each is one chain of dependent loads
+    const dim3 groups((unsigned)(((long long)kGroup * (ncyl + 1) + kBlock - 1) / kBlock)), blk(kBlock);
+    if (ev) {
+        MDY_TRY(ensure(c.mid, (size_t)3 * ncyl));
+        MDY_TRY(ensure(c.cell_rank, ncyl));
+        MDY_TRY(ensure(c.cell_range, nbuckets));
+        MDY_TRY(ensure(c.cell_list, sizeof(CellEntry) / sizeof(int4) * (size_t)ncyl));
+        CellEntry *list = reinterpret_cast<CellEntry *>(c.cell_list.p);
+        MDY_TRY(ensure(c.near, (size_t)kNear * ncyl));
+        MDY_TRY(ensure(c.row_cnt, (size_t)ncyl + 1));
+        MDY_TRY(ensure(c.row_off, (size_t)ncyl + 1));
+        const dim3 cyl(grid1(c, ncyl));
+        hipLaunchKernelGGL(k_nl_cells, cyl, blk, 0, st, ncyl, c.c_b1.p, c.c_b2.p, d_x, g, c.mid.p, c.cell_rank.p,
+                           c.cell_cnt.p, misc + 2);
+        hipLaunchKernelGGL(k_nl_ranges, dim3(nbuckets / kRoomBlock), dim3(kRoomBlock), 0, st, c.cell_cnt.p,
+                           c.cell_range.p, misc);
+        hipLaunchKernelGGL(k_nl_fill, cyl, blk, 0, st, ncyl, C, g, c.mid.p, c.cell_rank.p, c.cell_range.p, list);
+        hipLaunchKernelGGL(k_pair_count, groups, blk, 0, st, ncyl, C, g, c.cell_range.p, list, rmin2,
+                           rmax2, c.row_cnt.p, c.near.p);
+        size_t tmp = 0;
+        MDY_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, c.row_cnt.p, c.row_off.p, ncyl + 1, st));
+        MDY_TRY(ensure(c.scan_tmp, tmp / sizeof(int) + 1));
+        size_t cap = c.scan_tmp.n * sizeof(int);
+        MDY_HIP(hipcub::DeviceScan::ExclusiveSum(c.scan_tmp.p, cap, c.row_cnt.p, c.row_off.p, ncyl + 1, st));
+    }
+    const int nchunk = (ncyl + kBlock - 1) / kBlock, np = bd ? c.n_planes : 0;
+    if (bd) {
+        MDY_TRY(ensure(c.bd_flag, (size_t)np * ncyl));
+        MDY_TRY(ensure(c.bd_off, (size_t)np * nchunk));
+        hipLaunchKernelGGL(k_bd_flag, dim3(np * nchunk), blk, 0, st, ncyl, nchunk, c.c_b1.p, c.c_b2.p, c.c_minus.p, d_x,
+                           c.planes.p, c.bd_cut, c.bd_flag.p, c.bd_off.p);
+    }
+    MDY_TRY(ensure(c.nl_out, (size_t)c.n_planes + 3));
+    hipLaunchKernelGGL(k_nl_totals, dim3(1), dim3(1024), 0, st, np, nchunk, c.bd_off.p,
+                       ev ? c.row_off.p + ncyl : nullptr, ev ? misc + 2 : nullptr, c.nl_out.p);
+    std::vector<long long> tot((size_t)np + 3);
+    MDY_HIP(hipMemcpyAsync(tot.data(), c.nl_out.p, tot.size() * sizeof(long long), hipMemcpyDeviceToHost, st));
+    MDY_HIP(hipStreamSynchronize(st));
+    if (!tot[1]) return MDY_ERR_NONFINITE;   // an infinite midpoint, or an axis without a number
+    c.n_pairs = (unsigned long long)tot[0] >> 32;
+    c.n_ev = (int)(unsigned)tot[0];
+    c.n_bd = (int)tot[2 + np];
+    c.h_bd_nneigh.assign(c.n_planes, 0);
+    for (int p = 0; p < np; p++) c.h_bd_nneigh[p] = (int)(tot[3 + p] - tot[2 + p]);
+    MDY_TRY(ensure(c.ev_bs, (size_t)c.n_ev + 1));
+    MDY_TRY(ensure(c.ev_kr, (size_t)c.n_ev + 1));
+    if (c.ev_mon) MDY_TRY(ensure(c.ev_cyl, (size_t)c.n_ev + 1));
+    MDY_TRY(ensure(c.bd_bead, (size_t)c.n_bd + 1));
+    MDY_TRY(ensure(c.bd_plane, (size_t)c.n_bd + 1));
+    MDY_TRY(ensure(c.bd_k, (size_t)c.n_bd + 1));
+    MDY_TRY(ensure(c.bd_sl, (size_t)c.n_bd + 1));
+    const int ndyn = 4 * c.n_ev + c.n_bd;
     // every row's last group may be filled up with three entries
-    const size_t groups = ((size_t)c.n_static + ndyn) / 4 + nb + 1;
-    MDY_TRY(ensure(c.row_idx, groups));
-    MDY_TRY(ensure(c.row_tmp, groups));
-    hipLaunchKernelGGL(k_fill_int, dim3(grid1(c, nb + 1)), dim3(kBlock), 0, st, c.row_cur.p, nb + 1, 0);
-    D = c.dev();
-    if (ndyn > 0) hipLaunchKernelGGL(k_row_count, dim3(grid1(c, ndyn)), dim3(kBlock), 0, st, D, c.row_cur.p);
-    hipLaunchKernelGGL(k_row_groups, dim3(grid1(c, nb + 1)), dim3(kBlock), 0, st, nb, c.st_off.p, c.row_cur.p,
-                       c.row_cnt4.p);
-    MDY_TRY(exclusive_scan(c, c.row_cnt4.p, c.row_off4.p, nb, st));
+    const size_t rows = ((size_t)c.n_static + ndyn) / 4 + nb + 1;
+    MDY_TRY(ensure(c.row, (size_t)nb + 1));
+    MDY_TRY(ensure(c.row_idx, rows));
+    MDY_TRY(ensure(c.row_tmp, rows));
+    if (c.n_pairs > 0) {
+        MDY_TRY(ensure(c.pairs, 2 * (size_t)c.n_pairs));
+        MDY_TRY(ensure(c.pair_tmp, (size_t)c.n_pairs));
+        hipLaunchKernelGGL(k_pair_emit, groups, blk, 0, st, ncyl, C, g, c.mid.p, c.cell_range.p,
+                           reinterpret_cast<const CellEntry *>(c.cell_list.p), rmin2, rmax2, c.row_off.p, c.near.p, c.pair_tmp.p, (int2 *)c.pairs.p,
+                           c.ev_bs.p, c.ev_kr.p, c.ev_mon ? c.ev_cyl.p : nullptr, c.row_cur.p);
+    }
+    if (c.n_bd > 0)
+        hipLaunchKernelGGL(k_bd_emit, dim3(np * nchunk), blk, 0, st, ncyl, nchunk, c.c_b1.p, c.c_b2.p, c.bd_flag.p,
+                           c.bd_off.p, c.plane_k.p, c.plane_sl.p, c.bd_bead.p, c.bd_plane.p, c.bd_k.p, c.bd_sl.p,
+                           c.row_cur.p);
+    c.have_nl = true;
+    const Dev D = c.dev();
+    hipLaunchKernelGGL(k_row_ranges, dim3((nb + kRoomBlock - 1) / kRoomBlock), dim3(kRoomBlock), 0, st, nb, c.st_off.p,
+                       c.row_cur.p, c.row.p, misc + 1);
     if (ndyn > 0)
-        hipLaunchKernelGGL(k_row_fill, dim3(grid1(c, ndyn)), dim3(kBlock), 0, st, D, c.st_off.p, c.row_cur.p,
+        hipLaunchKernelGGL(k_row_fill, dim3(grid1(c, ndyn)), blk, 0, st, D, c.st_off.p, c.row_cur.p,
                            reinterpret_cast<int *>(c.row_tmp.p));
-    hipLaunchKernelGGL(k_row_place, dim3(grid1(c, 8LL * nb)), dim3(kBlock), 0, st, D, c.st_off.p, c.st_idx.p,
-                       c.row_cur.p, reinterpret_cast<const int *>(c.row_tmp.p), reinterpret_cast<int *>(c.row_idx.p));
+    hipLaunchKernelGGL(k_row_place, dim3(grid1(c, 8LL * nb)), blk, 0, st, D, c.st_off.p, c.st_idx.p, c.row_cur.p,
+                       reinterpret_cast<const int *>(c.row_tmp.p), reinterpret_cast<int *>(c.row_idx.p));
     MDY_HIP(hipGetLastError());
     // evaluation scratch sized for the new slot count
     MDY_TRY(ensure(c.contrib, (size_t)3 * D.n_slots + 3));
