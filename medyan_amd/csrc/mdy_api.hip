@@ -45,7 +45,7 @@ Dev Ctx::dev() const {
     D.evq = nullptr;   // set by the one-shot launchers in quadrature mode
     D.cq = std::cos(0.5 * M_PI);   // BranchingPositionCosine.cpp:235, 372 (posheta = pi/2)
     D.sq = std::sin(0.5 * M_PI);
-    D.qe = qe.p; D.qe_n = qn.p; D.qf = qf.p; D.qf_n = qn.p + 1; D.err = err.p;
+    D.qe = qe.p; D.qe_n = qn.p + kOneShot; D.qf = qf.p; D.qf_n = qn.p + kOneShot + 1; D.err = err.p;
     return D;
 }
 
@@ -137,14 +137,14 @@ int mdy_create(mdy_ctx **out, int device, const mdy_opts *opts) {
     c.num_cu = prop.multiProcessorCount;
     if (!prop.cooperativeLaunch) { delete ctx; return MDY_ERR_LAUNCH; }
     if (hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking) != hipSuccess) { delete ctx; return MDY_ERR_HIP; }
-    if (ensure(c.qn, 16) || ensure(c.err, 4) || ensure(c.out, 16) || ensure(c.qe, 3 * kQueueCap) ||
+    if (ensure(c.qn, 2 * kOneShot) || ensure(c.err, 4) || ensure(c.out, 16) || ensure(c.qe, 3 * kQueueCap) ||
         ensure(c.qf, 3 * kQueueCap) || ensure(c.qe_u, 3 * kQueueCap) || ensure(c.red, (size_t)kRed * c.num_cu * 64) ||
-        ensure(c.simpson_part, (size_t)kRed * c.num_cu * 8)) {
+        ensure(c.simpson_part, (size_t)kRed * c.num_cu * 8) || ensure_host_out(c, 64) != MDY_OK) {
         mdy_destroy(ctx);
         return MDY_ERR_HIP;
     }
     (void)hipMemsetAsync(c.err.p, 0, 4 * sizeof(int), c.stream);
-    (void)hipMemsetAsync(c.qn.p, 0, 16 * sizeof(int), c.stream);
+    (void)hipMemsetAsync(c.qn.p, 0, 2 * kOneShot * sizeof(int), c.stream);
     if (resolve_noalloc_scratch(device) != MDY_OK) {
         mdy_destroy(ctx);
         return MDY_ERR_HIP;
@@ -168,12 +168,13 @@ void mdy_destroy(mdy_ctx *ctx) {
     release(c.c_mon); release(c.c_seg); release(c.ev_cyl);
     release(c.planes); release(c.plane_k); release(c.plane_sl);
     release(c.mid); release(c.cell_cnt); release(c.cell_range); release(c.near); release(c.cell_rank);
-    release(c.cell_list); release(c.row_cnt); release(c.row_off); release(c.pair_tmp); release(c.nl_out);
+    release(c.cell_list); release(c.row_cnt); release(c.row_off); release(c.pair_tmp);
     release(c.pairs); release(c.ev_bs); release(c.ev_kr); release(c.bd_flag); release(c.bd_off); release(c.bd_bead);
     release(c.bd_plane); release(c.bd_k); release(c.bd_sl); release(c.row);
     release(c.row_cur); release(c.row_idx); release(c.row_tmp); release(c.scan_tmp); release(c.x); release(c.xt); release(c.f);
     release(c.batch_args); release(c.batch_map); release(c.batch_done); release(c.evq); release(c.qpan); release(c.qcnt); release(c.qoff);
     release(c.qmap); release(c.qpart); release(c.qpe); release(c.qtot);
+    if (c.h_out) (void)hipHostFree(c.h_out);
     release(c.contrib); release(c.red); release(c.out); release(c.qe); release(c.qf); release(c.qn); release(c.err);
     release(c.qe_u); release(c.simpson_part); release(c.F0); release(c.F1); release(c.S0); release(c.S1);
     release(c.xmin); release(c.bar); release(c.cg_out); release(c.tr_lam); release(c.tr_e); release(c.tr_mf);
@@ -452,11 +453,9 @@ int mdy_energy_dev(mdy_ctx *ctx, const double *d_coord, double *d_out, void *str
     if (!c.have_sys || !c.have_nl) return fail(ctx, MDY_ERR_STATE, "network / neighbor list missing");
     (void)hipSetDevice(c.device);
     hipStream_t st = stream ? (hipStream_t)stream : c.stream;
-    int rc = launch_energy(c, d_coord, c.out.p, st);
-    if (rc != MDY_OK) return hipfail(ctx, "energy");
     // d_out: MDY_NFF energies then the total (sentinel form)
-    if (hipMemcpyAsync(d_out, c.out.p, sizeof(double) * (MDY_NFF + 1), hipMemcpyDeviceToDevice, st) != hipSuccess)
-        return hipfail(ctx, "energy copy");
+    int rc = launch_energy(c, d_coord, d_out, MDY_NFF + 1, st);
+    if (rc != MDY_OK) return hipfail(ctx, "energy");
     return MDY_OK;
 }
 
@@ -483,14 +482,12 @@ int mdy_energy(mdy_ctx *ctx, const double *coord, double *e_total, double *e_per
     (void)hipSetDevice(c.device);
     if (hipMemcpyAsync(c.xt.p, coord, sizeof(double) * 3 * c.nb, hipMemcpyHostToDevice, c.stream) != hipSuccess)
         return hipfail(ctx, "coord upload");
-    int rc = launch_energy(c, c.xt.p, c.out.p, c.stream);
+    // the last kernel writes to pinned memory: energies, total, total without the sentinel, error word
+    const double *h = reinterpret_cast<const double *>(c.h_out);
+    int rc = launch_energy(c, c.xt.p, reinterpret_cast<double *>(c.h_out), MDY_NFF + 3, c.stream);
     if (rc != MDY_OK) return hipfail(ctx, "energy");
-    double h[MDY_NFF + 2];
-    if (hipMemcpyAsync(h, c.out.p, sizeof(h), hipMemcpyDeviceToHost, c.stream) != hipSuccess ||
-        hipStreamSynchronize(c.stream) != hipSuccess)
-        return hipfail(ctx, "energy readback");
-    int e = 0;
-    (void)hipMemcpy(&e, c.err.p, sizeof(int), hipMemcpyDeviceToHost);
+    if (hipStreamSynchronize(c.stream) != hipSuccess) return hipfail(ctx, "energy readback");
+    const int e = (int)h[MDY_NFF + 2];
     if (e) return fail(ctx, e, "device error during energy");
     if (e_total) *e_total = h[MDY_NFF];
     if (e_per_ff)

@@ -28,39 +28,63 @@ __global__ void __launch_bounds__(kBlock, 3) k_energy(Dev D, P pos, double *red)
     if (threadIdx.x < 8) reinterpret_cast<unsigned long long *>(red)[(size_t)blockIdx.x * kRed + kXsE + threadIdx.x] = w;
 }
 
-// One block per queued pair: 2-D Simpson energy (energyN, 400 x 400 intervals).
+// Pair i's 2-D Simpson energy (energyN, 400 x 400 intervals), by one block.
 template <class P>
-__global__ void __launch_bounds__(kBlock) k_energy_simpson(Dev D, P pos, double *qe_u) {
-    __shared__ long long lds[17 * 8];
-    const int nq = min(*D.qe_n, kQueueCap);
+__device__ __noinline__ void simpson_energy(const Dev &D, const P &pos, int i, long long *lds, double *u) {
     const int N = 400;
-    for (int q = blockIdx.x; q < nq; q += gridDim.x) {
-        const int i = D.qe[q];
-        int4 b = D.ev_bs[i];
-        SimpsonGeo g = simpson_geo(pos(b.x), pos(b.y), pos(b.z), pos(b.w));
-        mdy_xsum X;
-        mdy_xs_zero(&X);
-        if (threadIdx.x == 0) mdy_xs_add(&X, simpson_e_corners(g));
-        for (int node = threadIdx.x; node < (N + 1) * (N + 1); node += blockDim.x)
-            simpson_e_node(g, node / (N + 1), node % (N + 1), N, X);
-        block_reduce_xsum(X, lds);
-        if (threadIdx.x == 0) {
-            const double ds = 1.0 / ((double)N);
-            qe_u[q] = D.ev_kr[i] * (ds * ds / 9.0) * mdy_xs_value(&X);
-        }
-        __syncthreads();
+    int4 b = D.ev_bs[i];
+    SimpsonGeo g = simpson_geo(pos(b.x), pos(b.y), pos(b.z), pos(b.w));
+    mdy_xsum X;
+    mdy_xs_zero(&X);
+    if (threadIdx.x == 0) mdy_xs_add(&X, simpson_e_corners(g));
+    for (int node = threadIdx.x; node < (N + 1) * (N + 1); node += blockDim.x)
+        simpson_e_node(g, node / (N + 1), node % (N + 1), N, X);
+    block_reduce_xsum(X, lds);
+    if (threadIdx.x == 0) {
+        const double ds = 1.0 / ((double)N);
+        *u = D.ev_kr[i] * (ds * ds / 9.0) * mdy_xs_value(&X);
     }
+    __syncthreads();
 }
 
-// out: the kNFF energies, the total (+inf for an invalid pair), and when
-// n_out = kNFF + 2 the total without the sentinel
-__global__ void __launch_bounds__(kBlock) k_energy_final(Dev D, const double *red, int nblk, const double *qe_u,
-                                                         double *out, int n_out) {
-    __shared__ double lds[17 * kNFF + 8];
-    double e[kNFF + 2];
-    energy_epilogue(D, red, nblk, *D.qe_n, D.qe, qe_u, lds, e, true);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < n_out; k++) out[k] = e[k];
+// What follows the sweep: the queued pairs' Simpson energies, a block each, and
+// by the last block to finish (block 0 if none is queued) the totals: the kNFF
+// energies, the total (+inf for an invalid pair), the total without the
+// sentinel, the error word. Leaves the queue count and the ticket at zero, so
+// no launch has to clear them before the next sweep. One kernel where Simpson,
+// totals, a clearing kernel and a copy were four: an energy call takes 20 us
+// at 40k cylinders (40 before) and 37 at 200k (69).
+constexpr int kTailGrid = 64;
+template <class P>
+__global__ void __launch_bounds__(kTailBlock) k_energy_tail(Dev D, P pos, const double *red, int nblk, double *qe_u,
+                                                            int *ticket, double *out, int n_out) {
+    __shared__ long long lds[17 * 8];
+    __shared__ int last;
+    const int nall = *D.qe_n, nq = min(nall, kQueueCap);
+    if (nq == 0) {
+        if (blockIdx.x != 0) return;
+    } else {
+        for (int q = blockIdx.x; q < nq; q += gridDim.x) simpson_energy(D, pos, D.qe[q], lds, qe_u + q);
+        if (threadIdx.x == 0) {
+            __threadfence();
+            last = atomicAdd(ticket, 1) == (int)gridDim.x - 1;
+            __threadfence();
+        }
+        __syncthreads();
+        if (!last) return;
+    }
+    double v[kNFF], e[kNFF + 2];
+    mdy_xsum X;
+    sum_records<true>(red, nblk, v, X);
+    if (threadIdx.x != 0) return;
+    energy_finish(X, v, nq, D.qe, qe_u, e);
+    for (int k = 0; k < kNFF + 2; k++)
+        if (k < n_out) out[k] = e[k];
+    if (n_out > kNFF + 2) out[kNFF + 2] = (double)*D.err;
+    if (nall != 0) {
+        *D.qe_n = 0;
+        *ticket = 0;
+    }
 }
 
 template <bool MIXED, class P, bool QUAD = false>
@@ -134,8 +158,16 @@ __global__ void __launch_bounds__(kBlock) k_force_simpson_final(Dev D, const dou
     }
 }
 
+// queued: null, or where to report the number of queued pairs; with any, the
+// forces wait for the quadrature and a second gather
 template <bool MIXED>
-__global__ void __launch_bounds__(kBlock) k_gather(Dev D, const double *contrib_, double *force, int accumulate) {
+__global__ void __launch_bounds__(kBlock) k_gather(Dev D, const double *contrib_, double *force, int accumulate,
+                                                   long long *queued) {
+    if (queued) {
+        const int nq = *D.qf_n;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *queued = nq;
+        if (nq) return;
+    }
     const auto *contrib = reinterpret_cast<const typename SlotT<MIXED>::T *>(contrib_);
     for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < D.ndof; o += gridDim.x * blockDim.x) {
         const double f = gather_coord(D, contrib, o);
@@ -158,13 +190,28 @@ static int grid_for(const Ctx &c, long long n) {
     return (int)g;
 }
 
-int launch_energy(Ctx &c, const double *d_x, double *d_out, hipStream_t st) {
+int ensure_host_out(Ctx &c, size_t n) {
+    if (n <= c.h_out_n) return MDY_OK;
+    if (c.h_out) (void)hipHostFree(c.h_out);
+    c.h_out = nullptr;
+    c.h_out_n = 0;
+    MDY_HIP(hipHostMalloc(reinterpret_cast<void **>(&c.h_out), n * sizeof(long long), hipHostMallocDefault));
+    c.h_out_n = n;
+    return MDY_OK;
+}
+
+// k_energy: no more blocks than fit at once (three per CU), each with a record
+static int energy_grid(const Ctx &c, long long n) {
+    const int g = grid_for(c, n);
+    return g > 3 * c.num_cu ? 3 * c.num_cu : g;
+}
+
+int launch_energy(Ctx &c, const double *d_x, double *out, int n_out, hipStream_t st) {
     Dev D = c.dev();
-    const int nblk = grid_for(c, D.n_lanes());
+    const int nblk = energy_grid(c, D.n_lanes());
     const bool quad = quad_on(c);
     const int nqb = quad ? quad_blocks(c) : 0;   // the quadrature pairs' block records follow the others
     MDY_TRY(ensure(c.red, (size_t)kRed * (nblk + nqb)));
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, c.qn.p, 4);
     if (quad) {
         MDY_TRY(quad_classify(c, D, d_x, st));
         hipLaunchKernelGGL((k_energy<PosX, true>), dim3(nblk), dim3(kBlock), 0, st, D, PosX{d_x}, c.red.p);
@@ -172,9 +219,8 @@ int launch_energy(Ctx &c, const double *d_x, double *d_out, hipStream_t st) {
     } else {
         hipLaunchKernelGGL(k_energy<PosX>, dim3(nblk), dim3(kBlock), 0, st, D, PosX{d_x}, c.red.p);
     }
-    hipLaunchKernelGGL(k_energy_simpson<PosX>, dim3(64), dim3(kBlock), 0, st, D, PosX{d_x}, c.qe_u.p);
-    hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(kBlock), 0, st, D, c.red.p, nblk + nqb, c.qe_u.p, d_out,
-                       kNFF + 2);
+    hipLaunchKernelGGL(k_energy_tail<PosX>, dim3(kTailGrid), dim3(kTailBlock), 0, st, D, PosX{d_x}, c.red.p, nblk + nqb,
+                       c.qe_u.p, c.qn.p + kOneShot + 4, out, n_out);
     return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
 }
 
@@ -223,7 +269,7 @@ int launch_energy_noalloc(Ctx &c, const double *d_x, double *d_out, hipStream_t 
     }
     if (!sc) return MDY_ERR_STATE;
     Dev D = c.dev();
-    const int nblk = grid_for(c, D.n_lanes());
+    const int nblk = energy_grid(c, D.n_lanes());
     if (nblk > kScratchBlocks) return MDY_ERR_CAPACITY;
     double *red = reinterpret_cast<double *>(sc + kScRed);
     int *qn = reinterpret_cast<int *>(sc + kScQn);
@@ -234,18 +280,17 @@ int launch_energy_noalloc(Ctx &c, const double *d_x, double *d_out, hipStream_t 
     D.err = reinterpret_cast<int *>(sc + kScErr);
     double *qe_u = reinterpret_cast<double *>(sc + kScQeU);
     // the counters and the error word keep the previous call's values: cleared by a kernel
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, qn, 4);
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, D.err, 4);
+    static_assert(kScErr == kScQn + 64 * sizeof(int), "");
+    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(128), 0, st, qn, 68);
     hipLaunchKernelGGL(k_energy<PosX>, dim3(nblk), dim3(kBlock), 0, st, D, PosX{d_x}, red);
-    hipLaunchKernelGGL(k_energy_simpson<PosX>, dim3(64), dim3(kBlock), 0, st, D, PosX{d_x}, qe_u);
-    hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(kBlock), 0, st, D, red, nblk, qe_u, d_out, kNFF + 1);
+    hipLaunchKernelGGL(k_energy_tail<PosX>, dim3(kTailGrid), dim3(kTailBlock), 0, st, D, PosX{d_x}, red, nblk, qe_u,
+                       qn + 4, d_out, kNFF + 1);
     return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
 }
 
 int launch_forces(Ctx &c, const double *d_x, double *d_force, int accumulate, hipStream_t st) {
     Dev D = c.dev();
     const int nblk = grid_for(c, D.n_lanes());
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, c.qn.p, 4);
     const bool mixed = c.opts.precision == MDY_PREC_MIXED;
     if (quad_on(c)) {   // FP64 only (the mode is refused for mixed-precision contexts)
         MDY_TRY(quad_classify(c, D, d_x, st));
@@ -257,35 +302,45 @@ int launch_forces(Ctx &c, const double *d_x, double *d_force, int accumulate, hi
     } else {
         hipLaunchKernelGGL((k_force<false, PosX>), dim3(nblk), dim3(kBlock), 0, st, D, PosX{d_x}, c.contrib.p);
     }
+    const auto gather = mixed ? k_gather<true> : k_gather<false>;
+    const dim3 ggrid(grid_for(c, D.ndof));
+    hipLaunchKernelGGL(gather, ggrid, dim3(kBlock), 0, st, D, c.contrib.p, d_force, accumulate,
+                       c.h_out + kOutForce);
     if (hipGetLastError() != hipSuccess) return MDY_ERR_HIP;
-    // quadrature fallbacks: rare; the count is read back to drive them
-    int h_q[4];
-    if (hipMemcpyAsync(h_q, c.qn.p, sizeof(h_q), hipMemcpyDeviceToHost, st) != hipSuccess) return MDY_ERR_HIP;
+    // quadrature fallbacks: rare; the gather has reported their count and left
+    // the forces to them (read back ahead of the gather: 48 us a call at 40k
+    // cylinders; so: 40)
     if (hipStreamSynchronize(st) != hipSuccess) return MDY_ERR_HIP;
-    if (h_q[1] > kQueueCap) return MDY_ERR_CAPACITY;
-    const int nq = h_q[1];
+    const long long nq = c.h_out[kOutForce];
+    if (nq == 0) return MDY_OK;
+    int *const words = c.qn.p + kOneShot, *const flags = words + 2;
+    int rc = nq > kQueueCap ? MDY_ERR_CAPACITY : MDY_OK;
     const int sblk = c.num_cu * 4;
-    MDY_TRY(ensure(c.simpson_part, (size_t)6 * kRed * sblk));
-    for (int q = 0; q < nq; q++) {
+    if (rc == MDY_OK) rc = ensure(c.simpson_part, (size_t)6 * kRed * sblk);
+    for (int q = 0; rc == MDY_OK && q < (int)nq; q++) {
         for (int moved = 0; moved < 2; moved++) {
             for (int comp = 0; comp < 6; comp++)
                 hipLaunchKernelGGL(k_force_simpson_part, dim3(sblk), dim3(kBlock), 0, st, D, d_x, q, moved, comp,
                                    c.simpson_part.p);
-            if (mixed)
-                hipLaunchKernelGGL(k_force_simpson_final<true>, dim3(1), dim3(kBlock), 0, st, D, d_x, q, moved,
-                                   c.simpson_part.p, sblk, c.contrib.p, c.qn.p + 2);
-            else
-                hipLaunchKernelGGL(k_force_simpson_final<false>, dim3(1), dim3(kBlock), 0, st, D, d_x, q, moved,
-                                   c.simpson_part.p, sblk, c.contrib.p, c.qn.p + 2);
-            int fl[2];
-            if (hipMemcpyAsync(fl, c.qn.p + 2, sizeof(fl), hipMemcpyDeviceToHost, st) != hipSuccess) return MDY_ERR_HIP;
-            if (hipStreamSynchronize(st) != hipSuccess) return MDY_ERR_HIP;
+            hipLaunchKernelGGL(mixed ? k_force_simpson_final<true> : k_force_simpson_final<false>, dim3(1), dim3(kBlock),
+                               0, st, D, d_x, q, moved, c.simpson_part.p, sblk, c.contrib.p, flags);
+            int fl[2] = {0, 0};
+            if (hipMemcpyAsync(fl, flags, sizeof(fl), hipMemcpyDeviceToHost, st) != hipSuccess ||
+                hipStreamSynchronize(st) != hipSuccess) {
+                rc = MDY_ERR_HIP;
+                break;
+            }
             if (!fl[0]) break;
-            if (moved || !fl[1]) return MDY_ERR_FORCE;  // the reference exits here
+            if (moved || !fl[1]) {   // the reference exits here
+                rc = MDY_ERR_FORCE;
+                break;
+            }
         }
     }
-    hipLaunchKernelGGL(mixed ? k_gather<true> : k_gather<false>, dim3(grid_for(c, D.ndof)), dim3(kBlock), 0, st, D,
-                       c.contrib.p, d_force, accumulate);
+    if (rc == MDY_OK)
+        hipLaunchKernelGGL(gather, ggrid, dim3(kBlock), 0, st, D, c.contrib.p, d_force, accumulate, nullptr);
+    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, st, words + 1, 3);
+    if (rc != MDY_OK) return rc;
     return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
 }
 

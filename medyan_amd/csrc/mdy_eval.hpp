@@ -669,14 +669,52 @@ __device__ __forceinline__ void energy_finish(mdy_xsum X, const double v_in[kNFF
     e[kNFF] = bad ? INFINITY : tot;
     e[kNFF + 1] = bad ? tot - 1.0 : tot;
 }
-// the same from per-block records: per-FF doubles at [0, kNFF), exact total at kXsE
-__device__ __forceinline__ void energy_epilogue(const Dev &D, const double *red, int nblk, int nq, const int *qe,
-                                                const double *qe_u, double *lds, double e[kNFF + 2], bool per_ff) {
-    double v[kNFF];
-    if (per_ff) grid_partials_reduce<kNFF>(red, nblk, v, lds);
-    mdy_xsum X;
-    grid_reduce_xsum(red, nblk, kXsE, X, reinterpret_cast<long long *>(lds));
-    energy_finish(X, per_ff ? v : nullptr, nq, qe, qe_u, e);
+// The blocks' records added up word by word by one block of kTailBlock threads:
+// v the per-FF doubles at [0, kNFF), X (EXACT) the exact total at kXsE; both
+// valid in thread 0. Thirty-two lanes read a record's words, 32 records at a
+// time with eight loads each in flight (a lane per record held one 256-byte
+// stride per load: 33 us for 2048 records).
+constexpr int kTailBlock = 1024;
+template <bool EXACT>
+__device__ __forceinline__ void sum_records(const double *red, int nblk, double v[kNFF], mdy_xsum &X) {
+    constexpr int kRows = kTailBlock / kRed, kDeep = 8;
+    __shared__ long long part[kRows][kRed];
+    const int w = threadIdx.x % kRed, r0 = threadIdx.x / kRed;
+    const bool is_d = w < kNFF, is_x = EXACT && w >= kXsE && w < kXsE + 8, is_f = w == kXsE + 7;
+    const long long *q = reinterpret_cast<const long long *>(red) + w;
+    double d = 0.0;
+    long long x = 0;
+    if (is_d || is_x)
+        for (int r = r0; r < nblk; r += kDeep * kRows) {
+            long long u[kDeep];
+#pragma unroll
+            for (int j = 0; j < kDeep; j++) u[j] = r + j * kRows < nblk ? q[(size_t)(r + j * kRows) * kRed] : 0;
+#pragma unroll
+            for (int j = 0; j < kDeep; j++) {
+                d += __longlong_as_double(u[j]);
+                x = is_f ? (x | u[j]) : x + u[j];
+            }
+        }
+    part[r0][w] = is_d ? __double_as_longlong(d) : x;
+    __syncthreads();
+    if (threadIdx.x < kRed) {
+        d = 0.0;
+        x = 0;
+        for (int r = 0; r < kRows; r++) {
+            const long long u = part[r][w];
+            d += __longlong_as_double(u);
+            x = is_f ? (x | u) : x + u;
+        }
+        part[0][w] = is_d ? __double_as_longlong(d) : x;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 0; k < kNFF; k++) v[k] = __longlong_as_double(part[0][k]);
+    if (EXACT) {
+        for (int k = 0; k < MDY_XS_N; k++) X.d[k] = part[0][kXsE + k];
+        X.flags = (int)part[0][kXsE + 7];
+        mdy_xs_norm(&X);
+    }
 }
 
 // ---- Simpson quadrature fallbacks (CylinderExclVolRepulsion.cpp:884-1254) ----

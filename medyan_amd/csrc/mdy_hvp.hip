@@ -125,7 +125,8 @@ __global__ void __launch_bounds__(kBlock, 2) k_hvp(Dev D, const double *__restri
 }
 
 __global__ void __launch_bounds__(kBlock) k_hvp_gather(Dev D, const double *__restrict__ contrib,
-                                                        double *__restrict__ hv) {
+                                                        double *__restrict__ hv, long long *told) {
+    if (told && blockIdx.x == 0 && threadIdx.x == 0) *told = *D.err;
     for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < D.ndof; o += gridDim.x * blockDim.x)
         hv[o] = gather_coord(D, contrib, o);
 }
@@ -185,10 +186,12 @@ __global__ void __launch_bounds__(kBlock) k_energy_jvp(Dev D, const double *__re
     if (threadIdx.x < kNFF) red[(size_t)blockIdx.x * kRed + threadIdx.x] = acc[threadIdx.x];
 }
 
-__global__ void __launch_bounds__(kBlock) k_energy_jvp_final(const double *red, int nblk, double *out) {
-    __shared__ double lds[17 * kNFF + 8];
+// err, told: the error word and where the host reads it
+__global__ void __launch_bounds__(kTailBlock) k_energy_jvp_final(const double *red, int nblk, double *out, const int *err,
+                                                                 long long *told) {
     double v[kNFF];
-    grid_partials_reduce<kNFF>(red, nblk, v, lds);
+    mdy_xsum none;
+    sum_records<false>(red, nblk, v, none);
     if (threadIdx.x == 0) {
         double t = 0.0;
         for (int k = 0; k < kNFF; k++) {
@@ -196,9 +199,11 @@ __global__ void __launch_bounds__(kBlock) k_energy_jvp_final(const double *red, 
             t += v[k];
         }
         out[kNFF] = t;
+        *told = *err;
     }
 }
 
+__global__ void k_tell_err(const int *err, long long *told) { *told = *err; }
 __global__ void k_clear_err(int *err) { *err = 0; }
 
 static int grid_of(const Ctx &c, long long n) {
@@ -206,18 +211,21 @@ static int grid_of(const Ctx &c, long long n) {
     return (int)(g > cap ? cap : g < 1 ? 1 : g);
 }
 
-// reads and clears the error word after the stream's work
-int sync_errors(Ctx &c, hipStream_t st) {
+// The error word after the stream's work, from pinned memory, where the last
+// kernel has written it (a copy to pageable memory took 9 us more); cleared if set.
+static int told_errors(Ctx &c, hipStream_t st) {
     if (hipGetLastError() != hipSuccess) return MDY_ERR_HIP;
-    int e = 0;
-    if (hipMemcpyAsync(&e, c.err.p, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess) return MDY_ERR_HIP;
     if (hipStreamSynchronize(st) != hipSuccess) return MDY_ERR_HIP;
+    const int e = (int)c.h_out[kOutErr];
     if (e) {
         hipLaunchKernelGGL(k_clear_err, dim3(1), dim3(1), 0, st, c.err.p);
         if (hipStreamSynchronize(st) != hipSuccess) return MDY_ERR_HIP;
-        return e;
     }
-    return MDY_OK;
+    return e;
+}
+int sync_errors(Ctx &c, hipStream_t st) {
+    hipLaunchKernelGGL(k_tell_err, dim3(1), dim3(1), 0, st, c.err.p, c.h_out + kOutErr);
+    return told_errors(c, st);
 }
 
 int launch_hvp(Ctx &c, const double *d_x, const double *d_v, double *d_hv, hipStream_t st, bool sync) {
@@ -226,9 +234,10 @@ int launch_hvp(Ctx &c, const double *d_x, const double *d_v, double *d_hv, hipSt
     if (quad) MDY_TRY(quad_classify(c, D, d_x, st));
     hipLaunchKernelGGL(k_hvp, dim3(grid_of(c, D.n_lanes())), dim3(kBlock), 0, st, D, d_x, d_v, c.contrib.p);
     if (quad) MDY_TRY(launch_quad(c, D, 2, d_x, d_v, c.contrib.p, 0, st));
-    hipLaunchKernelGGL(k_hvp_gather, dim3(grid_of(c, D.ndof)), dim3(kBlock), 0, st, D, c.contrib.p, d_hv);
+    hipLaunchKernelGGL(k_hvp_gather, dim3(grid_of(c, D.ndof)), dim3(kBlock), 0, st, D, c.contrib.p, d_hv,
+                       sync ? c.h_out + kOutErr : nullptr);
     if (!sync) return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
-    return sync_errors(c, st);
+    return told_errors(c, st);
 }
 
 int launch_energy_jvp(Ctx &c, const double *d_x, const double *d_w, double *d_out, hipStream_t st) {
@@ -240,8 +249,9 @@ int launch_energy_jvp(Ctx &c, const double *d_x, const double *d_w, double *d_ou
     if (quad) MDY_TRY(quad_classify(c, D, d_x, st));
     hipLaunchKernelGGL(k_energy_jvp, dim3(nblk), dim3(kBlock), 0, st, D, d_x, d_w, c.red.p);
     if (quad) MDY_TRY(launch_quad(c, D, 3, d_x, d_w, c.red.p, nblk, st));
-    hipLaunchKernelGGL(k_energy_jvp_final, dim3(1), dim3(kBlock), 0, st, c.red.p, nblk + nqb, d_out);
-    return sync_errors(c, st);
+    hipLaunchKernelGGL(k_energy_jvp_final, dim3(1), dim3(kTailBlock), 0, st, c.red.p, nblk + nqb, d_out, c.err.p,
+                       c.h_out + kOutErr);
+    return told_errors(c, st);
 }
 
 }  // namespace mdy

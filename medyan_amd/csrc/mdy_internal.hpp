@@ -13,6 +13,9 @@ namespace mdy {
 constexpr int kNFF = MDY_NFF;
 constexpr int kBlock = 256;          // threads per block of every kernel
 constexpr int kQueueCap = 4096;      // excluded-volume quadrature fallback queue
+constexpr int kOneShot = 16;         // qn words of the one-shot calls: energy, force queue counts, two flags, ticket; zero between calls
+// words of Ctx::h_out: host energies; queued force pairs; error word; rebuild totals from there on
+constexpr int kOutForce = 16, kOutErr = 17, kOutNl = 24;
 constexpr int kRed = 32;             // 8-byte words per block in a reduction record
 
 // Interaction tables on the device. The evaluation index space is
@@ -98,7 +101,6 @@ struct Ctx {
     DBuf<int> cell_cnt, cell_rank, near; DBuf<int2> cell_range; DBuf<int4> cell_list;
     DBuf<unsigned long long> row_cnt, row_off;   // per cylinder: pairs << 32 | kept pairs
     DBuf<int> pairs, pair_tmp;    // 2 * npairs (NL, before mother-daughter filtering); npairs
-    DBuf<long long> nl_out;       // totals for the host
     long long n_pairs = 0;
     DBuf<int4> ev_bs; DBuf<double> ev_kr; int n_ev = 0;
     DBuf<int2> ev_cyl;            // monomer-sum form: cylinders of each pair
@@ -115,7 +117,9 @@ struct Ctx {
     DBuf<double> x, xt, f, contrib;
     DBuf<double> red;             // per-block partials
     DBuf<double> out;             // small results
-    DBuf<int> qe, qf, qn, err;
+    DBuf<int> qe, qf, qn, err;    // qn: 16 words of the minimizer's phases, 16 of the one-shot calls (kOneShot)
+    long long *h_out = nullptr;   // pinned: what a call's last kernel tells the host
+    size_t h_out_n = 0;
     DBuf<double> qe_u, simpson_part;
     // CG state
     DBuf<double> F0, F1, S0, S1, xmin;

@@ -5,12 +5,16 @@
 namespace mdy {
 
 // mdy_eval.hip
-int launch_energy(Ctx &c, const double *d_x, double *d_out, hipStream_t st);
+// out: the first n_out of the kNFF energies, the total, the total without the
+// sentinel and the error word
+int launch_energy(Ctx &c, const double *d_x, double *out, int n_out, hipStream_t st);
 int launch_forces(Ctx &c, const double *d_x, double *d_force, int accumulate, hipStream_t st);
 // allocation-free energy: scratch in a file-scope device array of mdy_eval.hip
 int resolve_noalloc_scratch(int device);
 size_t noalloc_scratch_bytes();
 int launch_energy_noalloc(Ctx &c, const double *d_x, double *d_out, hipStream_t st);
+// pinned memory for at least n words; what it held is lost
+int ensure_host_out(Ctx &c, size_t n);
 // mdy_nl.hip
 int build_neighbors(Ctx &c, const double *d_x);
 // mdy_cg.hip

@@ -474,11 +474,11 @@ int build_neighbors(Ctx &c, const double *d_x) {
         hipLaunchKernelGGL(k_bd_flag, dim3(np * nchunk), blk, 0, st, ncyl, nchunk, c.c_b1.p, c.c_b2.p, c.c_minus.p, d_x,
                            c.planes.p, c.bd_cut, c.bd_flag.p, c.bd_off.p);
     }
-    MDY_TRY(ensure(c.nl_out, (size_t)c.n_planes + 3));
+    MDY_TRY(ensure_host_out(c, kOutNl + (size_t)c.n_planes + 3));
+    const long long *tot = c.h_out + kOutNl;
     hipLaunchKernelGGL(k_nl_totals, dim3(1), dim3(1024), 0, st, np, nchunk, c.bd_off.p,
-                       ev ? c.row_off.p + ncyl : nullptr, ev ? misc + 2 : nullptr, c.nl_out.p);
-    std::vector<long long> tot((size_t)np + 3);
-    MDY_HIP(hipMemcpyAsync(tot.data(), c.nl_out.p, tot.size() * sizeof(long long), hipMemcpyDeviceToHost, st));
+                       ev ? c.row_off.p + ncyl : nullptr, ev ? misc + 2 : nullptr, c.h_out + kOutNl);
+    MDY_HIP(hipGetLastError());
     MDY_HIP(hipStreamSynchronize(st));
     if (!tot[1]) return MDY_ERR_NONFINITE;   // an infinite midpoint, or an axis without a number
     c.n_pairs = (unsigned long long)tot[0] >> 32;
