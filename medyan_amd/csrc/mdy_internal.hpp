@@ -109,9 +109,9 @@ struct Ctx {
     DBuf<int> row_cur; DBuf<int2> row; DBuf<int4> row_idx, row_tmp;   // bead -> all slots (Dev::row_idx)
     int n_static = 0;             // entries of st_idx
     DBuf<unsigned char> evq;      // quadrature mode: per-pair flags of the current evaluation
-    DBuf<int> qpan, qcnt, qoff, qmap; // quadrature mode: panels, chunk counts, first chunks, chunk -> pair
-    DBuf<int> qtot;               // quadrature mode: running chunk total (zero between calls)
-    DBuf<double> qpart, qpe;      // quadrature mode: chunk records, per-pair values
+    DBuf<int> qpan, qcnt, qoff, qmap; // quadrature mode: panels, record counts, first records, record -> pair
+    DBuf<unsigned long long> qtot;    // quadrature mode: running record totals (zero between calls)
+    DBuf<double> qpart, qpe;      // quadrature mode: records, per-pair values
     DBuf<int> scan_tmp;
     // evaluation scratch
     DBuf<double> x, xt, f, contrib;

@@ -20,13 +20,16 @@
 // directional derivatives of a pair all differentiate the same discrete
 // rule, so they are mutually consistent to rounding.
 //
-// Work is split into chunks of at most kQuadChunk nodes (a pair with many
-// panels spans several chunks, so the closest pair does not set the kernel's
-// time): k_ev_classify flags the pairs and places each one's chunks, one
-// block per chunk sums its nodes (each thread a fixed subset in a fixed
-// order, then a fixed tree) into a chunk record, and one thread per pair adds
-// its chunk records in chunk order. Results are reproducible bit for bit.
-// The closed-form kernels skip the flagged pairs.
+// Work is split by tiles, a panel of s times a panel of t (16 x 16 nodes). A
+// pair of up to 8 x 8 panels is split into pieces of 4 tiles, each one wave's
+// work; a larger one into at most 16 pieces of at least 64 tiles, each one
+// block's, whose waves take its tiles in turn (so the closest pair does not
+// set the kernel's time). k_ev_classify flags the pairs and places their
+// pieces, k_quad_nodes sums each one's nodes (each lane a fixed subset in a
+// fixed order, then a fixed tree) into a record, and one thread per pair adds
+// its records in order. Results are reproducible bit for bit. The closed-form
+// kernels skip the flagged pairs.
+#include <algorithm>
 #include <cmath>
 
 #include "mdy_eval.hpp"
@@ -36,7 +39,18 @@ namespace mdy {
 
 constexpr double kQuadMaxQ = 1e-3;   // pairs with q below this are integrated numerically
 constexpr int kQuadPanels = 64;      // at most this many panels per cylinder
-constexpr int kQuadChunk = 65536;    // nodes per chunk (256 per thread)
+constexpr int kWavePanels = 8;       // pairs of up to this many panels go to waves, others to blocks
+constexpr int kWaveTiles = 4;        // a wave's piece
+constexpr int kBlockTiles = 64;      // a block's piece, at least
+constexpr int kPieces = 16;          // at most this many pieces per pair
+constexpr int kQuadBlock = 1024;     // threads per block of k_quad_nodes
+constexpr int kQuadWaves = kQuadBlock / 64;
+static_assert(kWavePanels * kWavePanels <= kPieces * kWaveTiles, "pieces of the largest wave pair");
+
+// tiles in a piece of a pair of m panels
+__device__ __forceinline__ int piece_tiles(int m) {
+    return m <= kWavePanels ? kWaveTiles : max(kBlockTiles, (m * m + kPieces - 1) / kPieces);
+}
 
 // 16-point Gauss-Legendre nodes and weights on [0, 1], ascending
 struct GL16 {
@@ -107,19 +121,21 @@ __device__ __forceinline__ int quad_panels(d3 c1, d3 c2, d3 c3, d3 c4) {
     return mr >= (double)kQuadPanels ? kQuadPanels : mr <= 1.0 ? 1 : (int)mr;
 }
 
-// flag[j]; for a flagged pair the panel count pan[j], its chunk count
-// cnt[j] and the index off[j] of its first chunk, taken from the running
-// total *tot (atomically: the order of pairs among the chunks changes no
-// result, since each chunk's nodes and each pair's sum over its chunks in
-// chunk order are fixed), and the chunk -> pair map entries
+// flag[j]; for a flagged pair the panel count pan[j], its record count cnt[j]
+// and its first record off[j], and the record -> pair map. Blocks' pieces take
+// records from the front of the cap records, waves' from the back: tot holds the
+// blocks' count in its low and the waves' in its high half, taken
+// atomically (the order of pairs among the records changes no result, since
+// each record's nodes and each pair's sum over its records are fixed).
 __global__ void __launch_bounds__(kBlock) k_ev_classify(Dev D, const double *__restrict__ x,
                                                          unsigned char *__restrict__ flag, int *__restrict__ pan,
                                                          int *__restrict__ cnt, int *__restrict__ off,
-                                                         int *__restrict__ cmap, int *__restrict__ tot, int cap) {
-    // one atomic per block and sweep turn: the block's chunk counts are
-    // scanned in LDS (wave prefix sums, then the wave totals)
-    __shared__ int wsum[kBlock / 64];
-    __shared__ int bbase;
+                                                         int *__restrict__ map, unsigned long long *__restrict__ tot,
+                                                         int cap) {
+    // one atomic per block and sweep turn: the block's counts are scanned in
+    // LDS (wave prefix sums, then the wave totals), both halves at once
+    __shared__ unsigned long long wsum[kBlock / 64];
+    __shared__ unsigned long long bbase;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int j0 = blockIdx.x * blockDim.x; j0 < D.n_ev; j0 += gridDim.x * blockDim.x) {
         const int j = j0 + threadIdx.x;
@@ -131,32 +147,37 @@ __global__ void __launch_bounds__(kBlock) k_ev_classify(Dev D, const double *__r
             flag[j] = f ? 1 : 0;
             if (f) {
                 m = quad_panels(c1, c2, c3, c4);
-                nc = (256 * m * m + kQuadChunk - 1) / kQuadChunk;   // (16 m)^2 nodes
+                const int pt = piece_tiles(m);
+                nc = (m * m + pt - 1) / pt;
             }
         }
-        int incl = nc;   // inclusive prefix within the wave
+        const bool to_waves = m <= kWavePanels;
+        const unsigned long long mine = to_waves ? (unsigned long long)nc << 32 : (unsigned long long)nc;
+        unsigned long long incl = mine;   // inclusive prefix within the wave
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64);
+            const unsigned long long v = __shfl_up(incl, o, 64);
             if (lane >= o) incl += v;
         }
         if (lane == 63) wsum[wave] = incl;
         __syncthreads();
         if (threadIdx.x == 0) {
-            int s = 0;
-            for (int w = 0; w < kBlock / 64; w++) { const int v = wsum[w]; wsum[w] = s; s += v; }
+            unsigned long long s = 0;
+            for (int w = 0; w < kBlock / 64; w++) { const unsigned long long v = wsum[w]; wsum[w] = s; s += v; }
             bbase = s ? atomicAdd(tot, s) : 0;
         }
         __syncthreads();
         if (j < D.n_ev) {
             if (nc) {
-                const int base = bbase + wsum[wave] + incl - nc;
+                const unsigned long long at = bbase + wsum[wave] + incl - mine;
+                const long long base = to_waves ? (long long)cap - nc - (long long)(at >> 32) : (long long)(at & 0xffffffffull);
                 pan[j] = m;
-                off[j] = base;
-                if (base + nc <= cap) {
-                    for (int q = 0; q < nc; q++) cmap[base + q] = j;
-                } else {
-                    set_err(D.err, MDY_ERR_CAPACITY);   // cannot happen with a cleared total (16 chunks per pair at most)
+                if (base >= 0 && base + nc <= cap) {
+                    off[j] = (int)base;
+                    for (int q = 0; q < nc; q++) map[base + q] = j;
+                } else {   // cannot happen with a cleared total (kPieces records per pair at most)
+                    nc = 0;
+                    set_err(D.err, MDY_ERR_CAPACITY);
                 }
             }
             cnt[j] = nc;
@@ -165,7 +186,7 @@ __global__ void __launch_bounds__(kBlock) k_ev_classify(Dev D, const double *__r
     }
 }
 
-__global__ void k_quad_zero(int *tot) { *tot = 0; }
+__global__ void k_quad_zero(unsigned long long *tot) { *tot = 0; }
 
 __device__ __forceinline__ double clamp01(double v) { return v < 0.0 ? 0.0 : v > 1.0 ? 1.0 : v; }
 
@@ -193,84 +214,160 @@ __device__ __forceinline__ double segment_distance(d3 c1, d3 c2, d3 c3, d3 c4) {
 enum { Q_ENERGY = 0, Q_FORCE = 1, Q_HVP = 2, Q_JVP = 3 };
 template <int W> struct QuadAcc { static constexpr int N = W == Q_ENERGY ? 1 : 9; };
 
-// One block per chunk: the chunk's nodes of its pair into part[chunk]. For
-// Q_ENERGY the sum of W |r|^-4; otherwise G, sum of s h, sum of t h with
-// h = W * 4 r/|r|^6 (Q_FORCE, Q_JVP: minus the gradient of |r|^-4) or
-// h = W grad^2 |r|^-4 dr (Q_HVP, dr the direction v along r).
+// Sum over the wave, the same bits in every lane: 16 lanes by data-parallel
+// moves (no LDS), then the four rows.
+template <int CTRL> __device__ __forceinline__ double dpp_add(double v) {
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_total(double v) {
+    v = dpp_add<0xB1>(v);    // lanes 1 0 3 2
+    v = dpp_add<0x4E>(v);    // lanes 2 3 0 1
+    v = dpp_add<0x141>(v);   // 7 - lane, within eight
+    v = dpp_add<0x140>(v);   // 15 - lane, within sixteen
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
+}
+
+// The nodes of one lane: s node lane % 16 and the four t nodes lane / 16 + 4 q of a tile.
+// The t nodes stay in LDS (tw: node and weight): in registers they made H v spill.
+struct LaneNodes { double s, ws; const double2 *tw; };
+
+// Tiles k0, k0 + step, ... below k1 of pair j by one wave, summed into acc in
+// every lane: for Q_ENERGY the sum of W |r|^-4; otherwise G, sum of s h, sum
+// of t h with h = W r/|r|^6 (Q_FORCE, Q_JVP: minus the gradient of |r|^-4, but
+// for its factor 4) or h = W grad^2 |r|^-4 dr / 4 (Q_HVP, dr the direction v
+// along r). What depends on s only leaves the loop over t.
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_quad_chunks(Dev D, const double *__restrict__ x,
-                                                        const double *__restrict__ v, GL16 g,
-                                                        const int *__restrict__ off, const int *__restrict__ cmap,
-                                                        const int *__restrict__ pan, const int *__restrict__ tot, int cap,
-                                                        double *__restrict__ part) {
+__device__ __forceinline__ void quad_tiles(const Dev &D, const double *__restrict__ x, const double *__restrict__ v,
+                                           const LaneNodes &L, int j, int m, int k0, int k1, int step,
+                                           double acc[QuadAcc<W>::N]) {
     constexpr int NA = QuadAcc<W>::N;
-    __shared__ double lds[17 * NA + 8];
-    __shared__ double gt[16], gw[16];   // the rule, indexed per node (no dynamic indexing of kernel arguments)
-    if (threadIdx.x < 16) {
-        gt[threadIdx.x] = g.t[threadIdx.x];
-        gw[threadIdx.x] = g.w[threadIdx.x];
+    const int4 b = D.ev_bs[j];
+    const d3 c1 = ld3(x, b.x), c2 = ld3(x, b.y), c3 = ld3(x, b.z), c4 = ld3(x, b.w);
+    const d3 v1 = sub(c2, c1), v2 = sub(c4, c3), c13 = sub(c1, c3);
+    d3 e1{0, 0, 0}, e2{0, 0, 0}, e13{0, 0, 0};   // HVP: the direction at (c2 - c1), (c4 - c3), (c1 - c3)
+    if (W == Q_HVP) {
+        const d3 u1 = ld3(v, b.x), u2 = ld3(v, b.y), u3 = ld3(v, b.z), u4 = ld3(v, b.w);
+        e1 = sub(u2, u1);
+        e2 = sub(u4, u3);
+        e13 = sub(u1, u3);
     }
-    __syncthreads();
-    const int total = min(*tot, cap);
-    for (int ch = blockIdx.x; ch < total; ch += gridDim.x) {
-        const int j = cmap[ch];
-        const int4 b = D.ev_bs[j];
-        const d3 c1 = ld3(x, b.x), c2 = ld3(x, b.y), c3 = ld3(x, b.z), c4 = ld3(x, b.w);
-        const d3 v1 = sub(c2, c1), v2 = sub(c4, c3), c13 = sub(c1, c3);
-        const int m = pan[j];
-        const int n = 16 * m, nn = n * n;
-        const int k0 = (ch - off[j]) * kQuadChunk, k1 = min(nn, k0 + kQuadChunk);
-        const double im = 1.0 / (double)m;
-        d3 e1{0, 0, 0}, e2{0, 0, 0}, e13{0, 0, 0};   // HVP: the direction at (c2 - c1), (c4 - c3), (c1 - c3)
-        if (W == Q_HVP) {
-            const d3 u1 = ld3(v, b.x), u2 = ld3(v, b.y), u3 = ld3(v, b.z), u4 = ld3(v, b.w);
-            e1 = sub(u2, u1);
-            e2 = sub(u4, u3);
-            e13 = sub(u1, u3);
-        }
-        double acc[NA];
+    auto at = [](d3 o, double k, d3 d) {
+        return d3{__builtin_fma(k, d.x, o.x), __builtin_fma(k, d.y, o.y), __builtin_fma(k, d.z, o.z)};
+    };
+    const double im = 1.0 / (double)m;
+    int ps = k0 / m, pt = k0 - ps * m;
+    for (int k = k0; k < k1; k += step) {
+        const double s = ((double)ps + L.s) * im;
+        const d3 rs = at(c13, s, v1), es = at(e13, s, e1);
+        double g[NA == 1 ? 1 : 6];
 #pragma unroll
-        for (int k = 0; k < NA; k++) acc[k] = 0.0;
-        for (int k = k0 + threadIdx.x; k < k1; k += blockDim.x) {
-            const int i = k / n, l = k - i * n;
-            const double s = ((double)(i >> 4) + gt[i & 15]) * im, ws = gw[i & 15] * im;
-            const double t = ((double)(l >> 4) + gt[l & 15]) * im, wt = gw[l & 15] * im;
-            const d3 r{c13.x + s * v1.x - t * v2.x, c13.y + s * v1.y - t * v2.y, c13.z + s * v1.z - t * v2.z};
-            const double d2 = dot3(r, r), inv = 1.0 / d2, inv2 = inv * inv, wst = ws * wt;
+        for (int q = 0; q < (NA == 1 ? 1 : 6); q++) g[q] = 0.0;
+#pragma unroll 2
+        for (int q = 0; q < 4; q++) {
+            const double2 nt = L.tw[4 * q];
+            const double t = ((double)pt + nt.x) * im;
+            const d3 r = at(rs, -t, v2);
+            const double d2 = __builtin_fma(r.z, r.z, __builtin_fma(r.y, r.y, r.x * r.x));
+            const double inv = 1.0 / d2, inv2 = inv * inv;
             if (W == Q_ENERGY) {
-                acc[0] += wst * inv2;
+                g[0] = __builtin_fma(nt.y, inv2, g[0]);
             } else {
+                const double a = nt.y * (inv2 * inv);
                 d3 h;
                 if (W == Q_HVP) {
-                    // d/dt of the gradient of |r|^-4 along dr: -4 dr/|r|^6 + 24 (r.dr) r/|r|^8
-                    const d3 dr{e13.x + s * e1.x - t * e2.x, e13.y + s * e1.y - t * e2.y, e13.z + s * e1.z - t * e2.z};
-                    const double a = -4.0 * wst * inv2 * inv, c = 24.0 * wst * inv2 * inv2 * dot3(r, dr);
-                    h = d3{a * dr.x + c * r.x, a * dr.y + c * r.y, a * dr.z + c * r.z};
+                    // d/dt of the gradient of |r|^-4 along dr, over 4: -dr/|r|^6 + 6 (r.dr) r/|r|^8
+                    const d3 dr = at(es, -t, e2);
+                    const double rd = __builtin_fma(r.z, dr.z, __builtin_fma(r.y, dr.y, r.x * dr.x));
+                    const double c = 6.0 * (a * inv) * rd;
+                    h = d3{__builtin_fma(c, r.x, -a * dr.x), __builtin_fma(c, r.y, -a * dr.y),
+                           __builtin_fma(c, r.z, -a * dr.z)};
                 } else {
-                    // -grad of |r|^-4 with respect to r: 4 r / |r|^6
-                    const double a = 4.0 * wst * inv2 * inv;
                     h = d3{a * r.x, a * r.y, a * r.z};
                 }
-                acc[0] += h.x; acc[1] += h.y; acc[2] += h.z;
-                acc[3] += s * h.x; acc[4] += s * h.y; acc[5] += s * h.z;
-                acc[6] += t * h.x; acc[7] += t * h.y; acc[8] += t * h.z;
+                g[0] += h.x; g[1] += h.y; g[2] += h.z;
+                g[3] = __builtin_fma(t, h.x, g[3]); g[4] = __builtin_fma(t, h.y, g[4]); g[5] = __builtin_fma(t, h.z, g[5]);
             }
         }
-        block_reduce<NA>(acc, lds);
-        if (threadIdx.x < NA) part[(size_t)ch * NA + threadIdx.x] = acc[threadIdx.x];
+        acc[0] += g[0];
+        if constexpr (NA > 1) {
+            acc[1] += g[1]; acc[2] += g[2];
+            acc[3] = __builtin_fma(s, g[0], acc[3]); acc[4] = __builtin_fma(s, g[1], acc[4]);
+            acc[5] = __builtin_fma(s, g[2], acc[5]);
+            acc[6] += g[3]; acc[7] += g[4]; acc[8] += g[5];
+        }
+        for (pt += step; pt >= m; pt -= m) ps++;
+    }
+    // the weights' common factors: w_s / m^2, and the gradient's 4
+    const double f = (W == Q_ENERGY ? 1.0 : 4.0) * L.ws * (im * im);
+#pragma unroll
+    for (int q = 0; q < NA; q++) acc[q] = wave_total(acc[q] * f);
+}
+
+// The records' sums: the blocks' pieces first, one per block and turn, then the
+// waves', one per wave and turn. Bound by FP64 instruction issue on the CUs
+// that hold the closest pairs, and by a wave's chain of about 16 nodes; a lane
+// keeps its s node through a tile, and pieces are small so that they spread
+// over the CUs. At 66k pairs, 1.5k of them flagged, H v / force / energy take
+// 32 / 26 / 17 us; 107 / 89 / 67 with one block of 256 threads per 65536 nodes,
+// a division of the node's number into s and t and a block reduction per pair;
+// 49 / 41 / 28 with pieces of 16 tiles per wave and 256 per block.
+template <int W>
+__global__ void __launch_bounds__(kQuadBlock) k_quad_nodes(Dev D, const double *__restrict__ x,
+                                                           const double *__restrict__ v, GL16 g,
+                                                           const int *__restrict__ off, const int *__restrict__ map,
+                                                           const int *__restrict__ pan,
+                                                           const unsigned long long *__restrict__ tot, int cap,
+                                                           double *__restrict__ part) {
+    constexpr int NA = QuadAcc<W>::N;
+    __shared__ double sum[kQuadWaves][NA];
+    __shared__ double2 tw[16];   // the rule, indexed per lane (no dynamic indexing of kernel arguments)
+    if (threadIdx.x < 16) tw[threadIdx.x] = make_double2(g.t[threadIdx.x], g.w[threadIdx.x]);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const LaneNodes L{tw[lane & 15].x, tw[lane & 15].y, tw + (lane >> 4)};
+    const unsigned long long n = *tot;
+    const int nb = (int)min(n & 0xffffffffull, (unsigned long long)cap);
+    const int nw = (int)min(n >> 32, (unsigned long long)(cap - nb));
+    for (int at = blockIdx.x; at < nb; at += gridDim.x) {
+        const int j = map[at], m = pan[j], size = piece_tiles(m), k0 = (at - off[j]) * size;
+        double acc[NA] = {};
+        quad_tiles<W>(D, x, v, L, j, m, k0 + wave, min(m * m, k0 + size), kQuadWaves, acc);
+        if (lane == 0)
+#pragma unroll
+            for (int k = 0; k < NA; k++) sum[wave][k] = acc[k];
+        __syncthreads();
+        if (threadIdx.x < NA) {
+            double r = 0.0;
+            for (int w = 0; w < kQuadWaves; w++) r += sum[w][threadIdx.x];
+            part[(size_t)at * NA + threadIdx.x] = r;
+        }
+        __syncthreads();   // sum is rewritten by the next turn
+    }
+    // to the blocks in turn, so that few pieces spread over all CUs
+    for (int q = wave * gridDim.x + blockIdx.x; q < nw; q += kQuadWaves * gridDim.x) {
+        const int at = cap - 1 - q, j = map[at], m = pan[j], k0 = (at - off[j]) * kWaveTiles;
+        double acc[NA] = {};
+        quad_tiles<W>(D, x, v, L, j, m, k0, min(m * m, k0 + kWaveTiles), 1, acc);
+        if (lane == 0)
+#pragma unroll
+            for (int k = 0; k < NA; k++) part[(size_t)at * NA + k] = acc[k];
     }
 }
 
-// One thread per pair: its chunk records added in chunk order. Q_FORCE /
+// One thread per pair: its records added in order. Q_FORCE /
 // Q_HVP: the pair's four slots; Q_ENERGY: pe[j] = its energy; Q_JVP:
 // pe[j] = grad E_pair . w (pe[j] = 0 for pairs left to the closed form).
-// The running chunk total is cleared for the next call (this kernel follows
-// the chunk kernel on the stream, so every chunk has run).
+// The running totals are cleared for the next call (this kernel follows
+// k_quad_nodes on the stream, so every record is written).
 template <int W>
 __global__ void __launch_bounds__(kBlock) k_quad_finish(Dev D, const double *__restrict__ v,
                                                         const int *__restrict__ off, const int *__restrict__ cnt,
                                                         const double *__restrict__ part, double *__restrict__ slots,
-                                                        double *__restrict__ pe, int *__restrict__ tot, int cap) {
+                                                        double *__restrict__ pe,
+                                                        unsigned long long *__restrict__ tot) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *tot = 0;
     constexpr int NA = QuadAcc<W>::N;
     bool ok = true;
@@ -282,7 +379,7 @@ __global__ void __launch_bounds__(kBlock) k_quad_finish(Dev D, const double *__r
         double acc[NA];
 #pragma unroll
         for (int k = 0; k < NA; k++) acc[k] = 0.0;
-        for (int q = off[j], qe = min(off[j] + cnt[j], cap); q < qe; q++)
+        for (int q = off[j], qe = off[j] + cnt[j]; q < qe; q++)
 #pragma unroll
             for (int k = 0; k < NA; k++) acc[k] += part[(size_t)q * NA + k];
         const double kr = D.ev_kr[j];
@@ -348,9 +445,12 @@ bool quad_on(const Ctx &c) {
     return c.opts.coplanar_mode == MDY_COPLANAR_QUADRATURE && !c.ev_mon && c.n_ev > 0;
 }
 
+// one pair per thread up to one block per CU: more blocks only give the total
+// more records to read (4 per CU: k_energy_tail 10.4 us at
+// 66k pairs; so: 7.3)
 int quad_blocks(const Ctx &c) {
-    const int g = c.num_cu * 4;
-    return c.n_ev < g ? (c.n_ev < 1 ? 1 : c.n_ev) : g;
+    const int g = (c.n_ev + kBlock - 1) / kBlock;
+    return g < c.num_cu ? (g < 1 ? 1 : g) : c.num_cu;
 }
 
 int quad_classify(Ctx &c, Dev &D, const double *d_x, hipStream_t st) {
@@ -359,10 +459,10 @@ int quad_classify(Ctx &c, Dev &D, const double *d_x, hipStream_t st) {
     MDY_TRY(ensure(c.qpan, n));
     MDY_TRY(ensure(c.qcnt, n));
     MDY_TRY(ensure(c.qoff, n));
-    MDY_TRY(ensure(c.qmap, 16 * n));   // at most (16 * kQuadPanels)^2 / kQuadChunk = 16 chunks per pair
-    // everything the quadrature kernels use is allocated before the chunk total
-    // is taken, so nothing fails between this call and the kernel that clears it
-    MDY_TRY(ensure(c.qpart, 16 * n * 9));
+    MDY_TRY(ensure(c.qmap, kPieces * n));
+    // everything the quadrature kernels use is allocated before the totals
+    // are taken, so nothing fails between this call and the kernel that clears them
+    MDY_TRY(ensure(c.qpart, kPieces * n * 9));
     MDY_TRY(ensure(c.qpe, n));
     if (!c.qtot.p) {
         MDY_TRY(ensure(c.qtot, 1));
@@ -371,7 +471,7 @@ int quad_classify(Ctx &c, Dev &D, const double *d_x, hipStream_t st) {
     long long g = ((long long)n + kBlock - 1) / kBlock, cap = (long long)c.num_cu * 8;
     const dim3 grid((int)(g > cap ? cap : g < 1 ? 1 : g));
     hipLaunchKernelGGL(k_ev_classify, grid, dim3(kBlock), 0, st, D, d_x, c.evq.p, c.qpan.p, c.qcnt.p, c.qoff.p,
-                       c.qmap.p, c.qtot.p, (int)(16 * n));
+                       c.qmap.p, c.qtot.p, (int)(kPieces * n));
     D.evq = c.evq.p;
     return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
 }
@@ -380,14 +480,16 @@ template <int W>
 static void quad_launch(Ctx &c, const Dev &D, const double *d_x, const double *d_v, double *out, int rec0,
                         hipStream_t st) {
     const long long n = c.n_ev;
-    const dim3 blk(kBlock), chunks(c.num_cu * 8);
+    const dim3 blk(kBlock);
     long long g = (n + kBlock - 1) / kBlock, cap = (long long)c.num_cu * 8;
     const dim3 pairs((int)(g > cap ? cap : g < 1 ? 1 : g));
-    const int ccap = (int)(16 * n);
-    hipLaunchKernelGGL(k_quad_chunks<W>, chunks, blk, 0, st, D, d_x, d_v, gl16(), c.qoff.p, c.qmap.p, c.qpan.p,
-                       c.qtot.p, ccap, c.qpart.p);
+    const int rcap = (int)(kPieces * n);
+    // one block per CU, fewer where the table cannot hold as many flagged pairs
+    const int nodes = (int)std::min<long long>(c.num_cu, std::max<long long>(n / 8, 16));
+    hipLaunchKernelGGL(k_quad_nodes<W>, dim3(nodes), dim3(kQuadBlock), 0, st, D, d_x, d_v, gl16(), c.qoff.p, c.qmap.p,
+                       c.qpan.p, c.qtot.p, rcap, c.qpart.p);
     hipLaunchKernelGGL(k_quad_finish<W>, pairs, blk, 0, st, D, d_v, c.qoff.p, c.qcnt.p, c.qpart.p, out, c.qpe.p,
-                       c.qtot.p, ccap);
+                       c.qtot.p);
     if (W == Q_ENERGY || W == Q_JVP)
         hipLaunchKernelGGL(k_quad_records<W>, dim3(quad_blocks(c)), blk, 0, st, D, c.qpe.p, out, rec0);
 }
@@ -408,7 +510,7 @@ int quad_pair_count(Ctx &c, const double *d_x, hipStream_t st, int *count) {
     if (!quad_on(c)) return MDY_OK;
     Dev D = c.dev();
     MDY_TRY(quad_classify(c, D, d_x, st));
-    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(1), 0, st, c.qtot.p);   // no quadrature follows: clear the total
+    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(1), 0, st, c.qtot.p);   // no quadrature follows: clear the totals
     std::vector<unsigned char> h((size_t)c.n_ev);
     MDY_HIP(hipMemcpyAsync(h.data(), c.evq.p, h.size(), hipMemcpyDeviceToHost, st));
     MDY_HIP(hipStreamSynchronize(st));
