@@ -297,6 +297,21 @@ int mdy_hvp_dev_async(mdy_ctx *ctx, const double *d_coord, const double *d_v, do
 /* Waits for the stream (NULL = the context's) and returns the failure an
  * asynchronous call left, clearing it; MDY_OK if none. */
 int mdy_sync_errors(mdy_ctx *ctx, void *stream);
+/* (H + shift I) w = b by conjugate gradients on those products. On entry d_w
+ * is zero and d_r and d_p hold b; d_hp is scratch (3 n_beads doubles each). rr
+ * is b.b; iterates until r.r <= tol, at most maxiter times. Where p.(H + shift
+ * I)p is not positive the solve ends with that direction in d_p. The scalars
+ * stay on the device; returns when the solve has ended. No reference
+ * counterpart. */
+typedef struct mdy_solve_result {
+    int32_t iterations;
+    int32_t not_positive;   /* 1: ended at d_p's curvature */
+    double residual_sq;     /* r.r */
+    double curvature;       /* p.(H + shift I)p if not_positive */
+} mdy_solve_result;
+int mdy_solve_hessian_dev(mdy_ctx *ctx, const double *d_coord, double *d_w, double *d_r, double *d_p, double *d_hp,
+                          double rr, double tol, int32_t maxiter, double shift, void *stream,
+                          mdy_solve_result *result);
 /* Directional derivatives of the individual energies of the exact-gradient
  * force field: d_out[k] = grad E_k(x) . w for the MDY_NFF force fields, then
  * their sum. No reference counterpart (derivative of

@@ -115,6 +115,11 @@ class Opts(C.Structure):
                 ("block_size", C.c_int32), ("blocks_per_cu", C.c_int32)]
 
 
+class SolveResult(C.Structure):
+    _fields_ = [("iterations", C.c_int32), ("not_positive", C.c_int32), ("residual_sq", C.c_double),
+                ("curvature", C.c_double)]
+
+
 class GenParams(C.Structure):
     _fields_ = [("seed", C.c_uint64), ("n_filaments", C.c_int32), ("cyl_per_filament", C.c_int32),
                 ("box", C.c_double), ("n_linkers", C.c_int32), ("n_motors", C.c_int32),

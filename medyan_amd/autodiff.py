@@ -260,18 +260,28 @@ def solve_hessian(ctx: Context, x: torch.Tensor, b: torch.Tensor, rtol=1e-10, ma
     bb = rr
     if bb == 0.0:
         return w, 0, 0.0
+    tol = rtol * rtol * bb
     it = 0
-    while it < maxiter and rr > rtol * rtol * bb:
+    if modes is None and maxiter > 0 and rr > tol:   # nothing between two products needs torch
+        _check(ctx, x)
+        _check(ctx, b, "v")
+        hp = torch.empty_like(b)
+        res = []
+        _ordered(lambda s: res.append(ctx.solve_hessian_dev(
+            x.data_ptr(), w.data_ptr(), r.data_ptr(), p.data_ptr(), hp.data_ptr(), rr, tol,
+            math.ceil(min(maxiter, 2**31 - 1)), float(shift or 0.0), s)))
+        it, rr = int(res[0].iterations), float(res[0].residual_sq)
+        if res[0].not_positive:
+            _not_positive(p, float(res[0].curvature), shift, it)
+        return w, it, math.sqrt(rr / bb)
+    while it < maxiter and rr > tol:
         hp = hvp(ctx, x, p)
         if shift:
             hp.add_(p, alpha=shift)
         hp = P(hp)
         php = float(torch.dot(p, hp))
         if not php > 0.0:
-            pp = float(torch.dot(p, p))
-            raise NotAMinimum(f"Hessian not positive along a conjugate direction (p.Hp = {php:g}, "
-                              f"|p|^2 = {pp:g}, iteration {it}): not a minimum",
-                              p / math.sqrt(pp), php / pp - shift)
+            _not_positive(p, php, shift, it)
         a = rr / php
         w.add_(p, alpha=a)
         r.add_(hp, alpha=-a)
@@ -280,6 +290,13 @@ def solve_hessian(ctx: Context, x: torch.Tensor, b: torch.Tensor, rtol=1e-10, ma
         rr = rr_new
         it += 1
     return w, it, math.sqrt(rr / bb)
+
+
+def _not_positive(p, php, shift, it):
+    pp = float(torch.dot(p, p))
+    raise NotAMinimum(f"Hessian not positive along a conjugate direction (p.Hp = {php:g}, "
+                      f"|p|^2 = {pp:g}, iteration {it}): not a minimum",
+                      p / math.sqrt(pp), php / pp - shift)
 
 
 def stiffness_sensitivity(ctx: Context, x_star: torch.Tensor, grad_l: torch.Tensor, rtol=1e-10, maxiter=20000,

@@ -173,7 +173,7 @@ void mdy_destroy(mdy_ctx *ctx) {
     release(c.bd_plane); release(c.bd_k); release(c.bd_sl); release(c.row);
     release(c.row_cur); release(c.row_idx); release(c.row_tmp); release(c.scan_tmp); release(c.x); release(c.xt); release(c.f);
     release(c.batch_args); release(c.batch_map); release(c.batch_done); release(c.evq); release(c.qpan); release(c.qcnt); release(c.qoff);
-    release(c.qmap); release(c.qpart); release(c.qpe); release(c.qtot);
+    release(c.qmap); release(c.solve); release(c.qpart); release(c.qpe); release(c.qtot);
     if (c.h_out) (void)hipHostFree(c.h_out);
     release(c.contrib); release(c.red); release(c.out); release(c.qe); release(c.qf); release(c.qn); release(c.err);
     release(c.qe_u); release(c.simpson_part); release(c.F0); release(c.F1); release(c.S0); release(c.S1);
@@ -567,6 +567,19 @@ int mdy_sync_errors(mdy_ctx *ctx, void *stream) {
     if (!c.err.p) return MDY_OK;
     int rc = sync_errors(c, st);
     if (rc != MDY_OK) return fail(ctx, rc, "a device call enqueued earlier failed");
+    return MDY_OK;
+}
+
+int mdy_solve_hessian_dev(mdy_ctx *ctx, const double *d_coord, double *d_w, double *d_r, double *d_p, double *d_hp,
+                          double rr, double tol, int32_t maxiter, double shift, void *stream,
+                          mdy_solve_result *result) {
+    if (!ctx || !d_coord || !d_w || !d_r || !d_p || !d_hp || !result) return MDY_ERR_ARG;
+    Ctx &c = ctx->c;
+    if (!c.have_sys || !c.have_nl) return fail(ctx, MDY_ERR_STATE, "network / neighbor list missing");
+    (void)hipSetDevice(c.device);
+    hipStream_t st = stream ? (hipStream_t)stream : c.stream;
+    int rc = solve_hessian(c, d_coord, d_w, d_r, d_p, d_hp, rr, tol, maxiter, shift, st, result);
+    if (rc != MDY_OK) return fail(ctx, rc, "hvp failed");
     return MDY_OK;
 }
 

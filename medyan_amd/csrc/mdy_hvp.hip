@@ -228,16 +228,167 @@ int sync_errors(Ctx &c, hipStream_t st) {
     return told_errors(c, st);
 }
 
+// H v's slots; the quadrature pairs' classification stays for another product with `keep`
+static int hvp_slots(Ctx &c, const Dev &D, const double *d_x, const double *d_v, hipStream_t st, bool keep) {
+    hipLaunchKernelGGL(k_hvp, dim3(grid_of(c, D.n_lanes())), dim3(kBlock), 0, st, D, d_x, d_v, c.contrib.p);
+    return quad_on(c) ? launch_quad(c, D, 2, d_x, d_v, c.contrib.p, 0, st, keep) : MDY_OK;
+}
+
 int launch_hvp(Ctx &c, const double *d_x, const double *d_v, double *d_hv, hipStream_t st, bool sync) {
     Dev D = c.dev();
-    const bool quad = quad_on(c);
-    if (quad) MDY_TRY(quad_classify(c, D, d_x, st));
-    hipLaunchKernelGGL(k_hvp, dim3(grid_of(c, D.n_lanes())), dim3(kBlock), 0, st, D, d_x, d_v, c.contrib.p);
-    if (quad) MDY_TRY(launch_quad(c, D, 2, d_x, d_v, c.contrib.p, 0, st));
+    if (quad_on(c)) MDY_TRY(quad_classify(c, D, d_x, st));
+    MDY_TRY(hvp_slots(c, D, d_x, d_v, st, false));
     hipLaunchKernelGGL(k_hvp_gather, dim3(grid_of(c, D.ndof)), dim3(kBlock), 0, st, D, c.contrib.p, d_hv,
                        sync ? c.h_out + kOutErr : nullptr);
     if (!sync) return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
     return told_errors(c, st);
+}
+
+// ---------------------------------------------------------------------------
+// (H + shift I) w = b by conjugate gradients. An iteration is H p's slots and
+// three kernels: the gather with p.Hp, the step along p with r.r, and the next
+// direction. Each sums the block sums of the one before, in a fixed order, so
+// the scalars stay on the device and no iteration waits for the host, which
+// enqueues kSolveAhead iterations ahead of the last one it has seen end; after the
+// stop, the kernels of those do nothing to w, r and p. Bound by the latency of
+// its kernels (six with quadrature pairs) at a few thousand cylinders: 32 us
+// per iteration at 5k; one product with a host wait and its own classification
+// of the pairs, two dot products read back and five vector kernels took 126.
+// ---------------------------------------------------------------------------
+constexpr int kSolveAhead = 2;
+enum { S_RR = 0, S_STOP = 2, S_ITER, S_PHP, S_SUMS = 8 };   // scalars: r.r of even and odd iterations, ...
+enum { STOP_CONVERGED = 1, STOP_CURVATURE, STOP_ERROR };
+
+__global__ void k_solve_begin(double *s, double rr) {
+    s[S_RR] = rr;
+    s[S_STOP] = s[S_ITER] = s[S_PHP] = 0.0;
+}
+
+// the blocks' sums added up by every block alike
+__device__ __forceinline__ double sum_of_blocks(const double *__restrict__ part, int n, double *lds) {
+    double v[1] = {0.0};
+    for (int k = threadIdx.x; k < n; k += blockDim.x) v[0] += part[k];
+    block_reduce<1>(v, lds);
+    return v[0];
+}
+
+__global__ void __launch_bounds__(kBlock) k_solve_gather(Dev D, const double *__restrict__ contrib,
+                                                         const double *__restrict__ p, double shift,
+                                                         double *__restrict__ hp, const double *s,
+                                                         double *__restrict__ part) {
+    __shared__ double lds[24];
+    if (s[S_STOP] != 0.0) return;
+    double v[1] = {0.0};
+    for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < D.ndof; o += gridDim.x * blockDim.x) {
+        const double q = p[o], h = __builtin_fma(shift, q, gather_coord(D, contrib, o));
+        hp[o] = h;
+        v[0] = __builtin_fma(q, h, v[0]);
+    }
+    block_reduce<1>(v, lds);
+    if (threadIdx.x == 0) part[blockIdx.x] = v[0];
+}
+
+__global__ void __launch_bounds__(kBlock) k_solve_step(int n, int odd, double *s, const double *__restrict__ php_part,
+                                                       int nphp, const double *__restrict__ p,
+                                                       const double *__restrict__ hp, double *__restrict__ w,
+                                                       double *__restrict__ r, double *__restrict__ rr_part) {
+    __shared__ double lds[24];
+    if (s[S_STOP] != 0.0) return;
+    const double php = sum_of_blocks(php_part, nphp, lds);
+    if (!(php > 0.0)) {   // the same in every block
+        if (blockIdx.x == 0 && threadIdx.x == 0) { s[S_PHP] = php; s[S_STOP] = STOP_CURVATURE; }
+        return;
+    }
+    const double a = s[S_RR + odd] / php;
+    double v[1] = {0.0};
+    for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < n; o += gridDim.x * blockDim.x) {
+        w[o] = __builtin_fma(a, p[o], w[o]);
+        const double q = __builtin_fma(-a, hp[o], r[o]);
+        r[o] = q;
+        v[0] = __builtin_fma(q, q, v[0]);
+    }
+    block_reduce<1>(v, lds);
+    if (threadIdx.x == 0) rr_part[blockIdx.x] = v[0];
+}
+
+// told: pinned, the reason to stop. A block that sees the stop of this launch
+// leaves its part of p, which nothing reads then.
+__global__ void __launch_bounds__(kBlock) k_solve_dir(int n, int odd, double *s, const double *__restrict__ rr_part,
+                                                      int nrr, const double *__restrict__ r, double *__restrict__ p,
+                                                      double tol, const int *err, long long *told) {
+    __shared__ double lds[24];
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    const double stop = s[S_STOP];
+    if (stop != 0.0) {   // no curvature: p is the direction to report
+        if (first && stop == STOP_CURVATURE) *told = *err ? STOP_ERROR : STOP_CURVATURE;
+        return;
+    }
+    const double rr = sum_of_blocks(rr_part, nrr, lds), beta = rr / s[S_RR + odd];
+    for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < n; o += gridDim.x * blockDim.x)
+        p[o] = __builtin_fma(p[o], beta, r[o]);
+    if (first) {
+        s[S_RR + 1 - odd] = rr;
+        s[S_ITER] += 1.0;
+        const int why = *err ? STOP_ERROR : !(rr > tol) ? STOP_CONVERGED : 0;
+        if (why) {
+            s[S_STOP] = why;
+            *told = why;
+        }
+    }
+}
+
+static int solve_loop(Ctx &c, const Dev &D, const double *d_x, double *d_w, double *d_r, double *d_p, double *d_hp,
+                      double tol, int maxiter, double shift, hipStream_t st, hipEvent_t *ended) {
+    const int n = D.ndof, ng = grid_of(c, n), nv = ng < c.num_cu ? ng : c.num_cu;
+    double *s = c.solve.p, *php = s + S_SUMS, *rr = php + ng;
+    volatile long long *told = c.h_out + kOutSolve;
+    for (int it = 0; it < maxiter && *told == 0; it++) {
+        if (it >= kSolveAhead) {
+            MDY_HIP(hipEventSynchronize(ended[it % kSolveAhead]));
+            if (*told != 0) break;
+        }
+        MDY_TRY(hvp_slots(c, D, d_x, d_p, st, true));
+        hipLaunchKernelGGL(k_solve_gather, dim3(ng), dim3(kBlock), 0, st, D, c.contrib.p, d_p, shift, d_hp, s, php);
+        hipLaunchKernelGGL(k_solve_step, dim3(nv), dim3(kBlock), 0, st, n, it & 1, s, php, ng, d_p, d_hp, d_w, d_r, rr);
+        hipLaunchKernelGGL(k_solve_dir, dim3(nv), dim3(kBlock), 0, st, n, it & 1, s, rr, nv, d_r, d_p, tol, c.err.p,
+                           c.h_out + kOutSolve);
+        MDY_HIP(hipGetLastError());
+        MDY_HIP(hipEventRecord(ended[it % kSolveAhead], st));
+    }
+    return MDY_OK;
+}
+
+int solve_hessian(Ctx &c, const double *d_x, double *d_w, double *d_r, double *d_p, double *d_hp, double rr, double tol,
+                  int maxiter, double shift, hipStream_t st, mdy_solve_result *res) {
+    Dev D = c.dev();
+    MDY_TRY(ensure(c.solve, S_SUMS + 2 * (size_t)grid_of(c, D.ndof)));
+    hipEvent_t ended[kSolveAhead] = {};
+    int rc = MDY_OK;
+    for (hipEvent_t &e : ended)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) rc = MDY_ERR_HIP;
+    c.h_out[kOutSolve] = 0;
+    const bool quad = quad_on(c);
+    if (rc == MDY_OK) {
+        hipLaunchKernelGGL(k_solve_begin, dim3(1), dim3(1), 0, st, c.solve.p, rr);
+        if (quad) rc = quad_classify(c, D, d_x, st);
+        if (rc == MDY_OK) {
+            rc = solve_loop(c, D, d_x, d_w, d_r, d_p, d_hp, tol, maxiter, shift, st, ended);
+            if (quad && quad_end(c, st) != MDY_OK) rc = MDY_ERR_HIP;
+        }
+    }
+    // errors of the products, and the end of everything enqueued
+    const int e = sync_errors(c, st);
+    if (rc == MDY_OK) rc = e;
+    for (hipEvent_t &v : ended)
+        if (v) (void)hipEventDestroy(v);
+    if (rc != MDY_OK) return rc;
+    double s[S_SUMS];
+    MDY_HIP(hipMemcpy(s, c.solve.p, sizeof(s), hipMemcpyDeviceToHost));
+    res->iterations = (int32_t)s[S_ITER];
+    res->residual_sq = s[S_RR + (res->iterations & 1)];
+    res->curvature = s[S_PHP];
+    res->not_positive = s[S_STOP] == STOP_CURVATURE;
+    return MDY_OK;
 }
 
 int launch_energy_jvp(Ctx &c, const double *d_x, const double *d_w, double *d_out, hipStream_t st) {

@@ -15,7 +15,7 @@ constexpr int kBlock = 256;          // threads per block of every kernel
 constexpr int kQueueCap = 4096;      // excluded-volume quadrature fallback queue
 constexpr int kOneShot = 16;         // qn words of the one-shot calls: energy, force queue counts, two flags, ticket; zero between calls
 // words of Ctx::h_out: host energies; queued force pairs; error word; rebuild totals from there on
-constexpr int kOutForce = 16, kOutErr = 17, kOutNl = 24;
+constexpr int kOutForce = 16, kOutErr = 17, kOutSolve = 18, kOutNl = 24;
 constexpr int kRed = 32;             // 8-byte words per block in a reduction record
 
 // Interaction tables on the device. The evaluation index space is
@@ -121,6 +121,7 @@ struct Ctx {
     long long *h_out = nullptr;   // pinned: what a call's last kernel tells the host
     size_t h_out_n = 0;
     DBuf<double> qe_u, simpson_part;
+    DBuf<double> solve;           // linear solve: its scalars, block sums of p.Hp and of r.r
     // CG state
     DBuf<double> F0, F1, S0, S1, xmin;
     DBuf<unsigned long long> bar, acc;

@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(kBlock) k_quad_finish(Dev D, const double *__r
                                                         const double *__restrict__ part, double *__restrict__ slots,
                                                         double *__restrict__ pe,
                                                         unsigned long long *__restrict__ tot) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *tot = 0;
+    if (tot && blockIdx.x == 0 && threadIdx.x == 0) *tot = 0;
     constexpr int NA = QuadAcc<W>::N;
     bool ok = true;
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < D.n_ev; j += gridDim.x * blockDim.x) {
@@ -478,7 +478,7 @@ int quad_classify(Ctx &c, Dev &D, const double *d_x, hipStream_t st) {
 
 template <int W>
 static void quad_launch(Ctx &c, const Dev &D, const double *d_x, const double *d_v, double *out, int rec0,
-                        hipStream_t st) {
+                        hipStream_t st, bool keep) {
     const long long n = c.n_ev;
     const dim3 blk(kBlock);
     long long g = (n + kBlock - 1) / kBlock, cap = (long long)c.num_cu * 8;
@@ -489,19 +489,24 @@ static void quad_launch(Ctx &c, const Dev &D, const double *d_x, const double *d
     hipLaunchKernelGGL(k_quad_nodes<W>, dim3(nodes), dim3(kQuadBlock), 0, st, D, d_x, d_v, gl16(), c.qoff.p, c.qmap.p,
                        c.qpan.p, c.qtot.p, rcap, c.qpart.p);
     hipLaunchKernelGGL(k_quad_finish<W>, pairs, blk, 0, st, D, d_v, c.qoff.p, c.qcnt.p, c.qpart.p, out, c.qpe.p,
-                       c.qtot.p);
+                       keep ? nullptr : c.qtot.p);
     if (W == Q_ENERGY || W == Q_JVP)
         hipLaunchKernelGGL(k_quad_records<W>, dim3(quad_blocks(c)), blk, 0, st, D, c.qpe.p, out, rec0);
 }
 
 int launch_quad(Ctx &c, const Dev &D, int what, const double *d_x, const double *d_v, double *out, int rec0,
-                hipStream_t st) {
+                hipStream_t st, bool keep) {
     switch (what) {
-        case 0: quad_launch<Q_ENERGY>(c, D, d_x, d_v, out, rec0, st); break;
-        case 1: quad_launch<Q_FORCE>(c, D, d_x, d_v, out, rec0, st); break;
-        case 2: quad_launch<Q_HVP>(c, D, d_x, d_v, out, rec0, st); break;
-        default: quad_launch<Q_JVP>(c, D, d_x, d_v, out, rec0, st); break;
+        case 0: quad_launch<Q_ENERGY>(c, D, d_x, d_v, out, rec0, st, keep); break;
+        case 1: quad_launch<Q_FORCE>(c, D, d_x, d_v, out, rec0, st, keep); break;
+        case 2: quad_launch<Q_HVP>(c, D, d_x, d_v, out, rec0, st, keep); break;
+        default: quad_launch<Q_JVP>(c, D, d_x, d_v, out, rec0, st, keep); break;
     }
+    return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
+}
+
+int quad_end(Ctx &c, hipStream_t st) {
+    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(1), 0, st, c.qtot.p);
     return hipGetLastError() == hipSuccess ? MDY_OK : MDY_ERR_HIP;
 }
 
@@ -510,7 +515,7 @@ int quad_pair_count(Ctx &c, const double *d_x, hipStream_t st, int *count) {
     if (!quad_on(c)) return MDY_OK;
     Dev D = c.dev();
     MDY_TRY(quad_classify(c, D, d_x, st));
-    hipLaunchKernelGGL(k_quad_zero, dim3(1), dim3(1), 0, st, c.qtot.p);   // no quadrature follows: clear the totals
+    MDY_TRY(quad_end(c, st));   // no quadrature follows
     std::vector<unsigned char> h((size_t)c.n_ev);
     MDY_HIP(hipMemcpyAsync(h.data(), c.evq.p, h.size(), hipMemcpyDeviceToHost, st));
     MDY_HIP(hipStreamSynchronize(st));

@@ -79,6 +79,8 @@ def load_library(path: str = LIB_PATH):
         "mdy_energy_dev_noalloc": (C.c_int, [vp, vp, vp, vp]),
         "mdy_hvp_dev": (C.c_int, [vp, vp, vp, vp, vp]),
         "mdy_hvp_dev_async": (C.c_int, [vp, vp, vp, vp, vp]),
+        "mdy_solve_hessian_dev": (C.c_int, [vp, vp, vp, vp, vp, vp, C.c_double, C.c_double, C.c_int32, C.c_double, vp,
+                                            C.POINTER(_abi.SolveResult)]),
         "mdy_sync_errors": (C.c_int, [vp, vp]),
         "mdy_energy_jvp_dev": (C.c_int, [vp, vp, vp, vp, vp]),
         "mdy_quadrature_pair_count": (C.c_int, [vp, f64p, i32p]),
@@ -352,6 +354,16 @@ class Context:
         sync_errors (or the next call that waits)."""
         self._check(self.lib.mdy_hvp_dev_async(self.h, C.c_void_p(d_coord), C.c_void_p(d_v), C.c_void_p(d_hv),
                                                C.c_void_p(stream) if stream else None))
+
+    def solve_hessian_dev(self, d_coord: int, d_w: int, d_r: int, d_p: int, d_hp: int, rr: float, tol: float,
+                          maxiter: int, shift: float, stream: int = 0) -> _abi.SolveResult:
+        """(H + shift I) w = b by conjugate gradients until r.r <= tol; w is zero and r and p
+        hold b on entry, rr = b.b, hp is scratch."""
+        res = _abi.SolveResult()
+        self._check(self.lib.mdy_solve_hessian_dev(self.h, C.c_void_p(d_coord), C.c_void_p(d_w), C.c_void_p(d_r),
+                                                   C.c_void_p(d_p), C.c_void_p(d_hp), rr, tol, maxiter, shift,
+                                                   C.c_void_p(stream) if stream else None, C.byref(res)))
+        return res
 
     def sync_errors(self, stream: int = 0):
         """Waits for the stream and raises the failure an asynchronous call left."""
