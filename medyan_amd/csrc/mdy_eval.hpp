@@ -293,7 +293,9 @@ __device__ __forceinline__ void ev_duo_item(const Dev &D, int i, const P &pos, d
             m1 = pick3(h, m1, c2e);
         }
     }
-    if (!h) {
+    // a pair is queued for its quadrature energy only where energies are summed:
+    // nothing takes the entries of a sweep for forces alone out of the queue
+    if (!h && (xs.x || PER_FF)) {
         if (ev_energy_bad(U)) {
             enqueue(D.qe, D.qe_n, j, D.err);
         } else {
