@@ -818,7 +818,11 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
                 }
             }
             K.ph++;
-        } else if (op != OP_NONE && op != OP_GATHER) {
+        } else if (op == OP_NONE) {
+            // a resume's first turn has no phase and so no barrier of its own: every
+            // wave has read S before thread 0 writes the first operation into it
+            __syncthreads();
+        } else if (op != OP_GATHER) {
             // collective work: every thread takes part beyond the barrier
             double Eff = 0.0, Effp = 0.0, step = 0.0;
             if (op == OP_EVAL_FF) {
