@@ -250,18 +250,22 @@ int launch_hvp(Ctx &c, const double *d_x, const double *d_v, double *d_hv, hipSt
 // direction. Each sums the block sums of the one before, in a fixed order, so
 // the scalars stay on the device and no iteration waits for the host, which
 // enqueues kSolveAhead iterations ahead of the last one it has seen end; after the
-// stop, the kernels of those do nothing to w, r and p. Bound by the latency of
+// stop, the kernels of those do nothing to w, r and p. No kernel writes a scalar
+// that its own blocks test: k_solve_dir writes the stop, which the next gather
+// hands on to the next k_solve_dir, so every block of a launch sees the same. Bound by the latency of
 // its kernels (six with quadrature pairs) at a few thousand cylinders: 32 us
 // per iteration at 5k; one product with a host wait and its own classification
 // of the pairs, two dot products read back and five vector kernels took 126.
 // ---------------------------------------------------------------------------
 constexpr int kSolveAhead = 2;
-enum { S_RR = 0, S_STOP = 2, S_ITER, S_PHP, S_SUMS = 8 };   // scalars: r.r of even and odd iterations, ...
+// scalars: r.r of even and odd iterations, the reason to stop, iterations done, the last p.(H + shift I)p,
+// the stop as the iteration's gather saw it
+enum { S_RR = 0, S_STOP = 2, S_ITER, S_PHP, S_SEEN, S_SUMS = 8 };
 enum { STOP_CONVERGED = 1, STOP_CURVATURE, STOP_ERROR };
 
 __global__ void k_solve_begin(double *s, double rr) {
     s[S_RR] = rr;
-    s[S_STOP] = s[S_ITER] = s[S_PHP] = 0.0;
+    s[S_STOP] = s[S_ITER] = s[S_PHP] = s[S_SEEN] = 0.0;
 }
 
 // the blocks' sums added up by every block alike
@@ -274,10 +278,12 @@ __device__ __forceinline__ double sum_of_blocks(const double *__restrict__ part,
 
 __global__ void __launch_bounds__(kBlock) k_solve_gather(Dev D, const double *__restrict__ contrib,
                                                          const double *__restrict__ p, double shift,
-                                                         double *__restrict__ hp, const double *s,
+                                                         double *__restrict__ hp, double *s,
                                                          double *__restrict__ part) {
     __shared__ double lds[24];
-    if (s[S_STOP] != 0.0) return;
+    const double stop = s[S_STOP];
+    if (blockIdx.x == 0 && threadIdx.x == 0) s[S_SEEN] = stop;
+    if (stop != 0.0) return;
     double v[1] = {0.0};
     for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < D.ndof; o += gridDim.x * blockDim.x) {
         const double q = p[o], h = __builtin_fma(shift, q, gather_coord(D, contrib, o));
@@ -294,11 +300,9 @@ __global__ void __launch_bounds__(kBlock) k_solve_step(int n, int odd, double *s
                                                        double *__restrict__ r, double *__restrict__ rr_part) {
     __shared__ double lds[24];
     if (s[S_STOP] != 0.0) return;
-    const double php = sum_of_blocks(php_part, nphp, lds);
-    if (!(php > 0.0)) {   // the same in every block
-        if (blockIdx.x == 0 && threadIdx.x == 0) { s[S_PHP] = php; s[S_STOP] = STOP_CURVATURE; }
-        return;
-    }
+    const double php = sum_of_blocks(php_part, nphp, lds);   // the same in every block
+    if (blockIdx.x == 0 && threadIdx.x == 0) s[S_PHP] = php;
+    if (!(php > 0.0)) return;
     const double a = s[S_RR + odd] / php;
     double v[1] = {0.0};
     for (int o = blockIdx.x * blockDim.x + threadIdx.x; o < n; o += gridDim.x * blockDim.x) {
@@ -311,16 +315,18 @@ __global__ void __launch_bounds__(kBlock) k_solve_step(int n, int odd, double *s
     if (threadIdx.x == 0) rr_part[blockIdx.x] = v[0];
 }
 
-// told: pinned, the reason to stop. A block that sees the stop of this launch
-// leaves its part of p, which nothing reads then.
+// told: pinned, the reason to stop
 __global__ void __launch_bounds__(kBlock) k_solve_dir(int n, int odd, double *s, const double *__restrict__ rr_part,
                                                       int nrr, const double *__restrict__ r, double *__restrict__ p,
                                                       double tol, const int *err, long long *told) {
     __shared__ double lds[24];
     const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-    const double stop = s[S_STOP];
-    if (stop != 0.0) {   // no curvature: p is the direction to report
-        if (first && stop == STOP_CURVATURE) *told = *err ? STOP_ERROR : STOP_CURVATURE;
+    if (s[S_SEEN] != 0.0) return;
+    if (!(s[S_PHP] > 0.0)) {   // no step was taken; p is the direction to report
+        if (first) {
+            s[S_STOP] = STOP_CURVATURE;
+            *told = *err ? STOP_ERROR : STOP_CURVATURE;
+        }
         return;
     }
     const double rr = sum_of_blocks(rr_part, nrr, lds), beta = rr / s[S_RR + odd];
