@@ -52,6 +52,7 @@ struct CgArgs {
     // batched passes: suspend at the top of an iteration once this many force
     // calls are done (0: never), and resume from the state a suspension saved
     int suspend_calls, resume;
+    int other;            // blocks of the launch that takes over from this one (run_minimize); 0: none
     int poll_sleep;       // barrier: 128-clock sleeps between two polls
 };
 
@@ -63,9 +64,8 @@ enum {
     R_NEC, R_NFC, R_NIT, R_GIN, R_ERC, R_NEE, R_NSM, R_NREC, R_STATUS, R_TRN, R_LAST, R_FOUT, R_NPH,
     R_T0, R_T1,            // 100 MHz wall clock at the leader's start and end
     R_DIR, R_PEND, R_BETA, R_DPREV,   // search direction at the end (buffer ids 0 F0, 1 F1, 2 S0, 3 S1)
-    R_SUSP,                // 1: the run suspended at the top of an iteration (batched passes)
-    R_RS,                  // the state a suspension saves (26 words)
-    R_SIZE = R_RS + 26
+    R_SUSP,                // 1: the run suspended and resumes in another launch
+    R_RS                   // the CgState a suspension saves
 };
 
 __device__ __forceinline__ int ld_i(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -90,6 +90,7 @@ struct Cg {
     // minimizations (nullable)
     int *done_ctr = nullptr;
     int status = MDY_OK;         // set by a collective step, the same in every thread
+    bool leave = false;          // likewise: the launch ends, to be taken up by one of more blocks
 
     // blk: this block's index within the cluster of G blocks that runs the
     // minimization (the whole grid, or one network's share of a batch)
@@ -278,6 +279,10 @@ struct Cg {
             status = MDY_ERR_CAPACITY;
             return true;
         }
+        if (nqe > G && A.other > G) {   // the larger grid repeats this evaluation
+            leave = true;
+            return true;
+        }
         if (__builtin_expect(nqe > 0, 0) && !energy_fallback(pos, d, nqe, qb)) return false;
         double v[kNFF], e[kNFF + 2];
         grid_partials_reduce<kNFF>(r, G, v, lds);
@@ -411,6 +416,7 @@ __device__ __attribute__((always_inline)) void spec_direction(Cg<MIXED> &K, cons
 // The first trial of a line search that follows an accepted step is taken
 // along s = F + beta*d while s itself is formed in the same phase; if s.F <= 0
 // (resetCGParams) that trial is discarded and redone along F.
+constexpr int kQuiet = 16;   // force calls without a fallback after which the larger grid hands back (run_minimize)
 enum Op { OP_NONE, OP_EVAL_FF, OP_EVAL, OP_EFALLBACK, OP_GATHER, OP_MINSTEP, OP_SDONLY, OP_RESTORE, OP_EXIT };
 enum Stage {
     ST_INIT_FF, ST_INIT_F, ST_INIT_G, ST_ITER, ST_TRIAL, ST_SD, ST_QUAD, ST_QUAD_EVAL, ST_QUAD_DONE, ST_QUAD_AT,
@@ -429,6 +435,7 @@ struct CgState {
     // control
     int stage, status, cur, sidx, dv, dprev, safeMode, haveMin, pendingSpec, after, suspended, quadLS;
     unsigned flags;
+    int susp;                   // force calls at which an iteration suspends
     int nEC, nFC, nIter, nEE, nSM, nRec, doneSeen;
     long long trn;
     double gradInf, relE, maxF, FF, FFp, FFcur, E, xa, E0, prevEnergy, lastFDotF, slope, minimumE, lam, newE, armijo,
@@ -450,7 +457,24 @@ struct CgState {
     }
     __device__ void reset() { dv = cur; lastFDotF = FFcur; slope = FFcur; }   // resetCGParams
     __device__ void stop(int code) { status = code; after = 0; stage = ST_FINISH; }
+    // This launch ends; another one takes up the work next_op and then next_stage. Everything the
+    // minimization carries on is saved here or in the network's buffers (x, forces, directions,
+    // minimum-energy backup, trace). The phase counter restarts at 0 with cleared accumulators,
+    // which changes no value.
+    __device__ void suspend(double *R, bool leader, int next_op, int next_stage) {
+        op = next_op; stage = next_stage;
+        doneSeen = 0;
+        if (leader) {
+            *reinterpret_cast<CgState *>(R + R_RS) = *this;
+            R[R_SUSP] = 1.0;
+        }
+        suspended = 1;
+        after = 0;
+        op = OP_NONE;
+        stage = ST_FINISH;
+    }
 };
+constexpr int R_SIZE = R_RS + (int)((sizeof(CgState) + sizeof(double) - 1) / sizeof(double));
 
 // One block's thread 0: the control flow from the work just done to the next
 // (s.op). Returns nothing; s.op = OP_EXIT at the end.
@@ -495,20 +519,8 @@ __device__ __attribute__((always_inline)) void cg_control(CgState &s, const CgAr
                 s.stage = ST_FINAL;
                 break;
             }
-            if ((A.suspend_calls > 0 && s.nFC >= A.suspend_calls) ||
-                (BATCH && suspend_done > 0 && s.doneSeen >= suspend_done)) {   // this pass ends; the next resumes here
-                if (leader) {
-                    double *S = R + R_RS;
-                    S[0] = s.flags; S[1] = s.nEC; S[2] = s.nFC; S[3] = s.nIter; S[4] = s.nEE; S[5] = s.nSM;
-                    S[6] = s.nRec; S[7] = (double)s.trn; S[8] = s.gradInf; S[9] = s.relE; S[10] = s.cur; S[11] = s.sidx;
-                    S[12] = s.dv; S[13] = s.maxF; S[14] = s.FFcur; S[15] = s.E0; S[16] = s.prevEnergy;
-                    S[17] = s.lastFDotF; S[18] = s.slope; S[19] = s.safeMode; S[20] = s.minimumE; S[21] = s.haveMin;
-                    S[22] = s.beta; S[23] = s.pendingSpec; S[24] = s.dprev; S[25] = s.sNew;
-                    R[R_SUSP] = 1.0;
-                }
-                s.suspended = 1;
-                s.after = 0;
-                s.stage = ST_FINISH;
+            if (s.nFC >= s.susp || (BATCH && suspend_done > 0 && s.doneSeen >= suspend_done)) {
+                s.suspend(R, leader, OP_NONE, ST_ITER);
                 break;
             }
             s.nIter++;
@@ -737,25 +749,17 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
     const bool leader = (K.blk == 0 && tid == 0);
     if (leader) { R[R_T0] = (double)wall_clock64(); R[R_SUSP] = 0.0; }
     if (tid == 0) {
-        // everything the iterations carry from one to the next starts here, or
-        // from what a suspension saved; the vectors (x, forces, directions,
-        // minimum-energy backup, trace) stay in the network's buffers. The phase
-        // counter restarts at 0 with cleared accumulators, which changes no value.
-        S = CgState{};
-        S.op = OP_EVAL_FF; S.at_x(); S.stage = ST_INIT_FF;
-        S.gradInf = S.relE = S.minimumE = INFINITY;
-        S.after = 1;
-        S.dv = S.dprev = S.sNew = -1;
         if (A.resume) {
-            const double *Q = R + R_RS;
-            S.flags = (unsigned)Q[0]; S.nEC = (int)Q[1]; S.nFC = (int)Q[2]; S.nIter = (int)Q[3]; S.nEE = (int)Q[4];
-            S.nSM = (int)Q[5]; S.nRec = (int)Q[6]; S.trn = (long long)Q[7]; S.gradInf = Q[8]; S.relE = Q[9];
-            S.cur = (int)Q[10]; S.sidx = (int)Q[11]; S.dv = (int)Q[12]; S.maxF = Q[13]; S.FFcur = Q[14]; S.E0 = Q[15];
-            S.prevEnergy = Q[16]; S.lastFDotF = Q[17]; S.slope = Q[18]; S.safeMode = (int)Q[19]; S.minimumE = Q[20];
-            S.haveMin = (int)Q[21]; S.beta = Q[22]; S.pendingSpec = (int)Q[23]; S.dprev = (int)Q[24];
-            S.sNew = (int)Q[25];
-            S.op = OP_NONE; S.stage = ST_ITER;
+            S = *reinterpret_cast<const CgState *>(R + R_RS);
+        } else {
+            S = CgState{};
+            S.op = OP_EVAL_FF; S.at_x(); S.stage = ST_INIT_FF;
+            S.gradInf = S.relE = S.minimumE = INFINITY;
+            S.after = 1;
+            S.dv = S.dprev = S.sNew = -1;
         }
+        S.susp = A.suspend_calls > 0 ? A.suspend_calls : 0x7fffffff;
+        if (A.other && A.other < G) S.susp = S.nFC + kQuiet;
     }
     auto vec = [&](int id) -> double * {
         return id == 0 ? A.F0 : id == 1 ? A.F1 : id == 2 ? A.S0 : id == 3 ? A.S1 : nullptr;
@@ -776,9 +780,20 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
         if (op == OP_GATHER) {
             const int nqf = uni(S.nqf);
             if (__builtin_expect(nqf != 0, 0)) {
-                ok = K.force_fallback(P, nqf, uni(S.qb));
-                if (!ok) break;
-                failed = K.status != 0;
+                if (A.other > G) {   // the larger grid repeats the evaluation: its slots stay here, its queue does not
+                    __syncthreads();   // S is read
+                    if (tid == 0) {
+                        S.nEE--;
+                        S.suspend(R, leader, OP_EVAL, S.stage == ST_INIT_G ? ST_INIT_F
+                                                      : S.stage == ST_ACCEPT ? ST_LS_DONE : ST_REC_EVAL);
+                    }
+                    failed = true;
+                } else {
+                    ok = K.force_fallback(P, nqf, uni(S.qb));
+                    if (!ok) break;
+                    failed = K.status != 0;
+                    if (tid == 0 && A.other) S.susp = S.nFC + kQuiet;
+                }
             }
         }
         if (__builtin_expect((op == OP_EVAL || op == OP_GATHER || op == OP_SDONLY) && !failed, 1)) {
@@ -811,8 +826,17 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
                             S.nEE++;
                             S.E = v;
                             S.nqe = nqe; S.nqf = nqf; S.qb = p1 % 3;
-                            if (__builtin_expect(nqe > kQueueCap || nqf > kQueueCap, 0)) S.status = MDY_ERR_CAPACITY;
-                            else if (__builtin_expect(nqe > 0, 0)) S.op = OP_EFALLBACK;
+                            if (__builtin_expect(nqe > kQueueCap || nqf > kQueueCap, 0)) {
+                                S.status = MDY_ERR_CAPACITY;
+                            } else if (__builtin_expect(nqe > 0, 0)) {
+                                if (nqe > G && A.other > G) {   // the larger grid repeats this turn
+                                    S.nEE--;
+                                    S.suspend(R, leader, OP_EVAL, S.stage);
+                                } else {
+                                    S.op = OP_EFALLBACK;
+                                    if (A.other && nqe > A.other) S.susp = S.nFC + kQuiet;
+                                }
+                            }
                         }
                     }
                 }
@@ -827,6 +851,7 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
             double Eff = 0.0, Effp = 0.0, step = 0.0;
             if (op == OP_EVAL_FF) {
                 ok = K.eval_ff(P, R + (uni(S.ffAfter) ? R_EA : R_EB), Eff, Effp);
+                if (__builtin_expect(K.leave, 0) && tid == 0) S.suspend(R, leader, OP_EVAL_FF, S.stage);
             } else if (op == OP_EFALLBACK) {
                 ok = K.energy_fallback(P, K.dv(uni(S.qb)), uni(S.nqe), uni(S.qb));
             } else if (op == OP_MINSTEP) {
@@ -926,8 +951,9 @@ static const void *cg_batch_kernel(bool mixed, bool quad) {
 
 // ---------------------------------------------------------------------------
 // Buffers and arguments of one minimization run by a cluster of G blocks on
-// stream st (the counters and flags it relies on are cleared there).
-static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, hipStream_t st, CgArgs &A) {
+// stream st (the counters and flags it relies on are cleared there; the error
+// word where it starts, not where it resumes).
+static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, bool resume, hipStream_t st, CgArgs &A) {
     const int ndof = 3 * c.nb;
     MDY_TRY(ensure(c.F0, ndof)); MDY_TRY(ensure(c.F1, ndof));
     MDY_TRY(ensure(c.S0, ndof)); MDY_TRY(ensure(c.S1, ndof));
@@ -948,7 +974,7 @@ static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, hipStr
     MDY_HIP(hipMemsetAsync(c.bar.p, 0, 32 * sizeof(unsigned long long), st));
     MDY_HIP(hipMemsetAsync(c.qn.p, 0, 16 * sizeof(int), st));
     MDY_HIP(hipMemsetAsync(c.acc.p, 0, 3 * kAccWords * sizeof(unsigned long long), st));
-    MDY_HIP(hipMemsetAsync(c.err.p, 0, sizeof(int), st));
+    if (!resume) MDY_HIP(hipMemsetAsync(c.err.p, 0, sizeof(int), st));
     if (c.prof_cap > 0) MDY_HIP(hipMemsetAsync(c.prof.p, 0, (5 * (size_t)c.prof_cap + 5) * sizeof(long long), st));
     A.D = c.dev();
     A.x = d_x; A.F0 = c.F0.p; A.F1 = c.F1.p; A.S0 = c.S0.p; A.S1 = c.S1.p; A.xmin = c.xmin.p;
@@ -965,7 +991,8 @@ static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, hipStr
     A.spin_limit = 20000000LL;   // polls (about 10 s) before the watchdog fires
     A.grid = G;
     A.suspend_calls = 0;
-    A.resume = 0;
+    A.resume = resume;
+    A.other = 0;
     // Polls go past L2. Below 64 blocks their traffic is small and the shorter wait wins; at 256
     // blocks 2k clocks measured best (40k cylinders: 81.7 / 79.7 / 85.8 us per iteration at 512 /
     // 2k / 8k clocks)
@@ -1076,24 +1103,37 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
     // lanes, of 768 (three waves per SIMD) beyond: 200k cylinders 191 against 195.
     const int lanes = c.dev().n_lanes();
     const int threads = lanes > c.num_cu * 512 ? kCgBlock : 512;
-    int G = per_cu * c.num_cu;
-    if (c.opts.blocks_per_cu <= 0) G = std::min(G, std::max(8, (lanes + threads - 1) / threads));
-    c.coop_blocks = G;
-    CgArgs A;
-    MDY_TRY(prepare_cg(c, p, d_x, G, st, A));
+    // The fallbacks' quadratures want every CU: 260 us for a turn of queued
+    // energies, a block each, and 155 ms per queued force on 8 blocks (5 on 256). An
+    // evaluation that queues more energies than there are blocks, or a force
+    // that is needed, suspends the launch; one on all blocks repeats it and hands
+    // back after kQuiet force calls without another. 60 force calls from 64
+    // parallel pairs: 3.5 ms, 6.9 on 8 blocks alone, 4.1 on 256 alone; 2 force
+    // calls with both of 2 pairs by quadrature: 31 ms, 928 on 8 blocks alone.
+    const int all = per_cu * c.num_cu;
+    const int few = c.opts.blocks_per_cu > 0 ? all : std::min(all, std::max(8, (lanes + threads - 1) / threads));
+    int G = few;
     EventPair ev;
     MDY_HIP(hipEventCreate(&ev.a));
     MDY_HIP(hipEventCreate(&ev.b));
-    MDY_HIP(hipEventRecord(ev.a, st));
-    void *args[] = {&A};
-    if (hipLaunchCooperativeKernel(kern, dim3(G), dim3(threads), args, 0, st) != hipSuccess) return MDY_ERR_LAUNCH;
-    MDY_HIP(hipEventRecord(ev.b, st));
+    CgArgs A;
     double R[R_SIZE];
-    MDY_HIP(hipMemcpyAsync(R, c.cg_out.p, sizeof(R), hipMemcpyDeviceToHost, st));
-    MDY_HIP(hipStreamSynchronize(st));
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, ev.a, ev.b);
-    c.last_ms = ms;
+    c.last_ms = 0;
+    for (bool resume = false;; resume = true, G = G == few ? all : few) {
+        MDY_TRY(prepare_cg(c, p, d_x, G, resume, st, A));
+        if (few < all && c.prof_cap == 0) A.other = G == few ? all : few;   // a profile is one launch's
+        MDY_HIP(hipEventRecord(ev.a, st));
+        void *args[] = {&A};
+        if (hipLaunchCooperativeKernel(kern, dim3(G), dim3(threads), args, 0, st) != hipSuccess) return MDY_ERR_LAUNCH;
+        MDY_HIP(hipEventRecord(ev.b, st));
+        MDY_HIP(hipMemcpyAsync(R, c.cg_out.p, sizeof(R), hipMemcpyDeviceToHost, st));
+        MDY_HIP(hipStreamSynchronize(st));
+        float ms = 0;
+        (void)hipEventElapsedTime(&ms, ev.a, ev.b);
+        c.last_ms += ms;
+        if (R[R_SUSP] == 0.0 || R[R_STATUS] != MDY_OK) break;
+    }
+    c.coop_blocks = G;
     collect(c, R, p, A, res);
     MDY_TRY(copy_force_out(c, R, d_force_out, st));
     MDY_HIP(hipStreamSynchronize(st));
@@ -1198,8 +1238,7 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
             map.clear();
             for (int i = 0; i < m && rc == MDY_OK; i++) {
                 const int k = todo[lo + i];
-                rc = prepare_cg(*cs[k], &p[k], d_x[k], gsz[i], st, args[i]);
-                args[i].resume = resume[k];
+                rc = prepare_cg(*cs[k], &p[k], d_x[k], gsz[i], resume[k] != 0, st, args[i]);
                 if (cap > 0 && cap < (long long)args[i].force_call_limit) args[i].suspend_calls = (int)cap;
                 for (int b = 0; b < gsz[i]; b++) map.push_back(make_int2(i, b));
             }
