@@ -52,7 +52,7 @@ struct CgArgs {
     // batched passes: suspend at the top of an iteration once this many force
     // calls are done (0: never), and resume from the state a suspension saved
     int suspend_calls, resume;
-    int other;            // blocks of the launch that takes over from this one (run_minimize); 0: none
+    int other;            // blocks of the launch that takes over from this one; 0: none
     int poll_sleep;       // barrier: 128-clock sleeps between two polls
 };
 
@@ -64,7 +64,7 @@ enum {
     R_NEC, R_NFC, R_NIT, R_GIN, R_ERC, R_NEE, R_NSM, R_NREC, R_STATUS, R_TRN, R_LAST, R_FOUT, R_NPH,
     R_T0, R_T1,            // 100 MHz wall clock at the leader's start and end
     R_DIR, R_PEND, R_BETA, R_DPREV,   // search direction at the end (buffer ids 0 F0, 1 F1, 2 S0, 3 S1)
-    R_SUSP,                // 1: the run suspended and resumes in another launch
+    R_SUSP,                // 1: the run suspended and resumes in another launch; kWants: on more blocks
     R_RS                   // the CgState a suspension saves
 };
 
@@ -416,6 +416,7 @@ __device__ __attribute__((always_inline)) void spec_direction(Cg<MIXED> &K, cons
 // The first trial of a line search that follows an accepted step is taken
 // along s = F + beta*d while s itself is formed in the same phase; if s.F <= 0
 // (resetCGParams) that trial is discarded and redone along F.
+constexpr int kWants = 1 << 20;   // in a batch's count of finished networks: above all counts
 constexpr int kQuiet = 16;   // force calls without a fallback after which the larger grid hands back (run_minimize)
 enum Op { OP_NONE, OP_EVAL_FF, OP_EVAL, OP_EFALLBACK, OP_GATHER, OP_MINSTEP, OP_SDONLY, OP_RESTORE, OP_EXIT };
 enum Stage {
@@ -461,14 +462,14 @@ struct CgState {
     // minimization carries on is saved here or in the network's buffers (x, forces, directions,
     // minimum-energy backup, trace). The phase counter restarts at 0 with cleared accumulators,
     // which changes no value.
-    __device__ void suspend(double *R, bool leader, int next_op, int next_stage) {
+    __device__ void suspend(double *R, bool leader, int next_op, int next_stage, int why = 1) {
         op = next_op; stage = next_stage;
         doneSeen = 0;
         if (leader) {
             *reinterpret_cast<CgState *>(R + R_RS) = *this;
-            R[R_SUSP] = 1.0;
+            R[R_SUSP] = why;
         }
-        suspended = 1;
+        suspended = why;
         after = 0;
         op = OP_NONE;
         stage = ST_FINISH;
@@ -785,7 +786,7 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
                     if (tid == 0) {
                         S.nEE--;
                         S.suspend(R, leader, OP_EVAL, S.stage == ST_INIT_G ? ST_INIT_F
-                                                      : S.stage == ST_ACCEPT ? ST_LS_DONE : ST_REC_EVAL);
+                                                      : S.stage == ST_ACCEPT ? ST_LS_DONE : ST_REC_EVAL, kWants);
                     }
                     failed = true;
                 } else {
@@ -831,7 +832,7 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
                             } else if (__builtin_expect(nqe > 0, 0)) {
                                 if (nqe > G && A.other > G) {   // the larger grid repeats this turn
                                     S.nEE--;
-                                    S.suspend(R, leader, OP_EVAL, S.stage);
+                                    S.suspend(R, leader, OP_EVAL, S.stage, kWants);
                                 } else {
                                     S.op = OP_EFALLBACK;
                                     if (A.other && nqe > A.other) S.susp = S.nFC + kQuiet;
@@ -851,7 +852,7 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
             double Eff = 0.0, Effp = 0.0, step = 0.0;
             if (op == OP_EVAL_FF) {
                 ok = K.eval_ff(P, R + (uni(S.ffAfter) ? R_EA : R_EB), Eff, Effp);
-                if (__builtin_expect(K.leave, 0) && tid == 0) S.suspend(R, leader, OP_EVAL_FF, S.stage);
+                if (__builtin_expect(K.leave, 0) && tid == 0) S.suspend(R, leader, OP_EVAL_FF, S.stage, kWants);
             } else if (op == OP_EFALLBACK) {
                 ok = K.energy_fallback(P, K.dv(uni(S.qb)), uni(S.nqe), uni(S.qb));
             } else if (op == OP_MINSTEP) {
@@ -897,7 +898,10 @@ __device__ __attribute__((always_inline)) void cg_run(const CgArgs &A, double *l
         // that shift is pending until the next trial
         R[R_DIR] = S.dv; R[R_PEND] = S.pendingSpec; R[R_BETA] = S.beta; R[R_DPREV] = S.dprev;
         R[R_T1] = (double)wall_clock64();
-        if (BATCH && done && !S.suspended) atomicAdd(done, 1);
+        if (BATCH && done) {
+            if (S.suspended == kWants) atomicOr(done, kWants);
+            else if (!S.suspended) atomicAdd(done, 1);
+        }
     }
 }
 
@@ -1156,10 +1160,17 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
 // finished minimizations on the device, and once max(1, m / k) have finished
 // the others suspend at the top of their next iteration (each reads the
 // count once per iteration); the next pass re-splits all the blocks among
-// them, down to one network on the whole grid. cs[i] owns network i's
-// tables, neighbor lists and CG buffers; cs[0] the launch arrays.
+// them, down to one network on the whole grid. Quadrature fallbacks that want
+// more blocks than a network has lanes for (run_minimize) end a pass as well:
+// from the next one on the network gets some that nobody has lanes for, up to
+// kWideThreads (8 networks of 128 cylinders, 64 parallel pairs and 60 force
+// calls each: 4.2 ms, 36 on the two blocks that their lanes fill; 4 networks
+// with 2 force calls by 2 quadratures each: 232 ms and 7310 on one block).
+// cs[i] owns network i's tables, neighbor lists and CG buffers; cs[0] the
+// launch arrays.
 constexpr int kUncappedShare = 4096;   // threads per network at which a pass runs uncapped
 constexpr int kCapGrowth = 4;          // force-call cap growth from one pass to the next (x2 measured slower)
+constexpr int kWideThreads = 16384;    // threads of a network with quadrature fallbacks, at most
 constexpr int kBatchBlock = 512;       // threads per block while every network gets a block
 int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d_x, double *const *d_force_out,
                        mdy_min_result *res, double *net_ms, int threads_per_block, const double *weights,
@@ -1182,7 +1193,7 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
     }
     if (per_cu < 1) return MDY_ERR_LAUNCH;
     const int Gmax = per_cu * c0.num_cu;
-    std::vector<char> resume(n, 0);   // suspended in an earlier pass
+    std::vector<char> resume(n, 0), wide(n, 0);   // suspended in an earlier pass; for its fallbacks
     EventPair ev;
     MDY_HIP(hipEventCreate(&ev.a));
     MDY_HIP(hipEventCreate(&ev.b));
@@ -1196,7 +1207,7 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
     long long cap = first_pass_calls > 0 ? first_pass_calls : 0;
     const int by_done = first_pass_calls < 0 ? -first_pass_calls : 0;
     int rc = MDY_OK;
-    if (by_done) rc = ensure(c0.batch_done, 1);
+    rc = ensure(c0.batch_done, 1);
     while (!todo.empty() && rc == MDY_OK) {
         next.clear();
         const int nt = (int)todo.size();
@@ -1232,13 +1243,32 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
                       });
             for (int k = 0; k < spare - used && k < m; k++) gsz[frac[k].second]++;
             // one lane per thread: more blocks only slow a cluster's barrier down
-            for (int i = 0; i < m; i++)
+            int nwide = 0;
+            used = 0;
+            for (int i = 0; i < m; i++) {
                 gsz[i] = std::min(gsz[i], std::max(1, (cs[todo[lo + i]]->dev().n_lanes() + tpb - 1) / tpb));
+                used += gsz[i];
+                nwide += wide[todo[lo + i]];
+            }
+            // what that leaves is for the fallbacks: split among the networks that asked, or there to be asked for
+            std::vector<int> other(m, 0);
+            bool may_want = false;
+            const int left = Gmax - used, each = nwide ? left / nwide : 0;
+            for (int i = 0; i < m; i++) {
+                const int room = std::max(0, kWideThreads / tpb - gsz[i]);
+                if (wide[todo[lo + i]]) {
+                    gsz[i] += std::min(room, each);
+                } else if (std::min(room, left) > 0) {
+                    other[i] = gsz[i] + std::min(room, left);
+                    may_want = true;
+                }
+            }
             args.assign(m, CgArgs{});
             map.clear();
             for (int i = 0; i < m && rc == MDY_OK; i++) {
                 const int k = todo[lo + i];
                 rc = prepare_cg(*cs[k], &p[k], d_x[k], gsz[i], resume[k] != 0, st, args[i]);
+                args[i].other = other[i];
                 if (cap > 0 && cap < (long long)args[i].force_call_limit) args[i].suspend_calls = (int)cap;
                 for (int b = 0; b < gsz[i]; b++) map.push_back(make_int2(i, b));
             }
@@ -1254,14 +1284,14 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
                 rc = MDY_ERR_HIP;
                 break;
             }
-            if (by_done && hipMemsetAsync(c0.batch_done.p, 0, sizeof(int), st) != hipSuccess) {
+            if (hipMemsetAsync(c0.batch_done.p, 0, sizeof(int), st) != hipSuccess) {
                 rc = MDY_ERR_HIP;
                 break;
             }
             const CgArgs *pa = reinterpret_cast<const CgArgs *>(c0.batch_args.p);
             const int2 *pm = c0.batch_map.p;
-            int *done = by_done && m > 1 ? c0.batch_done.p : nullptr;
-            int suspend_done = done ? std::max(1, m / by_done) : 0;
+            int *done = (by_done || may_want) && m > 1 ? c0.batch_done.p : nullptr;
+            int suspend_done = !done ? 0 : by_done ? std::max(1, m / by_done) : kWants;
             void *kargs[] = {&pa, &pm, &done, &suspend_done};
             (void)hipEventRecord(e0, st);
             if (hipLaunchCooperativeKernel(kern, dim3(G), dim3(tpb), kargs, 0, st) != hipSuccess) {
@@ -1286,6 +1316,7 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
                 ci.coop_blocks = gsz[i];
                 if (R[R_SUSP] != 0.0 && R[R_STATUS] == MDY_OK) {   // resumes in the next pass
                     resume[k] = 1;
+                    wide[k] |= R[R_SUSP] == kWants;
                     next.push_back(k);
                     continue;
                 }

@@ -5,6 +5,7 @@ evaluation). Coordinates, forces, counts and trace are those of a
 minimization on the whole grid from the start, bit for bit."""
 import numpy as np
 import pytest
+import torch
 
 from medyan_amd import _abi, mechanics, network
 from test_gpu_one_shot import exact  # noqa: F401  (a fixture)
@@ -84,3 +85,54 @@ def test_queued_forces_take_the_whole_grid():
         ctx.close()
     print(f"[gpu] {ms[0]:.1f} ms, {ms[1]:.1f} on the whole grid from the start")
     assert ms[0] < 3.0 * ms[1]
+
+
+def in_batch(nets, p, passes, **opts):
+    ctxs = []
+    for net in nets:
+        c = mechanics.Context(0, **opts)
+        c.set_network(net)
+        c.build_neighbors()
+        ctxs.append(c)
+    xs = [torch.tensor(net.coord, device="cuda") for net in nets]
+    fs = [torch.zeros_like(x) for x in xs]
+    torch.cuda.synchronize()
+    res, _, ms = mechanics.minimize_batch(ctxs, p, [x.data_ptr() for x in xs], [f.data_ptr() for f in fs],
+                                          first_pass_calls=passes)
+    out = [(x.cpu().numpy(), f.cpu().numpy(),
+            np.array([r.energies_before[_abi.MDY_NFF], r.energies_after[_abi.MDY_NFF], r.grad_inf_norm]),
+            np.array([r.num_iter, r.num_energy_call, r.num_force_call, r.num_energy_eval, r.num_safe_mode,
+                      r.num_recovery, r.error_flags]), []) for x, f, r in zip(xs, fs, res)]
+    for c in ctxs:
+        c.close()
+    return out, ms
+
+
+@pytest.mark.parametrize("precision", [_abi.MDY_PREC_FP64, _abi.MDY_PREC_MIXED])
+@pytest.mark.parametrize("passes", [0, 5, -2])
+def test_queued_energies_in_a_batch(lib, passes, precision):
+    """Networks with and without queued energies, and more of them than may run uncapped: the ones that want
+    blocks suspend the launch for all."""
+    nets = [couples(n) if i % 3 == 0 else network.generate(lib, "net500", n_filaments=20, seed=30 + i % 5)
+            for i, n in enumerate([32, 0, 0, 1, 0, 0, 4, 0, 0, 12, 0, 0] * 3)]
+    p = _abi.default_cg_params(0, force_call_limit=40, energy_rel_tol=0.0, grad_tol=1e-9)
+    got, _ = in_batch(nets, p, passes, precision=precision)
+    want = {}
+    for i, (net, g) in enumerate(zip(nets, got)):
+        key = (net.n_cyl, i % 3 == 0, float(net.coord[0]))
+        if key not in want:
+            want[key] = minimized(net, p, precision=precision, blocks_per_cu=1)[:4] + ([],)
+        assert equal(g, want[key]), i
+
+
+@pytest.mark.parametrize("n", [1, 2, 5])
+def test_queued_forces_in_a_batch(lib, n):
+    """The first network's forces go by quadrature: on more blocks than its lanes need (one), so that the
+    batch takes about 230 ms (7300 on that one)."""
+    p = _abi.default_cg_params(0, force_call_limit=2, energy_rel_tol=0.0, grad_tol=1e-9)
+    opts = dict(coplanar_mode=_abi.MDY_COPLANAR_EXACT)
+    nets = [couples(1)] + [network.generate(lib, "net500", n_filaments=20, seed=30 + i) for i in range(n - 1)]
+    got, ms = in_batch(nets, p, 0, **opts)
+    for net, g in zip(nets, got):
+        assert equal(g, minimized(net, p, **opts)[:4] + ([],))
+    assert ms < 1000.0
