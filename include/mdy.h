@@ -357,12 +357,14 @@ int mdy_minimize_dev(mdy_ctx *ctx, const mdy_cg_params *params, double *d_coord,
 /* Batched form: n independent minimizations (CGMethod::minimize per network,
  * as above) in one cooperative launch. ctxs[i] holds network i with its
  * neighbor lists; all contexts share one device and one precision and appear
- * once. The resident blocks (of at least threads_per_block = 64, 128 or 256
- * threads, 0 = 64; of up to 512 while every network gets one) are split into
- * one cluster per network in proportion to weights[i] (nullable: default the
- * per-evaluation work, interactions + 2 x beads), at least one block each and
- * at most one thread per interaction lane; each cluster runs its own minimization with its own barrier.
- * Networks beyond the resident block count run in further launches.
+ * once. The resident blocks (of threads_per_block = 128 or 256 threads; 64 or
+ * 0: of 512 while every network gets one, else of 256, 128 or 64) are split
+ * into one cluster per network in proportion to weights[i] (nullable: default
+ * the per-evaluation work, interactions + 2 x beads), at least one block each
+ * and at most one thread per interaction lane, more where quadrature fallbacks
+ * want them and blocks are left; each cluster runs its own minimization with
+ * its own barrier. Networks beyond the resident block count run in further
+ * launches.
  * first_pass_calls > 0 runs the batch in passes: pass k suspends each
  * minimization at the top of an iteration after first_pass_calls * 4^(k-1)
  * force calls, and the next pass resumes the suspended ones where they
@@ -393,6 +395,9 @@ int mdy_set_trace(mdy_ctx *ctx, int64_t cap);
 
 /* Timing of the last minimization (device events), milliseconds. */
 int mdy_last_timing(mdy_ctx *ctx, double *ms_total);
+/* Blocks that ran the last minimization when it ended (of a batch: this
+ * network's) and their threads; 0 before the first. */
+int mdy_last_launch(mdy_ctx *ctx, int32_t *blocks, int32_t *threads);
 /* Phase profile of the last minimization: the device timestamp (100 MHz
  * wall clock) at the end of each grid-wide phase and the phase kind
  * (1 energy, 2 energy fallback, 3 energy and forces, 4 force fallback,

@@ -807,6 +807,13 @@ int mdy_get_profile_detail(mdy_ctx *ctx, int64_t *rec, int64_t cap, int64_t *n) 
     return MDY_OK;
 }
 
+int mdy_last_launch(mdy_ctx *ctx, int32_t *blocks, int32_t *threads) {
+    if (!ctx || !blocks || !threads) return MDY_ERR_ARG;
+    *blocks = ctx->c.coop_blocks;
+    *threads = ctx->c.coop_threads;
+    return MDY_OK;
+}
+
 int mdy_last_timing(mdy_ctx *ctx, double *ms_total) {
     if (!ctx || !ms_total) return MDY_ERR_ARG;
     *ms_total = ctx->c.last_ms;

@@ -1138,6 +1138,7 @@ int run_minimize(Ctx &c, const mdy_cg_params *p, double *d_x, double *d_force_ou
         if (R[R_SUSP] == 0.0 || R[R_STATUS] != MDY_OK) break;
     }
     c.coop_blocks = G;
+    c.coop_threads = threads;
     collect(c, R, p, A, res);
     MDY_TRY(copy_force_out(c, R, d_force_out, st));
     MDY_HIP(hipStreamSynchronize(st));
@@ -1180,16 +1181,17 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
     bool quad = false;
     for (int i = 0; i < n; i++) quad = quad || p[i].line_search == MDY_LS_QUADRATIC;
     const void *kern = cg_batch_kernel(mixed, quad);
-    // Blocks of 512 threads while every network gets one, then half as many, down
-    // to threads_per_block: every block of a launch writes its XCD's L2 back and
-    // invalidates it once per phase of its network, for all the others too, so
-    // fewer and larger ones win (32 networks of 500 to 5000 cylinders, kernel
-    // time: 156 ms with 64 threads, 67 with 256, 53 with 512; 256 networks: 333,
-    // 147, 112). The results do not depend on it.
-    int tpb = std::max(kBatchBlock, threads_per_block), per_cu = 0;
+    // Blocks of threads_per_block threads; for 64, the default, of 512 while every
+    // network gets one, then half as many, down to 64: every block of a launch
+    // writes its XCD's L2 back and invalidates it once per phase of its network,
+    // for all the others too, so fewer and larger ones win (32 networks of 500 to
+    // 5000 cylinders, kernel time: 156 ms with 64 threads, 67 with 256, 53 with 512;
+    // 256 networks: 333, 147, 112). The results do not depend on it.
+    const bool chosen = threads_per_block > 64;
+    int tpb = chosen ? threads_per_block : kBatchBlock, per_cu = 0;
     for (;; tpb /= 2) {
         MDY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, tpb, 0));
-        if (tpb <= threads_per_block || per_cu * c0.num_cu >= n) break;
+        if (chosen || tpb <= 64 || per_cu * c0.num_cu >= n) break;
     }
     if (per_cu < 1) return MDY_ERR_LAUNCH;
     const int Gmax = per_cu * c0.num_cu;
@@ -1314,6 +1316,7 @@ int run_minimize_batch(Ctx **cs, int n, const mdy_cg_params *p, double *const *d
                 }
                 if (t_origin < 0 || R[R_T0] < t_origin) t_origin = R[R_T0];
                 ci.coop_blocks = gsz[i];
+                ci.coop_threads = tpb;
                 if (R[R_SUSP] != 0.0 && R[R_STATUS] == MDY_OK) {   // resumes in the next pass
                     resume[k] = 1;
                     wide[k] |= R[R_SUSP] == kWants;

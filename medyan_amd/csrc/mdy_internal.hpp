@@ -139,7 +139,7 @@ struct Ctx {
     bool have_dir = false, dir_pend = false;
     int dir_buf = -1, dir_cur = 0, dir_prev = -1;
     double dir_beta = 0;
-    int coop_blocks = 0;
+    int coop_blocks = 0, coop_threads = 0;   // the last minimization's grid
     Dev dev() const;
 };
 

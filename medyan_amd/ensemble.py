@@ -63,8 +63,9 @@ def autotune(ctxs, params, d_coords, restore, threads=(64, 128, 256), first_pass
     """Block and tile shapes of the batched launch (mdy_minimize_batch) for
     one ensemble, by coordinate search over measured runs:
       1. threads per block, the unit every network's cluster is built from
-         (64: more, smaller blocks per network; 256: fewer, wider ones), with
-         the first pass rule;
+         (128 and 256 as they are; 64 leaves the choice to the launch: 512
+         while every network gets a block, else less), with the first pass
+         rule;
       2. the pass rule: a force-call cap for the first pass (how long each
          network keeps its first share of blocks before the blocks of
          finished networks are moved to the ones still running), or, for a

@@ -82,6 +82,7 @@ def load_library(path: str = LIB_PATH):
         "mdy_solve_hessian_dev": (C.c_int, [vp, vp, vp, vp, vp, vp, C.c_double, C.c_double, C.c_int32, C.c_double, vp,
                                             C.POINTER(_abi.SolveResult)]),
         "mdy_sync_errors": (C.c_int, [vp, vp]),
+        "mdy_last_launch": (C.c_int, [vp, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]),
         "mdy_energy_jvp_dev": (C.c_int, [vp, vp, vp, vp, vp]),
         "mdy_quadrature_pair_count": (C.c_int, [vp, f64p, i32p]),
         "mdy_minimize": (C.c_int, [vp, C.POINTER(_abi.CGParams), f64p, f64p, C.POINTER(_abi.MinResult)]),
@@ -425,6 +426,12 @@ class Context:
                                                     C.byref(n)))
         return rec[: 5 * m].reshape(-1, 5)
 
+    def last_launch(self):
+        """(blocks, threads per block) at the end of the last minimization."""
+        b, t = C.c_int32(), C.c_int32()
+        self._check(self.lib.mdy_last_launch(self.h, C.byref(b), C.byref(t)))
+        return b.value, t.value
+
     def last_ms(self):
         t = C.c_double()
         self._check(self.lib.mdy_last_timing(self.h, C.byref(t)))
@@ -436,13 +443,13 @@ def minimize_batch(ctxs, params, d_coords, d_forces=None, threads_per_block=64, 
     """Batched minimization (mdy_minimize_batch): ctxs[i] holds network i with
     its neighbor lists; d_coords[i] its device coordinates (updated in place).
     params: one CGParams / ConjugateGradientParams for all, or one per
-    network. threads_per_block: the smallest block the launch may use (it takes
-    larger ones while every network gets a block; same results). weights (optional): block shares. first_pass_calls > 0: passes
-    with force-call caps growing 4x; a capped network is suspended and resumed
-    on more blocks. first_pass_calls = -k: passes end by completions (once
-    max(1, m / k) of a pass's m networks have finished, the others are
-    suspended and resumed on all the blocks). Returns (results, per-network
-    completion ms, total ms)."""
+    network. threads_per_block: 128 or 256, or 64 for the library's choice (512
+    while every network gets a block, else less); same results. weights
+    (optional): block shares. first_pass_calls > 0: passes with force-call caps
+    growing 4x; a capped network is suspended and resumed on more blocks.
+    first_pass_calls = -k: passes end by completions (once max(1, m / k) of a
+    pass's m networks have finished, the others are suspended and resumed on
+    all the blocks). Returns (results, per-network completion ms, total ms)."""
     n = len(ctxs)
     lib = load_library()
     if not isinstance(params, (list, tuple)):
