@@ -27,7 +27,7 @@ HIPFLAGS = [f"--offload-arch={ARCH}", "-ffp-contract=off",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # The sweep's loops inline every interaction's code: constants and addresses
 # that the compiler hoists out of them cost registers, and so waves per SIMD,
-# for the whole loop (k_force 170 -> 125 registers, k_cg 256 -> 164 without spills).
+# for the whole loop (k_force 170 -> 126 registers, k_cg 256 -> 166, at most two spilled).
 HOIST = ["-mllvm", "-disable-machine-licm"]
 EXTRA = {"mdy_eval.hip": HOIST, "mdy_hvp.hip": HOIST,
          "mdy_cg.hip": [*HOIST, "-mllvm", "-sink-insts-to-avoid-spills"]}

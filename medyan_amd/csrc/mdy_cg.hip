@@ -992,7 +992,7 @@ static int prepare_cg(Ctx &c, const mdy_cg_params *p, double *d_x, int G, bool r
     A.max_dist = p->max_dist; A.lambda_max = p->lambda_max; A.grad_tol = p->grad_tol;
     A.energy_rel_tol = p->energy_rel_tol;
     A.report_call_limit = p->report_on_call_limit;
-    A.spin_limit = 20000000LL;   // polls (about 10 s) before the watchdog fires
+    A.spin_limit = 20000000LL;   // polls (tens of seconds) before the watchdog fires
     A.grid = G;
     A.suspend_calls = 0;
     A.resume = resume;

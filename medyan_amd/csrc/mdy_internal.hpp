@@ -11,7 +11,7 @@
 namespace mdy {
 
 constexpr int kNFF = MDY_NFF;
-constexpr int kBlock = 256;          // threads per block of every kernel
+constexpr int kBlock = 256;          // threads per block, where a kernel has no size of its own
 constexpr int kQueueCap = 4096;      // excluded-volume quadrature fallback queue
 constexpr int kOneShot = 16;         // qn words of the one-shot calls: energy, force queue counts, two flags, ticket; zero between calls
 // words of Ctx::h_out: host energies; queued force pairs; error word; rebuild totals from there on
